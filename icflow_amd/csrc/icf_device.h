@@ -80,6 +80,22 @@ struct DevConsts {
 template <typename T>
 __device__ inline T dot3(const T *a, const T *b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
+// What a call's kernels tell the host: words in pinned host memory, read after the wait that the
+// call makes anyway, so that no copy and no clearing launch is needed.  A word is set when it holds
+// the call's sequence number; the device copy of the words keeps all but the first few threads
+// that set one off the bus.
+constexpr int REPORT_WORDS = 16;
+struct Report {
+    unsigned *dev, *host;
+    unsigned seq;
+    __device__ inline void set(int k) const
+    {
+        if (__hip_atomic_load(dev + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == seq) return;
+        __hip_atomic_store(dev + k, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(host + k, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+};
+
 // Index of entry (r, c), r <= c, in a packed upper triangle of a 12x12 matrix.
 __host__ __device__ inline int upper12(int r, int c) { return r * 12 - (r * (r - 1)) / 2 + (c - r); }
 

@@ -212,6 +212,12 @@ struct icf_ctx {
     // adjacency lists may no longer match what they were built from: a graph captured at an
     // older epoch may point at stale memory and is refused by icf_graph_launch
     unsigned long long epoch = 1;
+    // bumped with it, except where the fields in question were found unchanged: the batched
+    // call's layout check holds as long as this stays (no graph is involved in it)
+    unsigned long long fields_epoch = 1;
+    // what kernels report to the host (Report): pinned words, their device copy, the last call's
+    // sequence number
+    unsigned *rep_host = nullptr, *rep_dev = nullptr, rep_seq = 0;
     int precision = ICF_FP64;
     DevConsts hc;
     DevBuf tet_rhs, tet_tan, cz_rhs, cz_tan, ct, scan_tmp;
@@ -307,6 +313,17 @@ int fail(icf_ctx *ctx, int code, const std::string &msg)
             return fail((ctx), (int)e_, std::string(#x) + ": " + hipGetErrorString(e_));           \
     } while (0)
 
+void bump(icf_ctx *ctx)
+{
+    ctx->epoch++;
+    ctx->fields_epoch++;
+}
+
+// A new report for the launches of one call; its words read as not set until a kernel sets them.
+Report new_report(icf_ctx *ctx) { return Report{ctx->rep_dev, ctx->rep_host, ++ctx->rep_seq}; }
+// After the stream has been waited for.
+bool reported(const Report &r, int k) { return ((volatile unsigned *)r.host)[k] == r.seq; }
+
 int grow(icf_ctx *ctx, DevBuf &b, size_t bytes)
 {
     if (b.bytes >= bytes) return 0;
@@ -319,7 +336,7 @@ int grow(icf_ctx *ctx, DevBuf &b, size_t bytes)
         b.bytes = 0;
     }
     size_t want = bytes + bytes / 4 + 256;
-    ctx->epoch++;
+    bump(ctx);
     HIPCHK(ctx, hipMalloc(&b.p, want));
     b.bytes = want;
     return 0;
@@ -361,11 +378,11 @@ void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = fal
 {
     if (ctx->adj.valid && ctx->adj.lo < hi && lo < ctx->adj.hi) {
         ctx->adj.valid = false;
-        ctx->epoch++;
+        bump(ctx);
     }
     for (auto it = ctx->maps.begin(); it != ctx->maps.end();) {
         const bool hit = map_keys_overlap(*it, lo, hi);
-        if (hit) ctx->epoch++;
+        if (hit) bump(ctx);
         if (hit && erase) {
             (void)hipStreamSynchronize(ctx->stream);
             free_map(*it);
@@ -375,6 +392,15 @@ void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = fal
             ++it;
         }
     }
+}
+
+// Fields in [lo, hi) were written again with the values they had: what was built from them holds,
+// and only graphs captured before are refused, as after any write to such fields.
+void touch_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi)
+{
+    bool hit = ctx->adj.valid && ctx->adj.lo < hi && lo < ctx->adj.hi;
+    for (const SlotMap &m : ctx->maps) hit = hit || map_keys_overlap(m, lo, hi);
+    if (hit) ctx->epoch++;
 }
 
 // A write by the library into caller memory [p, p + bytes) (copies, kernels that write int
@@ -514,7 +540,7 @@ int get_map(icf_ctx *ctx, int target, int fixed_nkeys, const std::vector<SrcKey>
             if (diff) {
                 free_map(m);
                 ctx->maps.erase(it);
-                ctx->epoch++;
+                bump(ctx);
                 break;
             }
             m.suspect = false;
@@ -1272,6 +1298,10 @@ int icf_create(int device, icf_ctx **out)
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev0);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev1);
     if (e == hipSuccess) e = hipMalloc(&ctx->small, 8 * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc(&ctx->rep_dev, REPORT_WORDS * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMemset(ctx->rep_dev, 0, REPORT_WORDS * sizeof(unsigned));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->rep_host, REPORT_WORDS * sizeof(unsigned), hipHostMallocMapped);
+    if (e == hipSuccess) memset(ctx->rep_host, 0, REPORT_WORDS * sizeof(unsigned));
     if (e == hipSuccess) e = scratch_for_device(device, (void **)&ctx->noalloc);
     if (e != hipSuccess) {
         delete ctx;
@@ -1295,6 +1325,8 @@ int icf_destroy(icf_ctx *ctx)
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->small) (void)hipFree(ctx->small);
+    if (ctx->rep_dev) (void)hipFree(ctx->rep_dev);
+    if (ctx->rep_host) (void)hipHostFree(ctx->rep_host);
     (void)hipEventDestroy(ctx->ev0);
     (void)hipEventDestroy(ctx->ev1);
     for (auto &p : ctx->pending) {
@@ -1496,7 +1528,7 @@ int icf_pattern_changed(icf_ctx *ctx)
     for (SlotMap &m : ctx->maps) m.suspect = true;
     ctx->adj.valid = false;
     ctx->patc.valid = false;
-    ctx->epoch++;
+    bump(ctx);
     return 0;
 }
 
@@ -2205,15 +2237,15 @@ int icf_assemble_batched(icf_ctx *ctx, const icf_worklist *wl, const int *ie, in
         B.off = off;
         B.n = n;
         B.checked.clear();
-        ctx->epoch++;              // a captured batch reads the old offsets
+        bump(ctx);                 // a captured batch reads the old offsets
     }
     const int *d = (const int *)B.d.p;
     const BatchOff bo{d, d + (n + 1), d + 2 * (n + 1), d + 3 * (n + 1), n};
     int *cnt = (int *)B.d.p + 4 * (n + 1);
     // The block-diagonal layout, checked before anything is written whenever the units or the
-    // slot fields may have changed (a library write to them moves the epoch).
+    // slot fields may have changed (a library write to them moves the fields' epoch).
     const std::vector<long long> sig{(long long)(uintptr_t)ie, (long long)(uintptr_t)icz, el_stride, cz_stride, nE,
-                                     nC, (long long)ctx->epoch};
+                                     nC, (long long)ctx->fields_epoch};
     if (sig != B.checked) {
         if (ctx->capturing)
             return fail(ctx, ICF_E_CAPTURE, "icf_assemble_batched: run the batch once uncaptured before capture");
@@ -2241,7 +2273,7 @@ int icf_assemble_batched(icf_ctx *ctx, const icf_worklist *wl, const int *ie, in
     if (ra) return ra;
     if (sig != B.checked) {
         B.checked = sig;
-        B.checked.back() = (long long)ctx->epoch;   // map checks inside the call may have moved it
+        B.checked.back() = (long long)ctx->fields_epoch;   // map checks inside the call may have moved it
     }
     OnLane ln(ctx, 0, [&] {
         return Access()
@@ -2480,26 +2512,33 @@ int icf_pack_pcsr(icf_ctx *ctx, const int *altId, int nNodes, const int *csr_row
         (nImpacts && !icr))
         return fail(ctx, ICF_E_INVALID, "icf_pack_pcsr: invalid argument");
     if (ctx->capturing) return fail(ctx, ICF_E_CAPTURE, "icf_pack_pcsr reports index errors to the host");
-    int *d_err = ctx->small + 1;
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, d_err, 1, 0);
-    PackSrc ps[3] = {{ie, nElems, el_stride, EL_NODES, EL_SLOTS, EL_ROWS, 4},
-                     {icz, nCZs, cz_stride, CZI_VRTS, CZI_SLOTS, CZI_ROWS, 6},
-                     {icr, nImpacts, cr_stride, CR_NODES, CR_SLOTS, CR_ROWS, 4}};
-    for (const PackSrc &p : ps) {
+    PackAll ps{{{ie, nElems, el_stride}, {icz, nCZs, cz_stride}, {icr, nImpacts, cr_stride}}, {}};
+    ps.wave1[0] = pack_waves(nElems, 4);
+    ps.wave1[1] = ps.wave1[0] + pack_waves(nCZs, 6);
+    ps.wave1[2] = ps.wave1[1] + pack_waves(nImpacts, 4);
+    if (ps.wave1[2] == 0) return 0;
+    const Report rep = new_report(ctx);
+    hipLaunchKernelGGL(k_pack_pcsr, dim3(blocks_for(ps.wave1[2], 4)), dim3(256), 0, ctx->stream, ps, altId, nNodes,
+                       csr_rows, csr_cols, N, rep);
+    const hipError_t launched = hipGetLastError();
+    const hipError_t waited = hipStreamSynchronize(ctx->stream);
+    const bool err = launched != hipSuccess || waited != hipSuccess || reported(rep, PACK_ERR);
+    // maps built from slot or row fields that changed are checked before their next use
+    for (int k = 0; k < 3; k++) {
+        const PackPart &p = ps.part[k];
         if (!p.n) continue;
-        hipLaunchKernelGGL(k_pack_pcsr, dim3(blocks_for((long long)p.n * p.K, 256)), dim3(256), 0, ctx->stream, p,
-                           altId, nNodes, csr_rows, csr_cols, N, d_err);
-        // slot and row fields changed: maps built from them are checked before their next use
-        invalidate_range(ctx, (uintptr_t)(p.base + (size_t)p.stride * p.slot0),
-                         (uintptr_t)(p.base + (size_t)p.stride * (p.row0 + p.K)));
+        const int slot0 = k == 1 ? CZI_SLOTS : EL_SLOTS, row0 = k == 1 ? CZI_ROWS : EL_ROWS, K = k == 1 ? 6 : 4;
+        const uintptr_t lo = (uintptr_t)(p.base + (size_t)p.stride * slot0),
+                        mid = (uintptr_t)(p.base + (size_t)p.stride * row0),
+                        hi = (uintptr_t)(p.base + (size_t)p.stride * (row0 + K));
+        for (int f = 0; f < 2; f++) {
+            const uintptr_t a = f ? mid : lo, b = f ? hi : mid;
+            if (err || reported(rep, PACK_CHANGED + 2 * k + f)) invalidate_range(ctx, a, b);
+            else touch_range(ctx, a, b);
+        }
     }
-    if (nCZs)
-        hipLaunchKernelGGL(k_pack_cz_flags, dim3(blocks_for(nCZs, 256)), dim3(256), 0, ctx->stream, icz, nCZs,
-                           cz_stride);
-    int err = 0;
-    HIPCHK(ctx, hipGetLastError());
-    HIPCHK(ctx, hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    HIPCHK(ctx, launched);
+    HIPCHK(ctx, waited);
     if (err) return fail(ctx, ICF_E_INDEX, "icf_pack_pcsr: a node id is out of range or a pair is not in the pattern");
     return 0;
 }
