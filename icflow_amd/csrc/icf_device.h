@@ -94,6 +94,11 @@ struct Report {
         __hip_atomic_store(dev + k, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(host + k, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    // a value, from one thread
+    __device__ inline void put(int k, unsigned v) const
+    {
+        __hip_atomic_store(host + k, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 };
 
 // Index of entry (r, c), r <= c, in a packed upper triangle of a 12x12 matrix.

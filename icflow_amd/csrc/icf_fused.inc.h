@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void k_phase1_fused(int nbt, int nbc, const in
 template <bool MIXED, bool ISO, typename L, int KEYS, int STAGE>
 __global__ __launch_bounds__(KEYS) void k_vals_force_fused(int nbf, const int *__restrict__ off,
                                                            const uint32_t *__restrict__ codes,
-                                                           const int2 *__restrict__ chunks, int nchunks,
+                                                           int nlist, int nchunks,
                                                            double *__restrict__ A, const int *__restrict__ foff,
                                                            const uint32_t *__restrict__ fcodes,
                                                            const int *__restrict__ fkeys, int nfkeys,
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_fused(int nbf, const int *_
     if (!split2(blockIdx.x, nbf, nchunks, ilv != 0, local))
         reduce_vec3<true, true>(local, nbf, foff, fcodes, fkeys, nfkeys, F, ns, 1, sv, tsum);
     else if (local < nchunks)
-        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, chunks, nchunks, A, sv);
+        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, nlist, A, sv);
 }
 
 // The CZ counters (workgroups [0, nbc); per specimen when cz_off is given: the CZs of specimen s
@@ -92,7 +92,7 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_fused(int nbf, const int *_
 // workgroups): the whole second half of the fused call as one launch.  Workgroups of KEYS lanes.
 template <bool MIXED, bool ISO, typename L, int KEYS, int STAGE>
 __global__ __launch_bounds__(KEYS) void k_vals_force_rhs_fused(int nbf, int nbc, const int *__restrict__ off,
-        const uint32_t *__restrict__ codes, const int2 *__restrict__ chunks, int nchunks, double *__restrict__ A,
+        const uint32_t *__restrict__ codes, int nlist, int nchunks, double *__restrict__ A,
         const int *__restrict__ foff, const uint32_t *__restrict__ fcodes, const int *__restrict__ fkeys, int nfkeys,
         double *__restrict__ F, int ns, const int *__restrict__ node_row, const int *__restrict__ roff,
         const uint32_t *__restrict__ rcodes, const int *__restrict__ cz_begin, double *__restrict__ b,
@@ -108,7 +108,7 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_rhs_fused(int nbf, int nbc,
     else if (!split2(w - nbc, nbf, nchunks, ilv != 0, local))
         reduce_force_rhs(local, nbf, foff, fcodes, fkeys, nfkeys, F, ns, node_row, roff, rcodes, cz_begin, b, sv);
     else if (local < nchunks)
-        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, chunks, nchunks, A, sv);
+        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, nlist, A, sv);
 }
 
 // rhs rows from the tet sums plus their CZ terms (workgroups [0, nbr)), then the CZ counters.
@@ -136,8 +136,8 @@ __global__ __launch_bounds__(KEYS) void k_contact_sums(int nb0, int nb1, const i
                                                        const int *__restrict__ fkeys, int nfkeys,
                                                        double *__restrict__ F, int ns, const int *__restrict__ voff,
                                                        const uint32_t *__restrict__ vcodes,
-                                                       const int *__restrict__ vkeys, const int2 *__restrict__ chunks,
-                                                       int nchunks, double *__restrict__ A,
+                                                       const int *__restrict__ vkeys, int nlist,
+                                                       double *__restrict__ A,
                                                        const int *__restrict__ roff,
                                                        const uint32_t *__restrict__ rcodes,
                                                        const int *__restrict__ rkeys, int nrkeys,
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(KEYS) void k_contact_sums(int nb0, int nb1, const i
     if (w < nb0)
         reduce_vec3<true, false>(w, nb0, foff, fcodes, fkeys, nfkeys, F, ns, 1, sv, nullptr);
     else if (w < nb0 + nb1)
-        reduce_vals<MIXED, false, true, L, KEYS, STAGE>(w - nb0, nb1, voff, vcodes, vkeys, chunks, nchunks, A, sv);
+        reduce_vals<MIXED, false, true, L, KEYS, STAGE>(w - nb0, nb1, voff, vcodes, vkeys, nlist, A, sv);
     else
         reduce_vec3<true, false>(w - nb0 - nb1, gridDim.x - nb0 - nb1, roff, rcodes, rkeys, nrkeys, b, 1, 3, sv,
                                  nullptr);

@@ -115,32 +115,32 @@ struct SrcKey {
 
 struct SlotMap {
     int target = 0;
-    int fixed_nkeys = -1;          // -1: number of keys = largest key + 1
+    int fixed_nkeys = -1;          // -1: as many keys as the fields turn out to need
     std::vector<SrcKey> srcs;
-    int nkeys = 0;
-    int ncodes = 0;
+    int nkeys = 0;                 // keys counted; without fixed_nkeys at least the largest key + 1
+    // grow-only buffers, kept when the map is built anew
+    DevBuf b_off, b_codes, b_keys, b_loff, b_snap;
     int *off = nullptr;            // nkeys + 1
-    uint32_t *codes = nullptr;     // ncodes
+    uint32_t *codes = nullptr;
     int *keys = nullptr;           // accumulate mode: the keys with contributions (null: all keys)
+    int *loff = nullptr;           // first code per list position (off when all keys are listed)
     int nlaunch = 0;               // keys a reduction visits
-    // BCSR-value maps, per candidate chunk shape c (cand_keys(c), cand_stage(c)) and staging
-    // type (0: FP32 values, 1: FP64 values): chunk starts (list position, code position)
-    int2 *chunks[NCAND][2] = {};
-    int nchunks[NCAND][2] = {};
     int id = 0;                    // unique per map built
     // rhs maps of the fused call: the force map (by id) whose per-node tet sums seed the rows,
     // the outcome of that check, and per row the node and the first non-tet code
-    int tsum_with = 0;
+    int tsum_with = -1;
     bool tsum_ok = false;
+    DevBuf b_row_node, b_cz_begin, b_node_row;
     int *row_node = nullptr, *cz_begin = nullptr;
     // ... and per node of the force map its rhs row (-1: none), when every row has one tet node
     // (then the node-force pass also writes the rhs rows)
     int *node_row = nullptr;
     bool merge_ok = false;
-    // copy of the key fields the map was built from; after a write that may have touched them
-    // (suspect) the map is kept if they still compare equal
-    int *snap = nullptr;
+    // copies of the key fields the map was built from, per source; after a write that may have
+    // touched the fields (suspect) the map is kept if they still compare equal
+    std::vector<int *> snap;
     bool suspect = false;
+    bool built = false;
 };
 
 std::atomic<int> g_next_ctx_id{1};
@@ -233,6 +233,7 @@ struct icf_ctx {
     DevBuf bp_c;                     // broad phase grid (cell counts, first sorted position per cell key)
     DevBuf bp_g;                     // broad phase pair grouping (counts and starts per tet, ranks)
     long long bp_cap = 0;            // pair keys the broad phase's buffer holds (grows with use)
+    DevBuf map_cnt, map_rank, map_sums;   // building slot maps: counts (zero in between), ranks, tile sums
     DevBuf tsum;                     // per-node tet sums of the fused call
     DevBuf ct_f;                     // impact forces (the tangent blocks are in ct)
     int tplane = 64;                 // plane stride of the staged tet records (tet_plane)
@@ -245,9 +246,9 @@ struct icf_ctx {
         DevBuf off, ids;
         bool valid = false;
     } adj;
-    int *small = nullptr;          // 8 ints of scratch (max key, error flag, sums)
+    int *small = nullptr;          // 16 ints of scratch (error flag, sums; 8-11: largest keys)
     unsigned char *noalloc = nullptr;   // this device's `scratch` array (device address)
-    std::list<SlotMap> maps;       // std::list: pointers handed out by get_map stay valid
+    std::list<SlotMap> maps;       // std::list: pointers handed out by get_maps stay valid
     int next_map_id = 0;
     std::string err;
     double last_ms = -1;
@@ -344,28 +345,17 @@ int grow(icf_ctx *ctx, DevBuf &b, size_t bytes)
 
 void free_map(SlotMap &m)
 {
-    if (m.off) (void)hipFree(m.off);
-    if (m.codes) (void)hipFree(m.codes);
-    if (m.keys) (void)hipFree(m.keys);
-    if (m.row_node) (void)hipFree(m.row_node);
-    if (m.cz_begin) (void)hipFree(m.cz_begin);
-    if (m.node_row) (void)hipFree(m.node_row);
-    m.node_row = nullptr;
-    m.merge_ok = false;
-    if (m.chunks[0][0]) (void)hipFree(m.chunks[0][0]);   // the start of the one allocation
-    for (int c = 0; c < NCAND; c++) m.chunks[c][0] = m.chunks[c][1] = nullptr;
-    if (m.snap) (void)hipFree(m.snap);
-    m.snap = nullptr;
-    m.off = nullptr;
-    m.codes = nullptr;
-    m.keys = nullptr;
-    m.row_node = m.cz_begin = nullptr;
+    for (DevBuf *b : {&m.b_off, &m.b_codes, &m.b_keys, &m.b_loff, &m.b_snap, &m.b_row_node, &m.b_cz_begin, &m.b_node_row}) {
+        if (b->p) (void)hipFree(b->p);
+        *b = DevBuf();
+    }
 }
 
 // Maps whose key fields overlap [lo, hi): dropped when the memory goes away (erase), else
 // marked suspect, to be compared against their snapshot before the next use.
 bool map_keys_overlap(const SlotMap &m, uintptr_t lo, uintptr_t hi)
 {
+    if (!m.built) return false;
     for (const SrcKey &s : m.srcs) {
         uintptr_t a = (uintptr_t)(s.base + (size_t)s.stride * s.field0);
         uintptr_t b = (uintptr_t)(s.base + (size_t)s.stride * (s.field0 + s.nq));
@@ -513,240 +503,268 @@ void prof_flush(icf_ctx *ctx)
         prof_end(ctx, name, ea_);                                            \
     } while (0)
 
-// Build (or fetch) the slot map for `srcs` with keys of `target`.
-int get_map(icf_ctx *ctx, int target, int fixed_nkeys, const std::vector<SrcKey> &srcs, SlotMap **out)
-{
-    for (auto it = ctx->maps.begin(); it != ctx->maps.end(); ++it) {
-        SlotMap &m = *it;
-        if (m.target != target || m.fixed_nkeys != fixed_nkeys || !(m.srcs == srcs)) continue;
-        if (m.suspect) {
-            if (ctx->capturing)
-                return fail(ctx, ICF_E_CAPTURE, "a slot map must be checked during capture: run the call once uncaptured");
-            int *d_diff = ctx->small + 1;
-            hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, d_diff, 1, 0);
-            long long off = 0;
-            for (const SrcKey &k : srcs) {
-                if (k.n == 0) continue;
-                MapSrc ms{k.base, k.n, k.stride, k.field0, k.nq, k.kind};
-                const long long tot = (long long)k.n * k.nq;
-                hipLaunchKernelGGL(k_snap_cmp, dim3(blocks_for(tot, 256)), dim3(256), 0, ctx->stream, ms,
-                                   m.snap + off, d_diff);
-                off += tot;
-            }
-            int diff = 1;
-            HIPCHK(ctx, hipGetLastError());
-            HIPCHK(ctx, hipMemcpyAsync(&diff, d_diff, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-            HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-            if (diff) {
-                free_map(m);
-                ctx->maps.erase(it);
-                bump(ctx);
-                break;
-            }
-            m.suspect = false;
-        }
-        *out = &m;
-        return 0;
-    }
-    if (ctx->capturing)
-        return fail(ctx, ICF_E_CAPTURE, "a slot map would be built during capture: run the call once uncaptured");
-    for (const SrcKey &s : srcs)
-        if ((uint32_t)s.n > CODE_UNIT_MAX + 1u)
-            return fail(ctx, ICF_E_CAPACITY, "more than 2^24 units in one pcsr array");
+int lane_barrier(icf_ctx *ctx);
 
-    SlotMap m;
-    m.target = target;
-    m.fixed_nkeys = fixed_nkeys;
-    m.srcs = srcs;
-    int *d_max = ctx->small, *d_err = ctx->small + 1;
-    int nkeys = fixed_nkeys;
-    if (nkeys < 0) {
-        int init = -1;
-        HIPCHK(ctx, hipMemcpyAsync(d_max, &init, sizeof(int), hipMemcpyHostToDevice, ctx->stream));
-        for (const SrcKey &s : srcs) {
-            if (s.n == 0) continue;
-            MapSrc ms{s.base, s.n, s.stride, s.field0, s.nq, s.kind};
-            long long tot = (long long)s.n * s.nq;
-            const unsigned nb = blocks_for(tot, 256);
-            hipLaunchKernelGGL(k_map_maxkey, dim3(nb < 1024 ? nb : 1024), dim3(256), 0, ctx->stream, ms, d_max);
-        }
-        int mx = -1;
-        HIPCHK(ctx, hipMemcpyAsync(&mx, d_max, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        nkeys = mx + 1;
+// A slot map that a call needs.
+struct MapReq {
+    int target, fixed_nkeys;
+    std::vector<SrcKey> srcs;
+    SlotMap *map = nullptr;
+};
+
+MapSrc map_src(const SrcKey &k) { return MapSrc{k.base, k.n, k.stride, k.field0, k.nq, k.kind}; }
+long long src_fields(const SrcKey &k) { return (long long)k.n * k.nq; }
+
+// The workgroups of k_map_count, k_map_fill and k_snap_cmp over one more map's sources.
+void add_srcs(MapJobs &J, int job, const SlotMap &m)
+{
+    for (size_t i = 0; i < m.srcs.size(); i++) {
+        const SrcKey &k = m.srcs[i];
+        if (k.n == 0) continue;
+        const int n = J.nsrc++;
+        J.src[n] = map_src(k);
+        J.job[n] = job;
+        J.snap[n] = m.snap[i];
+        J.at[n] = n ? J.at[n - 1] + (long long)J.src[n - 1].n * J.src[n - 1].nq : 0;
+        J.blk0[n + 1] = J.blk0[n] + blocks_for(k.n, 256) * (unsigned)k.nq;
     }
-    m.nkeys = nkeys;
-    HIPCHK(ctx, hipMalloc(&m.off, sizeof(int) * ((size_t)nkeys + 1)));
-    int *d_cnt = nullptr;
-    HIPCHK(ctx, hipMalloc(&d_cnt, sizeof(int) * ((size_t)nkeys + 1)));
-    HIPCHK(ctx, hipMemsetAsync(d_cnt, 0, sizeof(int) * ((size_t)nkeys + 1), ctx->stream));
-    HIPCHK(ctx, hipMemsetAsync(d_err, 0, sizeof(int), ctx->stream));
-    for (const SrcKey &s : srcs) {
-        if (s.n == 0) continue;
-        MapSrc ms{s.base, s.n, s.stride, s.field0, s.nq, s.kind};
-        long long tot = (long long)s.n * s.nq;
-        hipLaunchKernelGGL(k_map_count, dim3(blocks_for(tot, 256)), dim3(256), 0, ctx->stream, ms, nkeys, d_cnt, d_err);
-    }
-    size_t tmp_bytes = 0;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, tmp_bytes, d_cnt, m.off, nkeys + 1, ctx->stream));
-    if (grow(ctx, ctx->scan_tmp, tmp_bytes)) {
-        (void)hipFree(d_cnt);
-        return (int)hipErrorOutOfMemory;
-    }
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, tmp_bytes, d_cnt, m.off, nkeys + 1, ctx->stream));
-    int total = 0, errflag = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&total, m.off + nkeys, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipMemcpyAsync(&errflag, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (errflag) {
-        (void)hipFree(d_cnt);
-        free_map(m);
-        return fail(ctx, ICF_E_INDEX, "a slot/row/node index exceeds the declared size");
-    }
-    int *list = nullptr;           // accumulate mode: the keys with contributions
-    int nlist = nkeys;
-    if (fixed_nkeys < 0 && nkeys > 0) {
-        // accumulate-mode maps list the keys that have contributions, so that their reduction
-        // launches over those keys only
-        int *flag = nullptr, *pos = nullptr;
-        HIPCHK(ctx, hipMalloc(&flag, sizeof(int) * ((size_t)nkeys + 1)));
-        HIPCHK(ctx, hipMalloc(&pos, sizeof(int) * ((size_t)nkeys + 1)));
-        HIPCHK(ctx, hipMemsetAsync(flag + nkeys, 0, sizeof(int), ctx->stream));
-        hipLaunchKernelGGL(k_map_flag, dim3(blocks_for(nkeys, 256)), dim3(256), 0, ctx->stream, d_cnt, nkeys, flag);
-        HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, tmp_bytes, flag, pos, nkeys + 1, ctx->stream));
-        int nt = 0;
-        HIPCHK(ctx, hipMemcpyAsync(&nt, pos + nkeys, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        HIPCHK(ctx, hipMalloc(&list, sizeof(int) * ((size_t)nt + 1)));
-        hipLaunchKernelGGL(k_map_compact, dim3(blocks_for(nkeys, 256)), dim3(256), 0, ctx->stream, flag, pos, nkeys,
-                           list);
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        HIPCHK(ctx, hipFree(flag));
-        HIPCHK(ctx, hipFree(pos));
-        nlist = nt;
-    }
-    m.keys = list;                 // null when overwriting: every key, in order
-    if (target == TGT_VALS && nlist > 0) {
-        // chunks of consecutive list positions for the staged reduction of BCSR values, one
-        // table per candidate key limit and staging type: at most `keys` keys and
-        // flat_cap_of(FP32?, keys) contributions each (a single key with more contributions gets
-        // a chunk of its own, reduced without staging)
-        std::vector<int> h_off((size_t)nkeys + 1), h_list(list ? (size_t)nlist : 0);
-        HIPCHK(ctx, hipMemcpyAsync(h_off.data(), m.off, sizeof(int) * ((size_t)nkeys + 1), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-        if (list)
-            HIPCHK(ctx, hipMemcpyAsync(h_list.data(), list, sizeof(int) * (size_t)nlist, hipMemcpyDeviceToHost,
-                                       ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        // a chunk's codes are contiguous (keys in between, if any, have none): each entry is the
-        // chunk's first list position and first code position; the last entry closes the table
-        auto key_of = [&](int p) { return list ? h_list[p] : p; };
-        std::vector<int2> ch;          // every table, one after the other, in one allocation
-        size_t at[2 * NCAND];
-        for (int kc = 0; kc < 2 * NCAND; kc++) {
-            const int kind = kc & 1, keys = cand_keys(kc >> 1);
-            const int cap = flat_cap_of(kind == 0, keys, cand_stage(kc >> 1));
-            at[kc] = ch.size();
-            ch.push_back(make_int2(0, h_off[key_of(0)]));
-            int cnt = 0, nk = 0;
-            for (int p = 0; p < nlist; p++) {
-                const int k = key_of(p);
-                const int c = h_off[k + 1] - h_off[k];
-                if (nk > 0 && (nk == keys || cnt + c > cap)) {
-                    ch.push_back(make_int2(p, h_off[k]));
-                    cnt = 0;
-                    nk = 0;
-                }
-                cnt += c;
-                nk++;
-            }
-            ch.push_back(make_int2(nlist, h_off[key_of(nlist - 1) + 1]));
-            m.nchunks[kc >> 1][kind] = (int)(ch.size() - at[kc]) - 1;
-        }
-        int2 *d = nullptr;
-        HIPCHK(ctx, hipMalloc(&d, sizeof(int2) * ch.size()));
-        for (int kc = 0; kc < 2 * NCAND; kc++) m.chunks[kc >> 1][kc & 1] = d + at[kc];
-        HIPCHK(ctx, hipMemcpyAsync(d, ch.data(), sizeof(int2) * ch.size(), hipMemcpyHostToDevice, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    }
-    m.nlaunch = nlist;
-    m.ncodes = total;
-    m.id = ++ctx->next_map_id;
-    HIPCHK(ctx, hipMalloc(&m.codes, sizeof(uint32_t) * ((size_t)total + 1)));
-    HIPCHK(ctx, hipMemsetAsync(d_cnt, 0, sizeof(int) * ((size_t)nkeys + 1), ctx->stream));
-    for (const SrcKey &s : srcs) {
-        if (s.n == 0) continue;
-        MapSrc ms{s.base, s.n, s.stride, s.field0, s.nq, s.kind};
-        long long tot = (long long)s.n * s.nq;
-        hipLaunchKernelGGL(k_map_fill, dim3(blocks_for(tot, 256)), dim3(256), 0, ctx->stream, ms, nkeys, m.off, d_cnt,
-                           m.codes);
-    }
-    if (nkeys > 0)
-        hipLaunchKernelGGL(k_map_sort, dim3(blocks_for(nkeys, 256)), dim3(256), 0, ctx->stream, m.off, m.codes, nkeys);
-    {
-        long long snap_n = 0;
-        for (const SrcKey &s : srcs) snap_n += (long long)s.n * s.nq;
-        HIPCHK(ctx, hipMalloc(&m.snap, sizeof(int) * (size_t)(snap_n + 1)));
-        long long off = 0;
-        for (const SrcKey &s : srcs) {
-            if (s.n == 0) continue;
-            MapSrc ms{s.base, s.n, s.stride, s.field0, s.nq, s.kind};
-            const long long tot = (long long)s.n * s.nq;
-            hipLaunchKernelGGL(k_snap_copy, dim3(blocks_for(tot, 256)), dim3(256), 0, ctx->stream, ms, m.snap + off);
-            off += tot;
-        }
-    }
-    HIPCHK(ctx, hipGetLastError());
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    HIPCHK(ctx, hipFree(d_cnt));
-    ctx->maps.push_back(m);
-    *out = &ctx->maps.back();
+}
+
+// Rows of the rhs map starting from the per-node tet sums of the force map (k_rhs_check); the
+// outcome is in the report after the wait.
+int launch_link(icf_ctx *ctx, SlotMap *mr, const SlotMap *mf, const MapSrc &tet, const Report &rep)
+{
+    mr->tsum_ok = mr->merge_ok = false;
+    mr->tsum_with = -1;
+    if (int r = grow(ctx, mr->b_row_node, sizeof(int) * (size_t)mr->nkeys)) return r;
+    if (int r = grow(ctx, mr->b_cz_begin, sizeof(int) * (size_t)mr->nkeys)) return r;
+    if (int r = grow(ctx, mr->b_node_row, sizeof(int) * (size_t)mf->nkeys)) return r;
+    mr->row_node = (int *)mr->b_row_node.p;
+    mr->cz_begin = (int *)mr->b_cz_begin.p;
+    mr->node_row = (int *)mr->b_node_row.p;
+    if (mf->nkeys)
+        hipLaunchKernelGGL(k_fill_int, dim3(blocks_for(mf->nkeys, 256)), dim3(256), 0, ctx->stream, mr->node_row,
+                           mf->nkeys, -1);
+    if (mr->nkeys)
+        hipLaunchKernelGGL(k_rhs_check, dim3(blocks_for(mr->nkeys, 256)), dim3(256), 0, ctx->stream, mr->off,
+                           mr->codes, mr->nkeys, mf->off, mf->codes, mf->nkeys, tet, mr->row_node, mr->cz_begin,
+                           mr->node_row, rep);
     return 0;
 }
 
-// Whether the rows of rhs map mr can start from the per-node tet sums of force map mf (see
-// k_rhs_check); decided once per pair of maps.
-int get_tsum_link(icf_ctx *ctx, SlotMap *mr, const SlotMap *mf, const MapSrc &tet, bool *ok)
+// Launches that build the maps `todo` (at most MAX_JOBS) into their buffers, and the link of rhs
+// map `mr` to force map `mf` when given; then one wait.  A map without fixed_nkeys is counted over
+// the keys its buffers hold; `over` tells where that was too few.
+int build_maps(icf_ctx *ctx, const std::vector<SlotMap *> &todo, SlotMap *mr, const SlotMap *mf, const MapSrc *tet,
+               bool over[MAX_JOBS])
 {
-    *ok = false;
-    if (mr->tsum_with != mf->id) {
-        if (ctx->capturing)
-            return fail(ctx, ICF_E_CAPTURE, "a slot map would be built during capture: run the call once uncaptured");
-        if (mr->row_node) (void)hipFree(mr->row_node);
-        if (mr->cz_begin) (void)hipFree(mr->cz_begin);
-        if (mr->node_row) (void)hipFree(mr->node_row);
-        mr->row_node = mr->cz_begin = mr->node_row = nullptr;
-        mr->tsum_ok = mr->merge_ok = false;
+    MapJobs J{};
+    long long keys = 0, fields = 0;
+    for (SlotMap *m : todo) {
+        const int j = J.njob++;
+        long long codes = 0;
+        m->snap.assign(m->srcs.size(), nullptr);
+        for (const SrcKey &k : m->srcs) codes += src_fields(k);
+        if (int r = grow(ctx, m->b_off, sizeof(int) * ((size_t)m->nkeys + 1))) return r;
+        if (int r = grow(ctx, m->b_codes, sizeof(uint32_t) * (size_t)(codes + 1))) return r;
+        if (int r = grow(ctx, m->b_snap, sizeof(int) * (size_t)(codes + 1))) return r;
+        const bool list = m->fixed_nkeys < 0;
+        if (list) {
+            const size_t most = (size_t)std::min<long long>(m->nkeys, codes) + 1;
+            if (int r = grow(ctx, m->b_keys, sizeof(int) * most)) return r;
+            if (int r = grow(ctx, m->b_loff, sizeof(int) * most)) return r;
+        }
+        m->off = (int *)m->b_off.p;
+        m->codes = (uint32_t *)m->b_codes.p;
+        m->keys = list ? (int *)m->b_keys.p : nullptr;
+        m->loff = list ? (int *)m->b_loff.p : m->off;
+        int *snap = (int *)m->b_snap.p;
+        for (size_t i = 0; i < m->srcs.size(); i++) {
+            m->snap[i] = snap;
+            snap += src_fields(m->srcs[i]);
+        }
+        add_srcs(J, j, *m);
+        J.nkeys[j] = m->nkeys;
+        J.cnt0[j] = keys;
+        J.tile0[j + 1] = J.tile0[j] + blocks_for(m->nkeys, SCAN_TILE);
+        J.sort0[j + 1] = J.sort0[j] + blocks_for(m->nkeys, 256);
+        J.off[j] = m->off;
+        J.codes[j] = m->codes;
+        J.keys[j] = m->keys;
+        J.loff[j] = list ? m->loff : nullptr;
+        keys += m->nkeys;
+        fields += codes;
+    }
+    const size_t cnt_bytes = sizeof(int) * (size_t)std::max(keys, 1LL);
+    if (ctx->map_cnt.bytes < cnt_bytes) {
+        if (int r = grow(ctx, ctx->map_cnt, cnt_bytes)) return r;
+        HIPCHK(ctx, hipMemsetAsync(ctx->map_cnt.p, 0, ctx->map_cnt.bytes, ctx->stream));
+    }
+    if (int r = grow(ctx, ctx->map_rank, sizeof(int) * (size_t)std::max(fields, 1LL))) return r;
+    const unsigned tiles = J.tile0[J.njob], sorts = J.sort0[J.njob], places = J.nsrc ? J.blk0[J.nsrc] : 0;
+    if (int r = grow(ctx, ctx->map_sums, sizeof(unsigned long long) * std::max(tiles, 1u))) return r;
+    int *cnt = (int *)ctx->map_cnt.p, *rank = (int *)ctx->map_rank.p;
+    auto *sums = (unsigned long long *)ctx->map_sums.p;
+    const Report rep = new_report(ctx);
+    if (J.njob) {
+        const dim3 b(256);
+        if (places) hipLaunchKernelGGL(k_map_count, dim3(places), b, 0, ctx->stream, J, cnt, rank, rep);
+        if (tiles) hipLaunchKernelGGL(k_map_tiles, dim3(tiles), b, 0, ctx->stream, J, cnt, sums);
+        hipLaunchKernelGGL(k_map_scan, dim3(1), b, 0, ctx->stream, J, sums, rep);
+        if (tiles) hipLaunchKernelGGL(k_map_offsets, dim3(tiles), b, 0, ctx->stream, J, cnt, sums);
+        if (places) hipLaunchKernelGGL(k_map_fill, dim3(places), b, 0, ctx->stream, J, rank);
+        if (sorts) hipLaunchKernelGGL(k_map_sort, dim3(sorts), b, 0, ctx->stream, J);
+    }
+    if (mr)
+        if (int r = launch_link(ctx, mr, mf, *tet, rep)) return r;
+    HIPCHK(ctx, hipGetLastError());
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    for (int j = 0; j < J.njob; j++) {
+        SlotMap *m = todo[j];
+        over[j] = reported(rep, MAP_ERR + j);
+        m->nlaunch = m->fixed_nkeys < 0 ? (int)((volatile unsigned *)rep.host)[MAP_NLIST + j] : m->nkeys;
+        m->id = ++ctx->next_map_id;
+        m->suspect = false;
+        m->built = !over[j];
+    }
+    if (mr) {
         mr->tsum_with = mf->id;
-        if (mr->nkeys > 0) {
-            HIPCHK(ctx, hipMalloc(&mr->row_node, sizeof(int) * (size_t)mr->nkeys));
-            HIPCHK(ctx, hipMalloc(&mr->cz_begin, sizeof(int) * (size_t)mr->nkeys));
-            int *d_err = ctx->small + 1;
-            hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, d_err, 1, 0);
-            hipLaunchKernelGGL(k_rhs_check, dim3(blocks_for(mr->nkeys, 256)), dim3(256), 0, ctx->stream, mr->off,
-                               mr->codes, mr->nkeys, mf->off, mf->codes, mf->nkeys, tet, mr->row_node, mr->cz_begin,
-                               d_err);
-            int err = 1;
-            HIPCHK(ctx, hipGetLastError());
-            HIPCHK(ctx, hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-            HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-            mr->tsum_ok = err == 0;
-            if (mr->tsum_ok && mf->nkeys > 0) {
-                HIPCHK(ctx, hipMalloc(&mr->node_row, sizeof(int) * (size_t)mf->nkeys));
-                hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, d_err, 1, 0);
-                hipLaunchKernelGGL(k_fill_int, dim3(blocks_for(mf->nkeys, 256)), dim3(256), 0, ctx->stream,
-                                   mr->node_row, mf->nkeys, -1);
-                hipLaunchKernelGGL(k_node_row, dim3(blocks_for(mr->nkeys, 256)), dim3(256), 0, ctx->stream,
-                                   mr->row_node, mr->nkeys, mr->node_row, d_err);
-                err = 1;
-                HIPCHK(ctx, hipGetLastError());
-                HIPCHK(ctx, hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-                HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-                mr->merge_ok = err == 0;
-            }
+        mr->tsum_ok = mr->nkeys > 0 && !reported(rep, LINK_ERR);
+        mr->merge_ok = mr->tsum_ok && mf->nkeys > 0 && !reported(rep, LINK_ERR + 1);
+    }
+    return 0;
+}
+
+void drop_map(icf_ctx *ctx, SlotMap *m)
+{
+    for (auto it = ctx->maps.begin(); it != ctx->maps.end(); ++it)
+        if (&*it == m) {
+            (void)hipStreamSynchronize(ctx->stream);
+            free_map(*it);
+            ctx->maps.erase(it);
+            return;
+        }
+}
+
+// Finds or builds the slot maps of one call (at most MAX_JOBS): one wait when any had to be
+// compared with its fields, one when any had to be built.  `link`: requests 1 (rhs rows) and 2
+// (node forces, over the tets `tet`) are the fused call's, whose rows may start from the forces'
+// tet sums.  A map whose fields were written since is built anew in its own buffers, also for
+// another number of units: the unit lists of a Newton loop change from call to call.
+int get_maps(icf_ctx *ctx, std::vector<MapReq> &req, const MapSrc *tet = nullptr)
+{
+    const int nreq = (int)req.size();
+    MapJobs S{};
+    bool checked = false;
+    for (int i = 0; i < nreq; i++) {
+        MapReq &r = req[i];
+        for (SlotMap &m : ctx->maps)
+            if (m.target == r.target && m.fixed_nkeys == r.fixed_nkeys && m.srcs == r.srcs) r.map = &m;
+        if (r.map && r.map->suspect) {
+            if (ctx->capturing)
+                return fail(ctx, ICF_E_CAPTURE, "a slot map must be checked during capture: run the call once uncaptured");
+            add_srcs(S, i, *r.map);
+            checked = true;
         }
     }
-    *ok = mr->tsum_ok;
+    if (!ctx->capturing && (checked || !std::all_of(req.begin(), req.end(), [](const MapReq &r) { return r.map; })))
+        if (int r = lane_barrier(ctx)) return r;      // fields may have been written on the other lane
+    if (checked) {
+        const Report rep = new_report(ctx);
+        if (S.nsrc) hipLaunchKernelGGL(k_snap_cmp, dim3(S.blk0[S.nsrc]), dim3(256), 0, ctx->stream, S, rep);
+        HIPCHK(ctx, hipGetLastError());
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        for (int i = 0; i < nreq; i++)
+            if (req[i].map && req[i].map->suspect && !reported(rep, SNAP_DIFF + i)) req[i].map->suspect = false;
+    }
+    std::vector<SlotMap *> todo, first;
+    for (MapReq &r : req) {
+        if (r.map && !r.map->suspect) continue;
+        if (ctx->capturing)
+            return fail(ctx, ICF_E_CAPTURE, "a slot map would be built during capture: run the call once uncaptured");
+        for (const SrcKey &s : r.srcs)
+            if ((uint32_t)s.n > CODE_UNIT_MAX + 1u)
+                return fail(ctx, ICF_E_CAPACITY, "more than 2^24 units in one pcsr array");
+        if (!r.map) {
+            // a map over the same arrays whose fields were written since
+            auto same = [&](const SlotMap &m) {
+                if (m.target != r.target || (m.fixed_nkeys < 0) != (r.fixed_nkeys < 0) || !m.suspect ||
+                    m.srcs.size() != r.srcs.size())
+                    return false;
+                for (size_t k = 0; k < r.srcs.size(); k++)
+                    if (m.srcs[k].base != r.srcs[k].base || m.srcs[k].kind != r.srcs[k].kind) return false;
+                return std::none_of(req.begin(), req.end(), [&](const MapReq &q) { return q.map == &m; });
+            };
+            for (SlotMap &m : ctx->maps)
+                if (!r.map && same(m)) r.map = &m;
+            if (!r.map) {
+                ctx->maps.emplace_back();
+                r.map = &ctx->maps.back();
+            }
+        }
+        SlotMap &m = *r.map;
+        if (m.built) bump(ctx);
+        m.built = false;
+        m.suspect = true;              // until it is built
+        m.tsum_with = -1;
+        m.target = r.target;
+        m.fixed_nkeys = r.fixed_nkeys;
+        m.srcs = r.srcs;
+        if (r.fixed_nkeys >= 0) m.nkeys = r.fixed_nkeys;
+        else if (m.nkeys == 0) first.push_back(&m);
+        todo.push_back(&m);
+    }
+    auto drop = [&](int code, const char *msg) {
+        for (SlotMap *m : todo) drop_map(ctx, m);
+        return fail(ctx, code, msg);
+    };
+    // maps that count as many keys as their fields need: the largest key, with room for more
+    auto size_keys = [&](const std::vector<SlotMap *> &ms) -> int {
+        int *d_max = ctx->small + 8, init[4] = {-1, -1, -1, -1}, mx[4];
+        HIPCHK(ctx, hipMemcpyAsync(d_max, init, sizeof(init), hipMemcpyHostToDevice, ctx->stream));
+        for (size_t j = 0; j < ms.size(); j++)
+            for (const SrcKey &s : ms[j]->srcs) {
+                if (s.n == 0) continue;
+                const unsigned nb = blocks_for(src_fields(s), 256);
+                hipLaunchKernelGGL(k_map_maxkey, dim3(nb < 1024 ? nb : 1024), dim3(256), 0, ctx->stream, map_src(s),
+                                   d_max + j);
+            }
+        HIPCHK(ctx, hipMemcpyAsync(mx, d_max, sizeof(mx), hipMemcpyDeviceToHost, ctx->stream));
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        for (size_t j = 0; j < ms.size(); j++)
+            ms[j]->nkeys = (int)std::min<long long>(mx[j] + 1LL + (mx[j] + 1LL) / 8, INT_MAX - 1);
+        return 0;
+    };
+    SlotMap *mr = nullptr, *mf = nullptr;
+    if (tet && nreq == 3 &&
+        (!req[1].map->built || !req[2].map->built || req[1].map->tsum_with != req[2].map->id)) {
+        if (ctx->capturing)
+            return fail(ctx, ICF_E_CAPTURE, "a slot map would be built during capture: run the call once uncaptured");
+        mr = req[1].map;
+        mf = req[2].map;
+    }
+    if (todo.empty() && !mr) return 0;
+    bool over[MAX_JOBS] = {};
+    int err = first.empty() ? 0 : size_keys(first);
+    if (!err) err = build_maps(ctx, todo, mr, mf, tet, over);
+    std::vector<SlotMap *> again;
+    bool bad = false;
+    for (size_t j = 0; j < todo.size() && !err; j++)
+        if (over[j]) {
+            if (todo[j]->fixed_nkeys >= 0) bad = true;
+            else again.push_back(todo[j]);
+        }
+    if (!err && !bad && !again.empty()) {
+        err = size_keys(again);
+        bool over2[MAX_JOBS] = {};
+        if (!err) err = build_maps(ctx, again, mr, mf, tet, over2);
+        for (bool o : over2) bad = bad || o;
+    }
+    if (bad) return drop(ICF_E_INDEX, "a slot/row/node index exceeds the declared size");
+    if (err) {
+        const std::string why = ctx->err;
+        return drop(err, why.c_str());
+    }
     return 0;
 }
 
@@ -1094,18 +1112,17 @@ bool vals_force_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const SlotMap 
     if (mv->keys) return false;
     if (mv->nlaunch == 0 && mf->nlaunch == 0) return true;
     const bool mixed = ctx->precision == ICF_MIXED, iso = ctx->hc.iso != 0;
-    const int k = mixed ? 0 : 1;
     double *ts = (double *)ctx->tsum.p;
     const int c = tune_begin(ctx, false, !mixed, mv->nlaunch);
     const int ilv = shape_begin(ctx, ICF_SHAPE_ORDER, mv->nlaunch);
     with_cand(c, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
-        const int nch = mv->nlaunch ? mv->nchunks[c][k] : 0;
+        const int nch = (int)blocks_for(mv->nlaunch, K);
         const int nbf = mf->nlaunch ? round8(blocks_for(mf->nlaunch, K)) : 0;
         const dim3 g(interleave2_grid(nbf, nch)), b(K);   // not empty: at least one map has keys
 #define ICF_VF(MX, IS, L, NAME)                                                                                   \
-    LAUNCH(ctx, NAME, (k_vals_force_fused<MX, IS, L, K, S>), g, b, nbf, mv->off, mv->codes, mv->chunks[c][k], nch, A, \
-           mf->off, mf->codes, mf->keys, mf->nlaunch, F, ns, st, ts, ilv)
+    LAUNCH(ctx, NAME, (k_vals_force_fused<MX, IS, L, K, S>), g, b, nbf, mv->loff, mv->codes, mv->nlaunch, nch, A, \
+           mf->loff, mf->codes, mf->keys, mf->nlaunch, F, ns, st, ts, ilv)
         if (mixed && iso) ICF_VF(true, true, float, "k_vals_force<mixed,iso>");
         else if (mixed) ICF_VF(true, false, float, "k_vals_force<mixed,gen>");
         else if (iso) ICF_VF(false, true, double, "k_vals_force<fp64,iso>");
@@ -1127,12 +1144,11 @@ bool vals_force_rhs_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const Slot
     if (mv->keys || !mr->merge_ok || !mr->node_row) return false;
     if (mv->nlaunch == 0 && mf->nlaunch == 0 && nCZs == 0) return true;
     const bool mixed = ctx->precision == ICF_MIXED, iso = ctx->hc.iso != 0;
-    const int k = mixed ? 0 : 1;
     const int c = tune_begin(ctx, false, !mixed, mv->nlaunch);
     const int ilv = shape_begin(ctx, ICF_SHAPE_ORDER, mv->nlaunch);
     with_cand(c, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
-        const int nch = mv->nlaunch ? mv->nchunks[c][k] : 0;
+        const int nch = (int)blocks_for(mv->nlaunch, K);
         const int nbf = mf->nlaunch ? round8(blocks_for(mf->nlaunch, K)) : 0;
         // the CZ counters' workgroups: per specimen in a batched call (one or more specimens
         // each), else strided over all CZs
@@ -1142,8 +1158,8 @@ bool vals_force_rhs_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const Slot
                                  : nCZs ? round8(std::min<long long>(blocks_for(nCZs, K), 64)) : 0;
         const dim3 g(nbc + interleave2_grid(nbf, nch)), bl(K);   // not empty: something has keys or CZs
 #define ICF_VFR(MX, IS, L, NAME)                                                                                   \
-    LAUNCH(ctx, NAME, (k_vals_force_rhs_fused<MX, IS, L, K, S>), g, bl, nbf, nbc, mv->off, mv->codes, mv->chunks[c][k], \
-           nch, A, mf->off, mf->codes, mf->keys, mf->nlaunch, F, ns, mr->node_row, mr->off, mr->codes, mr->cz_begin, \
+    LAUNCH(ctx, NAME, (k_vals_force_rhs_fused<MX, IS, L, K, S>), g, bl, nbf, nbc, mv->loff, mv->codes, mv->nlaunch, \
+           nch, A, mf->loff, mf->codes, mf->keys, mf->nlaunch, F, ns, mr->node_row, mr->off, mr->codes, mr->cz_begin, \
            b, dmg, fld, nCZs, counts, per_spec ? bt.cz_off : nullptr, bt.n, bt.spec_counts, st, ilv)
         if (mixed && iso) ICF_VFR(true, true, float, "k_vals_force_rhs<mixed,iso>");
         else if (mixed) ICF_VFR(true, false, float, "k_vals_force_rhs<mixed,gen>");
@@ -1165,17 +1181,16 @@ bool contact_sums_fused(icf_ctx *ctx, const SlotMap *mf, double *F, int ns, cons
     if (!mv->keys) return false;
     if (mf->nlaunch == 0 && mv->nlaunch == 0 && mr->nlaunch == 0) return true;
     const bool mixed = ctx->precision == ICF_MIXED;
-    const int k = mixed ? 0 : 1;
     const int c = tune_begin(ctx, true, !mixed, mv->nlaunch);
     with_cand(c, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
-        const int nch = mv->nlaunch ? mv->nchunks[c][k] : 0;
+        const int nch = (int)blocks_for(mv->nlaunch, K);
         const int nb0 = mf->nlaunch ? round8(blocks_for(mf->nlaunch, K)) : 0, nb1 = round8(nch);
         const int nb2 = mr->nlaunch ? (int)blocks_for(mr->nlaunch, K) : 0;
         const dim3 g(nb0 + nb1 + nb2), bl(K);
 #define ICF_CS(MX, L, NAME)                                                                                       \
-    LAUNCH(ctx, NAME, (k_contact_sums<MX, L, K, S>), g, bl, nb0, nb1, mf->off, mf->codes, mf->keys, mf->nlaunch, F, ns, \
-           mv->off, mv->codes, mv->keys, mv->chunks[c][k], nch, A, mr->off, mr->codes, mr->keys, mr->nlaunch, b, st)
+    LAUNCH(ctx, NAME, (k_contact_sums<MX, L, K, S>), g, bl, nb0, nb1, mf->loff, mf->codes, mf->keys, mf->nlaunch, F, ns, \
+           mv->loff, mv->codes, mv->keys, mv->nlaunch, A, mr->loff, mr->codes, mr->keys, mr->nlaunch, b, st)
         if (mixed) ICF_CS(true, float, "k_contact_sums<mixed>");
         else ICF_CS(false, double, "k_contact_sums<fp64>");
 #undef ICF_CS
@@ -1204,13 +1219,12 @@ template <bool MX, bool IS, bool ACC, typename L>
 void vals_kernel(icf_ctx *ctx, const char *name, const SlotMap *m, double *A, const Stage &sv)
 {
     const int k = sizeof(L) == 4 ? 0 : 1;
-    if (m->nlaunch == 0) return;   // then no chunks for any key limit
+    if (m->nlaunch == 0) return;
     const int c = tune_begin(ctx, ACC, k == 1, m->nlaunch);
     with_cand(c, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
-        const int n = m->nchunks[c][k];
-        LAUNCH(ctx, name, (k_reduce_vals<MX, IS, ACC, L, K, S>), dim3(n), dim3(K), m->off, m->codes, m->keys,
-               m->chunks[c][k], n, A, sv);
+        LAUNCH(ctx, name, (k_reduce_vals<MX, IS, ACC, L, K, S>), dim3(blocks_for(m->nlaunch, K)), dim3(K), m->loff,
+               m->codes, m->keys, m->nlaunch, A, sv);
     });
     tune_end(ctx, ACC, k == 1);
 }
@@ -1252,10 +1266,10 @@ void launch_vec3(icf_ctx *ctx, const SlotMap *m, double *out, int comp_stride, i
     dim3 g(blocks_for(n, 256)), b(256);
     const bool force = elem_stride == 1;
     if (accumulate)
-        LAUNCH(ctx, force ? "k_reduce_vec3<force,acc>" : "k_reduce_vec3<rhs,acc>", k_reduce_vec3<true>, g, b, m->off,
+        LAUNCH(ctx, force ? "k_reduce_vec3<force,acc>" : "k_reduce_vec3<rhs,acc>", k_reduce_vec3<true>, g, b, m->loff,
                m->codes, keys, n, out, comp_stride, elem_stride, sv);
     else
-        LAUNCH(ctx, force ? "k_reduce_vec3<force>" : "k_reduce_vec3<rhs>", k_reduce_vec3<false>, g, b, m->off,
+        LAUNCH(ctx, force ? "k_reduce_vec3<force>" : "k_reduce_vec3<rhs>", k_reduce_vec3<false>, g, b, m->loff,
                m->codes, keys, n, out, comp_stride, elem_stride, sv);
 }
 
@@ -1297,7 +1311,7 @@ int icf_create(int device, icf_ctx **out)
     ctx->cur = ctx->stream;
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev0);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev1);
-    if (e == hipSuccess) e = hipMalloc(&ctx->small, 8 * sizeof(int));
+    if (e == hipSuccess) e = hipMalloc(&ctx->small, 16 * sizeof(int));
     if (e == hipSuccess) e = hipMalloc(&ctx->rep_dev, REPORT_WORDS * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(ctx->rep_dev, 0, REPORT_WORDS * sizeof(unsigned));
     if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->rep_host, REPORT_WORDS * sizeof(unsigned), hipHostMallocMapped);
@@ -1321,7 +1335,7 @@ int icf_destroy(icf_ctx *ctx)
     DevBuf *bufs[] = {&ctx->tet_rhs, &ctx->tet_tan, &ctx->cz_rhs, &ctx->cz_tan, &ctx->ct,   &ctx->scan_tmp,
                       &ctx->pat_a,   &ctx->pat_b,   &ctx->bp_f,   &ctx->bp_i, &ctx->bp_l, &ctx->bp_c,
                       &ctx->tsum,    &ctx->ct_f,    &ctx->adj.off, &ctx->adj.ids, &ctx->batch.d,
-                      &ctx->patc.snap, &ctx->patc.keys, &ctx->bp_g};
+                      &ctx->patc.snap, &ctx->patc.keys, &ctx->bp_g, &ctx->map_cnt, &ctx->map_rank, &ctx->map_sums};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->small) (void)hipFree(ctx->small);
@@ -1811,13 +1825,11 @@ int icf_elem_force(icf_ctx *ctx, const int *ie, double *dn, double h, double *A,
     if (nElems == 0) return 0;
     OnLane ln(ctx, 0, everything);
     if (ln.err) return ln.err;
-    SlotMap *mv, *mr, *mf;
-    std::vector<SrcKey> sv{{KIND_TET, ie, nElems, el_stride, EL_SLOTS, 16}};
-    std::vector<SrcKey> sr{{KIND_TET, ie, nElems, el_stride, EL_ROWS, 4}};
-    std::vector<SrcKey> sfv{{KIND_TET, ie, nElems, el_stride, EL_NODES, 4}};
-    if (int r = get_map(ctx, TGT_VALS, -1, sv, &mv)) return r;
-    if (int r = get_map(ctx, TGT_RHS, -1, sr, &mr)) return r;
-    if (int r = get_map(ctx, TGT_FORCE, -1, sfv, &mf)) return r;
+    std::vector<MapReq> req{{TGT_VALS, -1, {{KIND_TET, ie, nElems, el_stride, EL_SLOTS, 16}}},
+                            {TGT_RHS, -1, {{KIND_TET, ie, nElems, el_stride, EL_ROWS, 4}}},
+                            {TGT_FORCE, -1, {{KIND_TET, ie, nElems, el_stride, EL_NODES, 4}}}};
+    if (int r = get_maps(ctx, req)) return r;
+    SlotMap *mv = req[0].map, *mr = req[1].map, *mf = req[2].map;
     Timer tm(ctx);
     if (int r = stage_tets(ctx, ie, dn, nElems, el_stride, nd_stride)) return r;
     Stage st = make_stage(ctx, h);
@@ -1839,11 +1851,10 @@ int icf_cz_force(icf_ctx *ctx, double *dcz, int *icz, double *dn, double *A, dou
     if (nCZs == 0) return 0;
     OnLane ln(ctx, 0, everything);
     if (ln.err) return ln.err;
-    SlotMap *mv, *mr;
-    std::vector<SrcKey> sv{{KIND_CZ, icz, nCZs, cz_stride, CZI_SLOTS, 36}};
-    std::vector<SrcKey> sr{{KIND_CZ, icz, nCZs, cz_stride, CZI_ROWS, 6}};
-    if (int r = get_map(ctx, TGT_VALS, -1, sv, &mv)) return r;
-    if (int r = get_map(ctx, TGT_RHS, -1, sr, &mr)) return r;
+    std::vector<MapReq> req{{TGT_VALS, -1, {{KIND_CZ, icz, nCZs, cz_stride, CZI_SLOTS, 36}}},
+                            {TGT_RHS, -1, {{KIND_CZ, icz, nCZs, cz_stride, CZI_ROWS, 6}}}};
+    if (int r = get_maps(ctx, req)) return r;
+    SlotMap *mv = req[0].map, *mr = req[1].map;
     Timer tm(ctx);
     if (int r = stage_czs(ctx, dcz, icz, dn, nCZs, cz_stride, nd_stride)) return r;
     Stage st = make_stage(ctx, h);
@@ -2019,13 +2030,11 @@ int icf_collision_response(icf_ctx *ctx, const int *icr, double *dn, double h, d
     if (bad_units(nImpacts, cr_stride) || nd_stride < 0 || (nImpacts && (!icr || !dn || !A || !b)))
         return fail(ctx, ICF_E_INVALID, "icf_collision_response: invalid argument");
     if (nImpacts == 0) return 0;
-    SlotMap *mv, *mr, *mf;
-    std::vector<SrcKey> sv{{KIND_CONTACT, icr, nImpacts, cr_stride, CR_SLOTS, 16}};
-    std::vector<SrcKey> sr{{KIND_CONTACT, icr, nImpacts, cr_stride, CR_ROWS, 4}};
-    std::vector<SrcKey> sfv{{KIND_CONTACT, icr, nImpacts, cr_stride, CR_NODES, 4}};
-    if (int r = get_map(ctx, TGT_VALS, -1, sv, &mv)) return r;
-    if (int r = get_map(ctx, TGT_RHS, -1, sr, &mr)) return r;
-    if (int r = get_map(ctx, TGT_FORCE, -1, sfv, &mf)) return r;
+    std::vector<MapReq> req{{TGT_VALS, -1, {{KIND_CONTACT, icr, nImpacts, cr_stride, CR_SLOTS, 16}}},
+                            {TGT_RHS, -1, {{KIND_CONTACT, icr, nImpacts, cr_stride, CR_ROWS, 4}}},
+                            {TGT_FORCE, -1, {{KIND_CONTACT, icr, nImpacts, cr_stride, CR_NODES, 4}}}};
+    if (int r = get_maps(ctx, req)) return r;
+    SlotMap *mv = req[0].map, *mr = req[1].map, *mf = req[2].map;
     const bool mixed = ctx->precision == ICF_MIXED;
     if (int r = grow(ctx, ctx->ct, (mixed ? sizeof(float) : sizeof(double)) * CT_TAN_REC * (size_t)nImpacts)) return r;
     if (int r = grow(ctx, ctx->ct_f, sizeof(double) * CT_F_REC * (size_t)nImpacts)) return r;
@@ -2089,10 +2098,10 @@ int icf_sum_int(icf_ctx *ctx, const int *d, int n, int *out)
     return 0;
 }
 
-// The fused call; map_ids (optional) receives the ids of its value and rhs maps.
+// The fused call.
 static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride, double *dcz, int *icz, int nCZs,
                          int cz_stride, double *dn, int nd_stride, double h, double *A, int nnzb, double *b, int N,
-                         int *nCZDamaged, int *nCZFailed, int *map_ids)
+                         int *nCZDamaged, int *nCZFailed)
 {
     if (int r = check_ctx(ctx)) return r;
     if (bad_units(nElems, el_stride) || bad_units(nCZs, cz_stride) || nd_stride < 0 || nnzb < 0 || N < 0 ||
@@ -2114,32 +2123,23 @@ static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride,
             .wr(b, 3 * (size_t)N);
     });
     if (ln.err) return ln.err;
-    std::vector<SrcKey> sv, sr, sfv;
+    std::vector<SrcKey> sv, sr;
     if (nElems) {
         sv.push_back({KIND_TET, ie, nElems, el_stride, EL_SLOTS, 16});
         sr.push_back({KIND_TET, ie, nElems, el_stride, EL_ROWS, 4});
-        sfv.push_back({KIND_TET, ie, nElems, el_stride, EL_NODES, 4});
     }
     if (nCZs) {
         sv.push_back({KIND_CZ, icz, nCZs, cz_stride, CZI_SLOTS, 36});
         sr.push_back({KIND_CZ, icz, nCZs, cz_stride, CZI_ROWS, 6});
     }
-    SlotMap *mv, *mr, *mf = nullptr;
-    if (int r = get_map(ctx, TGT_VALS, nnzb, sv, &mv)) return r;
-    if (int r = get_map(ctx, TGT_RHS, N, sr, &mr)) return r;
-    if (nElems)
-        if (int r = get_map(ctx, TGT_FORCE, -1, sfv, &mf)) return r;
-    if (map_ids) {
-        map_ids[0] = mv->id;
-        map_ids[1] = mr->id;
-    }
-    bool tsum = false;
-    if (mf) {
-        MapSrc tet{ie, nElems, el_stride, EL_NODES, 4, KIND_TET};
-        if (int r = get_tsum_link(ctx, mr, mf, tet, &tsum)) return r;
-        if (tsum)
-            if (int r = grow(ctx, ctx->tsum, sizeof(double) * 3 * (size_t)mf->nkeys)) return r;
-    }
+    std::vector<MapReq> req{{TGT_VALS, nnzb, sv}, {TGT_RHS, N, sr}};
+    if (nElems) req.push_back({TGT_FORCE, -1, {{KIND_TET, ie, nElems, el_stride, EL_NODES, 4}}});
+    const MapSrc tet{ie, nElems, el_stride, EL_NODES, 4, KIND_TET};
+    if (int r = get_maps(ctx, req, nElems ? &tet : nullptr)) return r;
+    SlotMap *mv = req[0].map, *mr = req[1].map, *mf = nElems ? req[2].map : nullptr;
+    const bool tsum = mf && mr->tsum_ok;
+    if (tsum)
+        if (int r = grow(ctx, ctx->tsum, sizeof(double) * 3 * (size_t)mf->nkeys)) return r;
     // buffers grow before any work is issued (growing synchronizes the context's stream)
     if (int r = stage_tets(ctx, ie, dn, 0, el_stride, nd_stride, nElems)) return r;
     if (int r = stage_czs(ctx, dcz, icz, dn, 0, cz_stride, nd_stride, nCZs)) return r;
@@ -2167,7 +2167,7 @@ static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride,
         if (!(fuse && vals_force_fused(ctx, mv, A, mf, F, nd_stride, st))) {
             launch_vals(ctx, mv, A, 0, st);
             LAUNCH(ctx, "k_reduce_vec3<force,acc>", (k_reduce_vec3<true, true>), dim3(blocks_for(mf->nlaunch, 256)),
-                   dim3(256), mf->off, mf->codes, mf->keys, mf->nlaunch, F, nd_stride, 1, st, (double *)ctx->tsum.p);
+                   dim3(256), mf->loff, mf->codes, mf->keys, mf->nlaunch, F, nd_stride, 1, st, (double *)ctx->tsum.p);
         }
         if (fuse && (N || nCZs)) {
             const int nbr = N ? (int)(blocks_for(N, 256) + 7) / 8 * 8 : 0;
@@ -2203,7 +2203,7 @@ int icf_assemble_elems_and_czs(icf_ctx *ctx, const int *ie, int nElems, int el_s
                                int N, int *nCZDamaged, int *nCZFailed)
 {
     return assemble_impl(ctx, ie, nElems, el_stride, dcz, icz, nCZs, cz_stride, dn, nd_stride, h, A, nnzb, b, N,
-                         nCZDamaged, nCZFailed, nullptr);
+                         nCZDamaged, nCZFailed);
 }
 
 int icf_assemble_batched(icf_ctx *ctx, const icf_worklist *wl, const int *ie, int el_stride, double *dcz, int *icz,
@@ -2267,7 +2267,7 @@ int icf_assemble_batched(icf_ctx *ctx, const icf_worklist *wl, const int *ie, in
     B.spec_counts = cnt;
     B.spec_counted = false;
     const int ra = assemble_impl(ctx, ie, nE, el_stride, dcz, icz, nC, cz_stride, dn, nd_stride, h, A, nnzb, b, N,
-                                 nullptr, nullptr, nullptr);
+                                 nullptr, nullptr);
     B.cz_off = nullptr;
     B.spec_counts = nullptr;
     if (ra) return ra;

@@ -43,91 +43,230 @@ __global__ __launch_bounds__(256) void k_map_maxkey(MapSrc s, int *__restrict__ 
     }
 }
 
-__global__ __launch_bounds__(256) void k_map_count(MapSrc s, int nkeys, int *__restrict__ count, int *__restrict__ err)
+// ---- building slot maps ----------------------------------------------------------------------
+// The maps a call needs and does not have are built together, in six launches and without a word
+// from the host in between: count (each contribution also takes its rank among its key's), block
+// sums, their scan, offsets with the lists of keys that have contributions, fill, sort.  Every
+// buffer is sized by what it could hold, so nothing waits for a count; the host reads the number
+// of keys to visit and the errors from the report, after one wait.  A Newton loop with contact
+// builds four maps in each iteration (the impacts change, and with them every slot), a step in
+// which CZs failed three: with the chunk tables of the value reductions laid out on the host and
+// allocations in between this took 16.9 + 6.5 ms in an iteration of the 384,000-tet compression,
+// 0.38 + 0.11 ms as it is.  The atomics of the count bound it (5.8M contributions), then the scattered
+// stores of the fill.
+constexpr int MAX_JOBS = 3, MAX_MAP_SRCS = 6;
+constexpr int SCAN_ITEMS = 8, SCAN_TILE = 256 * SCAN_ITEMS;
+struct MapJobs {
+    int njob, nsrc;
+    MapSrc src[MAX_MAP_SRCS];
+    int job[MAX_MAP_SRCS];              // the map a source belongs to
+    unsigned blk0[MAX_MAP_SRCS + 1];    // first workgroup of a source: nq rows of ceil(n / 256)
+    long long at[MAX_MAP_SRCS];         // the source's place in `rank`
+    int *snap[MAX_MAP_SRCS];            // copy of the source's fields, as they are counted
+    int nkeys[MAX_JOBS];
+    long long cnt0[MAX_JOBS];           // the map's place in `cnt` (nkeys counts)
+    unsigned tile0[MAX_JOBS + 1];       // first scan tile of a map
+    unsigned sort0[MAX_JOBS + 1];       // first sorting workgroup of a map
+    int *off[MAX_JOBS];                 // nkeys + 1: first code of each key
+    uint32_t *codes[MAX_JOBS];
+    int *keys[MAX_JOBS], *loff[MAX_JOBS];   // the keys with contributions and their first codes, or null
+};
+// words of the report (MAP_NLIST holds values: no other call's words are there)
+constexpr int MAP_ERR = 0, LINK_ERR = 8, SNAP_DIFF = 10, MAP_NLIST = 13;
+static_assert(MAP_NLIST + MAX_JOBS <= REPORT_WORDS, "report words");
+
+// Source, unit and field of this thread; false beyond the units.
+__device__ inline bool map_place(const MapJobs &J, int &k, int &u, int &q)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)s.n * s.nq) return;
-    const int q = (int)(i / s.n), u = (int)(i % s.n);
+    k = 0;
+    while (k + 1 < J.nsrc && blockIdx.x >= J.blk0[k + 1]) k++;
+    const unsigned b = blockIdx.x - J.blk0[k], nbx = ((unsigned)J.src[k].n + 255u) / 256u;
+    q = (int)(b / nbx);
+    u = (int)(b % nbx) * 256 + (int)threadIdx.x;
+    return u < J.src[k].n;
+}
+
+// cnt (zero on entry) += the contributions of each key; rank[i] = the contribution's place among
+// its key's, in no particular order.
+__global__ __launch_bounds__(256) void k_map_count(MapJobs J, int *__restrict__ cnt, int *__restrict__ rank, Report rep)
+{
+    int k, u, q;
+    if (!map_place(J, k, u, q)) return;
+    const MapSrc &s = J.src[k];
     const int key = s.base[u + (size_t)s.stride * (s.field0 + q)];
+    const size_t i = (size_t)q * s.n + u;
+    J.snap[k][i] = key;
     if (key < 0) return;
-    if (key >= nkeys) {
-        atomicOr(err, 1);
+    const int j = J.job[k];
+    if (key >= J.nkeys[j]) rep.set(MAP_ERR + j);
+    else rank[J.at[k] + i] = atomicAdd(&cnt[J.cnt0[j] + key], 1);
+}
+
+// Counts and keys with contributions travel through the scan together: (keys << 32) + count.
+__device__ inline unsigned long long scan_item(int c) { return c > 0 ? (1ULL << 32) + (unsigned)c : 0ULL; }
+
+// The map a scan tile belongs to, and the first key of the tile.
+__device__ inline int tile_job(const MapJobs &J, int &k0)
+{
+    int j = 0;
+    while (j + 1 < J.njob && blockIdx.x >= J.tile0[j + 1]) j++;
+    k0 = (int)(blockIdx.x - J.tile0[j]) * SCAN_TILE;
+    return j;
+}
+
+// Exclusive scan over the 256 threads of the workgroup; total in every thread.
+__device__ inline unsigned long long scan256(unsigned long long v, unsigned long long *part, unsigned long long &total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    unsigned long long x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) part[wave] = x;
+    __syncthreads();
+    unsigned long long before = 0;
+    total = 0;
+    for (int w = 0; w < 4; w++) {
+        if (w < wave) before += part[w];
+        total += part[w];
+    }
+    __syncthreads();
+    return before + x - v;
+}
+
+__global__ __launch_bounds__(256) void k_map_tiles(MapJobs J, const int *__restrict__ cnt,
+                                                   unsigned long long *__restrict__ sums)
+{
+    __shared__ unsigned long long part[4];
+    int k0;
+    const int j = tile_job(J, k0);
+    unsigned long long v = 0, total;
+    for (int r = 0; r < SCAN_ITEMS; r++) {
+        const int k = k0 + r * 256 + (int)threadIdx.x;
+        if (k < J.nkeys[j]) v += scan_item(cnt[J.cnt0[j] + k]);
+    }
+    (void)scan256(v, part, total);
+    if (threadIdx.x == 0) sums[blockIdx.x] = total;
+}
+
+// One workgroup: each map's tile sums become the tiles' starts; the totals end the offsets.
+__global__ __launch_bounds__(256) void k_map_scan(MapJobs J, unsigned long long *__restrict__ sums, Report rep)
+{
+    __shared__ unsigned long long part[4];
+    for (int j = 0; j < J.njob; j++) {
+        unsigned long long run = 0, total;
+        for (unsigned t0 = J.tile0[j]; t0 < J.tile0[j + 1]; t0 += 256) {
+            const unsigned t = t0 + threadIdx.x;
+            const unsigned long long v = t < J.tile0[j + 1] ? sums[t] : 0ULL;
+            const unsigned long long x = scan256(v, part, total);
+            if (t < J.tile0[j + 1]) sums[t] = run + x;
+            run += total;
+        }
+        if (threadIdx.x == 0) {
+            const int n = (int)(run >> 32), c = (int)(run & 0xffffffffULL);
+            J.off[j][J.nkeys[j]] = c;
+            if (J.loff[j]) J.loff[j][n] = c;
+            rep.put(MAP_NLIST + j, (unsigned)n);
+        }
+    }
+}
+
+// First code of every key, the list of keys with contributions; cnt is left zero for the next maps.
+__global__ __launch_bounds__(256) void k_map_offsets(MapJobs J, int *__restrict__ cnt,
+                                                     const unsigned long long *__restrict__ sums)
+{
+    __shared__ unsigned long long part[4];
+    int k0;
+    const int j = tile_job(J, k0);
+    unsigned long long run = sums[blockIdx.x], total;
+    for (int r = 0; r < SCAN_ITEMS; r++) {
+        const int k = k0 + r * 256 + (int)threadIdx.x;
+        const bool in = k < J.nkeys[j];
+        int c = 0;
+        if (in) {
+            c = cnt[J.cnt0[j] + k];
+            if (c) cnt[J.cnt0[j] + k] = 0;
+        }
+        const unsigned long long x = run + scan256(scan_item(c), part, total);
+        run += total;
+        if (!in) continue;
+        const int first = (int)(x & 0xffffffffULL);
+        J.off[j][k] = first;
+        if (c && J.keys[j]) {
+            const int p = (int)(x >> 32);
+            J.keys[j][p] = k;
+            J.loff[j][p] = first;
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_map_fill(MapJobs J, const int *__restrict__ rank)
+{
+    int k, u, q;
+    if (!map_place(J, k, u, q)) return;
+    const size_t i = (size_t)q * J.src[k].n + u;
+    const int key = J.snap[k][i], j = J.job[k];
+    if (key < 0 || key >= J.nkeys[j]) return;
+    J.codes[j][J.off[j][key] + rank[J.at[k] + i]] = make_code(J.src[k].kind, (uint32_t)u, (uint32_t)q);
+}
+
+__device__ inline void sort_codes(uint32_t *c, int b, int e)
+{
+    for (int i = b + 1; i < e; i++) {
+        const uint32_t v = c[i];
+        int p = i - 1;
+        while (p >= b && c[p] > v) {
+            c[p + 1] = c[p];
+            p--;
+        }
+        c[p + 1] = v;
+    }
+}
+
+// Each key's codes ascending: 256 consecutive keys per workgroup, whose codes are one run, sorted
+// in LDS by one thread per key (insertion: a block receives a few tens of contributions at most);
+// in place where the run does not fit.  In memory the same sort took 219 us for the four maps of
+// the 384,000-tet compression, a chain of dependent loads and stores per key.
+constexpr int SORT_CAP = 4096;
+__global__ __launch_bounds__(256) void k_map_sort(MapJobs J)
+{
+    __shared__ uint32_t lds[SORT_CAP];
+    int j = 0;
+    while (j + 1 < J.njob && blockIdx.x >= J.sort0[j + 1]) j++;
+    const int n = J.nkeys[j], k0 = (int)(blockIdx.x - J.sort0[j]) * 256, k1 = min(k0 + 256, n);
+    const int *off = J.off[j];
+    uint32_t *codes = J.codes[j];
+    const int c0 = off[k0], c1 = off[k1], k = k0 + (int)threadIdx.x;
+    const int b = k < k1 ? off[k] : 0, e = k < k1 ? off[k + 1] : 0;
+    if (c1 - c0 > SORT_CAP) {
+        sort_codes(codes, b, e);
         return;
     }
-    atomicAdd(&count[key], 1);
+    for (int i = threadIdx.x; i < c1 - c0; i += 256) lds[i] = codes[c0 + i];
+    __syncthreads();
+    if (e > b) sort_codes(lds, b - c0, e - c0);
+    __syncthreads();
+    for (int i = threadIdx.x; i < c1 - c0; i += 256) codes[c0 + i] = lds[i];
 }
 
-__global__ __launch_bounds__(256) void k_map_fill(MapSrc s, int nkeys, const int *__restrict__ off,
-                                                  int *__restrict__ cursor, uint32_t *__restrict__ codes)
+// Whether a source's fields still are what the map was built from.
+__global__ __launch_bounds__(256) void k_snap_cmp(MapJobs J, Report rep)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)s.n * s.nq) return;
-    const int q = (int)(i / s.n), u = (int)(i % s.n);
-    const int key = s.base[u + (size_t)s.stride * (s.field0 + q)];
-    if (key < 0 || key >= nkeys) return;
-    const int pos = off[key] + atomicAdd(&cursor[key], 1);
-    codes[pos] = make_code(s.kind, (uint32_t)u, (uint32_t)q);
-}
-
-// Sort each key's codes ascending (insertion sort; lists are short: a BCSR slot receives
-// at most a few tens of contributions).
-__global__ __launch_bounds__(256) void k_map_sort(const int *__restrict__ off, uint32_t *__restrict__ codes, int nkeys)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nkeys) return;
-    const int b = off[k], e = off[k + 1];
-    for (int i = b + 1; i < e; i++) {
-        const uint32_t v = codes[i];
-        int j = i - 1;
-        while (j >= b && codes[j] > v) {
-            codes[j + 1] = codes[j];
-            j--;
-        }
-        codes[j + 1] = v;
-    }
-}
-
-// Copy of a source's key fields (q-major), and its comparison with the current fields.
-__global__ __launch_bounds__(256) void k_snap_copy(MapSrc s, int *__restrict__ snap)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)s.n * s.nq) return;
-    const int q = (int)(i / s.n), u = (int)(i % s.n);
-    snap[i] = s.base[u + (size_t)s.stride * (s.field0 + q)];
-}
-
-__global__ __launch_bounds__(256) void k_snap_cmp(MapSrc s, const int *__restrict__ snap, int *__restrict__ diff)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)s.n * s.nq) return;
-    const int q = (int)(i / s.n), u = (int)(i % s.n);
-    if (snap[i] != s.base[u + (size_t)s.stride * (s.field0 + q)]) atomicOr(diff, 1);
-}
-
-// flag[k] = 1 if key k has contributions
-__global__ __launch_bounds__(256) void k_map_flag(const int *__restrict__ cnt, int nkeys, int *__restrict__ flag)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nkeys) flag[k] = cnt[k] > 0;
-}
-
-// keys[pos[k]] = k for every key with contributions (pos = exclusive scan of the flags)
-__global__ __launch_bounds__(256) void k_map_compact(const int *__restrict__ flag, const int *__restrict__ pos,
-                                                     int nkeys, int *__restrict__ keys)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nkeys && flag[k]) keys[pos[k]] = k;
+    int k, u, q;
+    if (!map_place(J, k, u, q)) return;
+    const MapSrc &s = J.src[k];
+    if (J.snap[k][(size_t)q * s.n + u] != s.base[u + (size_t)s.stride * (s.field0 + q)]) rep.set(SNAP_DIFF + J.job[k]);
 }
 
 // Chunk shape of the staged BCSR-value reduction: keys per workgroup (one thread each; the
-// workgroup size) and contributions staged in LDS, STAGE FP32 or STAGE/2 FP64 values x 9 per
-// key.  STAGE = 2 is the least that still holds the chunk's output blocks (9 doubles per key)
+// workgroup size) and contributions staged in LDS at a time, STAGE FP32 or STAGE/2 FP64 values x 9
+// per key.  STAGE = 2 is the least that still holds the chunk's output blocks (9 doubles per key)
 // when they leave through the same LDS; a smaller buffer lets more workgroups share a CU, a
-// larger one ends fewer chunks on the contribution limit (keys average about 5
-// contributions).  A value map has a chunk table for every candidate shape and staging type,
-// and the library's autotuner picks the shape per role (overwrite or accumulate map, FP32 or
-// FP64 staging) by timing the candidates.  Every shape gives the same values: each key's
-// contributions are added in list order whatever the chunking.
+// larger one takes the contributions (about 5 per key) in fewer rounds.  The library's autotuner
+// picks the shape per role (overwrite or accumulate map, FP32 or FP64 staging) by timing the
+// candidates.  Every shape gives the same values: each key's contributions are added in list
+// order whatever the chunking.
 constexpr int NKC = 4, NSC = 2, NCAND = NKC * NSC;       // candidate key limits x stagings
 constexpr int KEY_CANDS[NKC] = {64, 128, 256, 512};
 constexpr int STAGE_CANDS[NSC] = {2, 3};
@@ -190,32 +329,28 @@ __device__ inline void contrib9(const Stage &sv, uint32_t code, L v[9])
     for (int k = 0; k < 9; k++) v[k] = (L)acc[k];
 }
 
-// Phase 2 for BCSR values, one workgroup per chunk of consecutive keys (at most KEYS keys and
-// flat_cap<L, KEYS>() contributions; the chunk table, built with the map, holds each
-// chunk's first list and code positions).  The chunk's contributions are contiguous in
-// `codes`: first every thread evaluates contributions
-// (uniform work across lanes) into LDS, then one thread per key adds its contributions from
-// LDS in list order into an FP64 accumulator and writes the block.  The values and their
-// order are those of a sequential loop over the key's list, so the result does not depend
-// on the chunking.
-//   keys   null: chunk positions are keys; else keys[position] (accumulate mode)
+// Phase 2 for BCSR values, one workgroup per KEYS consecutive list positions.  The chunk's
+// contributions are contiguous in `codes` and are taken in rounds of flat_cap: every thread
+// evaluates contributions (uniform work across lanes) into LDS, then one thread per key adds its
+// own of the round from LDS in list order into an FP64 accumulator.  The values and their order
+// are those of a sequential loop over the key's list, so the result does not depend on the
+// chunking.
+//   keys   null: list positions are keys; else keys[position] (accumulate mode)
+//   off    first code per list position
 //   ACC    add to A (single-kernel calls); otherwise overwrite, zero where nothing contributes
 // L is the staging type: float for tet and CZ blocks in mixed mode, double otherwise.
 template <bool MIXED, bool ISO, bool ACC, typename L, int KEYS, int STAGE>
 __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__restrict__ off,
-        const uint32_t *__restrict__ codes, const int *__restrict__ keys, const int2 *__restrict__ chunks, int nchunks,
-        double *__restrict__ A, Stage sv)
+        const uint32_t *__restrict__ codes, const int *__restrict__ keys, int nlist, double *__restrict__ A, Stage sv)
 {
     constexpr int CAP = flat_cap<L, KEYS, STAGE>();
     static_assert(CAP * 9 * sizeof(L) >= KEYS * 9 * sizeof(double), "output staging fits the LDS");
     constexpr int PER = (CAP + KEYS - 1) / KEYS;
     __shared__ L lds[CAP * 9];
-    const int ch = xcd_remap(bid_, nb_);
-    if (ch >= nchunks) return;
-    const int2 c0 = chunks[ch], c1 = chunks[ch + 1];
-    const int p0 = c0.x, p1 = c1.x, cb = c0.y, ce = c1.y;
-    const int nc = ce - cb;
-    const bool staged = nc <= CAP;
+    const int p0 = xcd_remap(bid_, nb_) * KEYS;
+    if (p0 >= nlist) return;
+    const int p1 = min(p0 + KEYS, nlist);
+    const int cb = off[p0], ce = off[p1];
     // this thread's key and its code range, loaded beside the chunk's codes
     const int p = p0 + threadIdx.x;
     const bool live = p < p1;
@@ -225,26 +360,28 @@ __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__rest
     for (int i = 0; i < 9; i++) acc[i] = 0.;
     if (live) {
         s = keys ? keys[p] : p;
-        b = off[s];
-        e = off[s + 1];
+        b = off[p];
+        e = off[p + 1];
         if (ACC) {   // the block's current values, also loaded before the contributions
             const double *src = A + (size_t)s * 9;
 #pragma unroll
             for (int i = 0; i < 9; i++) acc[i] = src[i];
         }
     }
-    if (staged) {
+    for (int c0 = cb; c0 < ce; c0 += CAP) {
+        const int c1 = min(c0 + CAP, ce);
         // codes first (coalesced), then the contributions, so their loads overlap
         uint32_t cd[PER];
 #pragma unroll
         for (int r = 0; r < PER; r++) {
-            const int i = threadIdx.x + r * KEYS;
-            cd[r] = i < nc ? codes[cb + i] : 0u;
+            const int i = c0 + threadIdx.x + r * KEYS;
+            cd[r] = i < c1 ? codes[i] : 0u;
         }
+        if (c0 != cb) __syncthreads();   // the previous round's values have been added
 #pragma unroll
         for (int r = 0; r < PER; r++) {
             const int i = threadIdx.x + r * KEYS;
-            if (i < nc) {
+            if (c0 + i < c1) {
                 L v[9];
                 contrib9<MIXED, ISO, L>(sv, cd[r], v);
 #pragma unroll
@@ -252,20 +389,10 @@ __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__rest
             }
         }
         __syncthreads();
-    }
-    if (live) {
-        if (staged) {
-            for (int c = b - cb; c < e - cb; c++) {
+        const int hi = min(e, c1) - c0;
+        for (int c = max(b, c0) - c0; c < hi; c++) {
 #pragma unroll
-                for (int k = 0; k < 9; k++) acc[k] += (double)lds[c * 9 + k];
-            }
-        } else {
-            for (int c = b; c < e; c++) {
-                L v[9];
-                contrib9<MIXED, ISO, L>(sv, codes[c], v);
-#pragma unroll
-                for (int k = 0; k < 9; k++) acc[k] += (double)v[k];
-            }
+            for (int k = 0; k < 9; k++) acc[k] += (double)lds[c * 9 + k];
         }
     }
     if (ACC) {
@@ -294,13 +421,14 @@ __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__rest
 
 template <bool MIXED, bool ISO, bool ACC, typename L, int KEYS, int STAGE>
 __global__ __launch_bounds__(KEYS) void k_reduce_vals(const int *__restrict__ off, const uint32_t *__restrict__ codes,
-                                                           const int *__restrict__ keys, const int2 *__restrict__ chunks,
-                                                           int nchunks, double *__restrict__ A, Stage sv)
+                                                      const int *__restrict__ keys, int nlist, double *__restrict__ A,
+                                                      Stage sv)
 {
-    reduce_vals<MIXED, ISO, ACC, L, KEYS, STAGE>(blockIdx.x, gridDim.x, off, codes, keys, chunks, nchunks, A, sv);
+    reduce_vals<MIXED, ISO, ACC, L, KEYS, STAGE>(blockIdx.x, gridDim.x, off, codes, keys, nlist, A, sv);
 }
 
-// Phase 2 for rhs rows (b[row*3+k]) or node forces (dn[node + ns*(F+k)]): one thread per key.
+// Phase 2 for rhs rows (b[row*3+k]) or node forces (dn[node + ns*(F+k)]): one thread per list
+// position (off: first code per position).
 // TSUM (node forces of the fused call): the sum of the key's contributions from zero is also
 // written to tsum[3 key .. 3 key + 2], from which k_reduce_rhs_tsum starts the rhs rows.
 template <bool ACC, bool TSUM>
@@ -311,7 +439,7 @@ __device__ __forceinline__ void reduce_vec3(int bid_, int nb_, const int *__rest
     const int t = xcd_remap(bid_, nb_) * blockDim.x + threadIdx.x;
     if (t >= nkeys) return;
     const int s = keys ? keys[t] : t;
-    const int b = off[s], e = off[s + 1];
+    const int b = off[t], e = off[t + 1];
     double *dst = out + (size_t)s * elem_stride;
     double a0, a1, a2, t0 = 0., t1 = 0., t2 = 0.;
     if (ACC) {
@@ -364,7 +492,7 @@ __device__ __forceinline__ void reduce_force_rhs(int bid_, int nb_, const int *_
     const int t = xcd_remap(bid_, nb_) * blockDim.x + threadIdx.x;
     if (t >= nfkeys) return;
     const int s = fkeys ? fkeys[t] : t;
-    const int b = foff[s], e = foff[s + 1];
+    const int b = foff[t], e = foff[t + 1];
     const int r = node_row[s];
     double *dst = F + s;
     double a0 = dst[0], a1 = dst[ns], a2 = dst[2 * (size_t)ns], t0 = 0., t1 = 0., t2 = 0.;
@@ -410,13 +538,14 @@ __global__ __launch_bounds__(256) void k_reduce_vec3(const int *__restrict__ off
 }
 
 // For each rhs row r of the fused call: the length of its leading run of tet codes and the
-// node those tets share.  The row's tet contributions must be exactly the force key's list
-// of that node (same codes, same order); any other case sets *err.
+// node those tets share; node_row (-1 before) gets the row of each such node.  The row's tet
+// contributions must be exactly the force key's list of that node (same codes, same order), else
+// LINK_ERR is set; a row without a tet node, or a node with two rows, sets LINK_ERR + 1.
 __global__ __launch_bounds__(256) void k_rhs_check(const int *__restrict__ roff, const uint32_t *__restrict__ rcodes,
                                                    int N, const int *__restrict__ foff,
                                                    const uint32_t *__restrict__ fcodes, int nfkeys, MapSrc tet,
                                                    int *__restrict__ row_node, int *__restrict__ cz_begin,
-                                                   int *__restrict__ err)
+                                                   int *__restrict__ node_row, Report rep)
 {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= N) return;
@@ -426,33 +555,21 @@ __global__ __launch_bounds__(256) void k_rhs_check(const int *__restrict__ roff,
     cz_begin[r] = b + L;
     if (L == 0) {
         row_node[r] = -1;
+        rep.set(LINK_ERR + 1);
         return;
     }
     const uint32_t c0 = rcodes[b];
     const int u = (int)code_unit(c0), q = (int)code_q(c0);
     const int n = (u < tet.n && q < 4) ? tet.base[u + (size_t)tet.stride * (tet.field0 + q)] : -1;
-    if (n < 0 || n >= nfkeys || foff[n + 1] - foff[n] != L) {
-        atomicOr(err, 1);
+    bool ok = n >= 0 && n < nfkeys && foff[n + 1] - foff[n] == L;
+    const int fb = ok ? foff[n] : 0;
+    for (int k = 0; ok && k < L; k++) ok = fcodes[fb + k] == rcodes[b + k];
+    if (!ok) {
+        rep.set(LINK_ERR);
         return;
     }
-    const int fb = foff[n];
-    for (int k = 0; k < L; k++)
-        if (fcodes[fb + k] != rcodes[b + k]) {
-            atomicOr(err, 1);
-            return;
-        }
     row_node[r] = n;
-}
-
-// node_row[row_node[r]] = r for every rhs row r (node_row filled with -1 before).  A row
-// without a tet node, or a node with two rows, sets *err.
-__global__ __launch_bounds__(256) void k_node_row(const int *__restrict__ row_node, int N, int *__restrict__ node_row,
-                                                  int *__restrict__ err)
-{
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= N) return;
-    const int n = row_node[r];
-    if (n < 0 || atomicExch(node_row + n, r) != -1) atomicOr(err, 1);
+    if (atomicExch(node_row + n, r) != -1) rep.set(LINK_ERR + 1);
 }
 
 // rhs rows of the fused call: the node's tet sum (k_reduce_vec3 TSUM), then the row's CZ
