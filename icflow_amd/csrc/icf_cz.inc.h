@@ -10,7 +10,7 @@
 //    one pow per factor;
 //  - B = [s (x) I3, -s (x) I3] (ModelPrms.cs:324-349), so the 18x18 tangent is
 //    K_ab = sgn_a sgn_b sum_gp s_a,gp s_b,gp Q_gp with Q_gp = (w a_J) R^T T_d R; phase 1
-//    stages the three symmetric Q_gp (18 values), phase 2 forms each block from them.
+//    stages the six distinct symmetric sums (36 values), phase 2 only picks one and its sign.
 #pragma once
 
 namespace icf {
@@ -24,11 +24,28 @@ __device__ inline void pow3(double x, double e, double &p0, double &p1, double &
         double r = 1.0 / x;
         p1 = p0 * r;
         p2 = p1 * r;
-    } else {
-        p0 = pow(x, e);
-        p1 = pow(x, e - 1.0);
+    } else if (x == 0.0) {
+        auto at0 = [](double k) { return k > 0.0 ? 0.0 : k == 0.0 ? 1.0 : __builtin_inf(); };
+        p0 = at0(e);
+        p1 = at0(e - 1.0);
+        p2 = at0(e - 2.0);
+    } else {               // negative: real for integer exponents only
         p2 = pow(x, e - 2.0);
+        p1 = p2 * x;
+        p0 = p1 * x;
     }
+}
+
+// x^n, x^(n-1), x^(n-2) for an integer n >= 2 (the same for every lane): products, at most as many
+// rounding errors as exp(n log x) has and a twentieth of its instructions.  The shape parameters
+// alpha and beta are small integers as a rule; the two logarithms and exponentials they took were
+// a quarter of a Gauss point's work, and the CZs' is what keeps the VALUs of phase 1 busy.
+__device__ inline void pow3_int(double x, int n, double &p0, double &p1, double &p2)
+{
+    p2 = 1.0;
+    for (int k = 2; k < n; k++) p2 *= x;
+    p1 = p2 * x;
+    p0 = p1 * x;
 }
 
 // Powers of one direction of the PPR potential at one opening value.
@@ -46,7 +63,8 @@ __device__ __attribute__((always_inline)) inline PprPow ppr_pow_n(double Dn)
         return r;
     }
     double d = Dn / g_c.deln;
-    pow3(1.0 - d, g_c.alpha, r.a0, r.a1, r.a2);
+    if (g_c.alpha_n) pow3_int(1.0 - d, g_c.alpha_n, r.a0, r.a1, r.a2);
+    else pow3(1.0 - d, g_c.alpha, r.a0, r.a1, r.a2);
     pow3(g_c.pm_alpha + d, g_c.p_m, r.b0, r.b1, r.b2);
     return r;
 }
@@ -60,7 +78,8 @@ __device__ __attribute__((always_inline)) inline PprPow ppr_pow_t(double Dt)
         return r;
     }
     double d = Dt / g_c.delt;
-    pow3(1.0 - d, g_c.beta, r.a0, r.a1, r.a2);
+    if (g_c.beta_n) pow3_int(1.0 - d, g_c.beta_n, r.a0, r.a1, r.a2);
+    else pow3(1.0 - d, g_c.beta, r.a0, r.a1, r.a2);
     pow3(g_c.pn_beta + d, g_c.p_n, r.b0, r.b1, r.b2);
     return r;
 }
@@ -226,22 +245,16 @@ __device__ inline void cz_frame(const double p[9], double R[9], double &area)
     R[3] = r0 / lr; R[4] = r1 / lr; R[5] = r2 / lr;
 }
 
-// Phase 2: add tangent block (a,b), a,b in 0..5, of CZ record `rec` to acc.
-template <typename T>
-__device__ inline void cz_block(double acc[9], const T *__restrict__ rec, int a, int b)
+// Phase 2: a tangent block from its pair's six values.
+template <typename T, typename L>
+__device__ inline void cz_spread(const T c[6], bool neg, L v[9])
 {
-    const int ia = a % 3, ib = b % 3;
-    const T sg = ((a < 3) == (b < 3)) ? (T)1 : (T)-1;
-    T blk[6] = {0, 0, 0, 0, 0, 0};
+    T s[6];
 #pragma unroll
-    for (int gp = 0; gp < 3; gp++) {
-        const T w = sg * (T)g_c.sf[ia * 3 + gp] * (T)g_c.sf[ib * 3 + gp];
-#pragma unroll
-        for (int q = 0; q < 6; q++) blk[q] += w * rec[6 * gp + q];
-    }
-    acc[0] += (double)blk[0]; acc[1] += (double)blk[1]; acc[2] += (double)blk[2];
-    acc[3] += (double)blk[1]; acc[4] += (double)blk[3]; acc[5] += (double)blk[4];
-    acc[6] += (double)blk[2]; acc[7] += (double)blk[4]; acc[8] += (double)blk[5];
+    for (int k = 0; k < 6; k++) s[k] = neg ? -c[k] : c[k];
+    v[0] = (L)s[0]; v[1] = (L)s[1]; v[2] = (L)s[2];
+    v[3] = (L)s[1]; v[4] = (L)s[3]; v[5] = (L)s[4];
+    v[6] = (L)s[2]; v[7] = (L)s[4]; v[8] = (L)s[5];
 }
 
 }  // namespace icf

@@ -3,9 +3,15 @@
 // Restates kczCZForce (cz_kernels9/cz_kernels.h:210-434).  Each CZ is shared by three lanes of
 // a wavefront, one per Gauss point (21 CZs per 64-lane wave, lane 63 idle).  All three lanes
 // compute the midplane frame and the local top-bottom differences (cheap, identical); each
-// evaluates its own Gauss point's opening, PPR law, traction and tangent, writes its own
-// Q_gp into the tangent record, and the per-CZ results are combined with wavefront shuffles
-// in Gauss-point order 0, 1, 2 -- the order in which the reference accumulates them.
+// evaluates its own Gauss point's opening, PPR law, traction and tangent, and the per-CZ
+// results are combined with wavefront shuffles in Gauss-point order 0, 1, 2 -- the order in which
+// the reference accumulates them.  Each lane forms two of the six node-pair blocks of the tangent
+// record from the three Q_gp: a block is read from there with two 16-byte loads by the instructions
+// that read a tet's, where forming it from the Q_gp took nine loads and 18 products for each of a
+// CZ's 21 contributions (12.7M -> 6.5M load instructions in phase 2 on 256 batched specimens).  The
+// residual record holds the top nodes only.  Phase 1 is bound by VALU work at three waves per SIMD
+// (the law's registers): 830,320 CZs take 187 us (218 before the integer powers and the shorter
+// record), beside 276 us for 4.26M tets.
 
 #pragma once
 
@@ -19,6 +25,7 @@ template <bool MIXED>
 __device__ __forceinline__ void cz_phase1(int bid_, int nb_, double *__restrict__ dcz, int *__restrict__ icz,
         const double *__restrict__ dn, int n, int cs, int ns, double *__restrict__ st_rhs, void *__restrict__ st_tan)
 {
+    using T = typename std::conditional<MIXED, float, double>::type;
     const int wl = threadIdx.x & 63;                              // lane in the wave
     const int wave = (bid_ * blockDim.x + threadIdx.x) >> 6;
     const int slot = wl / 3, gp = wl % 3;                         // CZ within the wave, Gauss point
@@ -154,23 +161,40 @@ __device__ __forceinline__ void cz_phase1(int bid_, int nb_, double *__restrict_
         }
         own[r] = ((0.0 + a0) + a1) + a2;
     }
+    // the pair blocks 2 gp and 2 gp + 1, from the rounded Q_gp
+    T pair[12];
+    {
+        T qa[3][6];
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            const T v = (T)q[k];
+            qa[0][k] = __shfl(v, l0, 64);
+            qa[1][k] = __shfl(v, l1, 64);
+            qa[2][k] = __shfl(v, l2, 64);
+        }
+#pragma unroll
+        for (int p = 0; p < 2; p++) {
+            T blk[6];
+#pragma unroll
+            for (int g = 0; g < 3; g++) {
+                // 0: 00 01, 1: 02 11, 2: 12 22
+                const T s0 = (T)g_c.sf[g], s1 = (T)g_c.sf[3 + g], s2 = (T)g_c.sf[6 + g];
+                const T w = gp == 0 ? (p ? s0 * s1 : s0 * s0) : gp == 1 ? (p ? s1 * s1 : s0 * s2) : (p ? s2 * s2 : s1 * s2);
+#pragma unroll
+                for (int k = 0; k < 6; k++) blk[k] = g ? fma(w, qa[g][k], blk[k]) : w * qa[g][k];
+            }
+#pragma unroll
+            for (int k = 0; k < 6; k++) pair[6 * p + k] = blk[k];
+        }
+    }
     if (!live) return;
     double *orhs = st_rhs + (size_t)u * CZ_RHS_REC;
+    T *tan = (T *)st_tan + (size_t)u * CZ_TAN_REC + 12 * gp;   // pairs 2 gp, 2 gp + 1
     if (!work || failed) {
 #pragma unroll
-        for (int r = 0; r < 3; r++) {
-            orhs[3 * gp + r] = 0.;
-            orhs[9 + 3 * gp + r] = 0.;
-        }
-        if (MIXED) {
-            float *t = (float *)st_tan + (size_t)u * CZ_TAN_REC + 6 * gp;
+        for (int r = 0; r < 3; r++) orhs[3 * gp + r] = 0.;
 #pragma unroll
-            for (int i = 0; i < 6; i++) t[i] = 0.f;
-        } else {
-            double *t = (double *)st_tan + (size_t)u * CZ_TAN_REC + 6 * gp;
-#pragma unroll
-            for (int i = 0; i < 6; i++) t[i] = 0.;
-        }
+        for (int i = 0; i < 12; i++) tan[i] = (T)0;
         if (!work) return;               // currently failed: no outputs at all (cz_kernels.h:219)
     }
     // tentative history and flags (cz_kernels.h:404-422): lane gp writes slot gp
@@ -189,19 +213,9 @@ __device__ __forceinline__ void cz_phase1(int bid_, int nb_, double *__restrict_
         dcz[u + cs * CZD_TT] = avgTt;
     }
 #pragma unroll
-    for (int r = 0; r < 3; r++) {
-        orhs[3 * gp + r] = own[r];
-        orhs[9 + 3 * gp + r] = -own[r];
-    }
-    if (MIXED) {
-        float *t = (float *)st_tan + (size_t)u * CZ_TAN_REC + 6 * gp;
+    for (int r = 0; r < 3; r++) orhs[3 * gp + r] = own[r];
 #pragma unroll
-        for (int i = 0; i < 6; i++) t[i] = (float)q[i];
-    } else {
-        double *t = (double *)st_tan + (size_t)u * CZ_TAN_REC + 6 * gp;
-#pragma unroll
-        for (int i = 0; i < 6; i++) t[i] = q[i];
-    }
+    for (int i = 0; i < 12; i++) tan[i] = pair[i];
 }
 
 template <bool MIXED>

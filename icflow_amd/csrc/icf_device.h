@@ -28,9 +28,34 @@ __host__ __device__ inline uint32_t make_code(uint32_t kind, uint32_t unit, uint
 {
     return (kind << 30) | (unit << 6) | q;
 }
+constexpr uint32_t CODE_NONE = 0xffffffffu;      // no contribution (kind 3 does not exist)
 __host__ __device__ inline uint32_t code_kind(uint32_t c) { return c >> 30; }
-__host__ __device__ inline uint32_t code_unit(uint32_t c) { return (c >> 6) & CODE_UNIT_MAX; }
+// The unit is hidden from the optimizer after the mask: knowing it to be 24 bits, the compiler
+// (ROCm 7.2) takes a record's address for a 24-bit product, drops the mask that such a product
+// would not need, and then emits the full-width v_mad_u64_u32 -- an address kind << 24 records off.
+__device__ inline uint32_t code_unit(uint32_t c)
+{
+    uint32_t u = (c >> 6) & CODE_UNIT_MAX;
+    asm("" : "+v"(u));
+    return u;
+}
 __host__ __device__ inline uint32_t code_q(uint32_t c) { return c & 63u; }
+
+// In the lists of BCSR blocks the local index of a CZ's block (a, b) = (q / 6, q % 6) is kept as
+// what its value needs: the pair of midplane nodes and whether the block is negated (top with
+// bottom nodes).
+__host__ __device__ inline int cz_pair(int ia, int ib)
+{
+    const int lo = ia < ib ? ia : ib, hi = ia < ib ? ib : ia;
+    return lo * 3 - lo * (lo - 1) / 2 + (hi - lo);   // 00 01 02 11 12 22
+}
+__device__ inline uint32_t czv_code(uint32_t q)
+{
+    const int a = (int)(q / 6), b = (int)(q % 6);
+    return (uint32_t)cz_pair(a % 3, b % 3) | ((a < 3) != (b < 3) ? 8u : 0u);
+}
+__device__ inline uint32_t czv_pair(uint32_t c) { return c & 7u; }
+__device__ inline bool czv_neg(uint32_t c) { return (c & 8u) != 0; }
 
 // ---- staged per-unit records (AoS, one record per unit) -----------------------------------
 // tet tangent, isotropic E: corotated gradients g~ = R g (12), rest volume V, 3 pad.
@@ -39,10 +64,11 @@ constexpr int TET_ISO_REC = 16;
 constexpr int TET_GEN_REC = 24;
 // tet residual: 12 doubles.
 constexpr int TET_RHS_REC = 12;
-// CZ tangent: per Gauss point the symmetric 3x3 Q = (w a_J) R^T T_d R as xx,xy,xz,yy,yz,zz.
-constexpr int CZ_TAN_REC = 18;
-// CZ residual: 18 doubles.
-constexpr int CZ_RHS_REC = 18;
+// CZ tangent: per pair (ia, ib), ia <= ib, of midplane nodes the symmetric 3x3 block
+// sum_gp s_ia s_ib Q_gp, Q = (w a_J) R^T T_d R, as xx,xy,xz,yy,yz,zz.
+constexpr int CZ_PAIRS = 6, CZ_TAN_REC = 6 * CZ_PAIRS;
+// CZ residual: the three top nodes' parts; the bottom nodes' are their negatives.
+constexpr int CZ_RHS_REC = 9;
 // contact: 78 packed upper-triangle entries of (k/2) Hess d^2, then 12 forces, 6 pad.
 // impact records: the 10 upper 3x3 blocks of the 12x12 tangent, block (a, b) a <= b at
 // ct_block(a, b), each whole and row-major (90 values, FP32 in mixed mode), and the 12 node
@@ -60,7 +86,11 @@ struct DevConsts {
     double sf[9];           // sf[node*3 + gp]
     double lam, mu;         // isotropic split of E (valid when iso != 0)
     double m4[16];          // M[(3i)*12 + 3j]: the mass block (i,j) is m4[4i+j] I3 when iso != 0
+    double m_ii, m_ij;      // its two values, where it has only two: on and off the diagonal
+    float m_iif, m_ijf;
+    int m_two;              // whether it has
     int iso;
+    int alpha_n, beta_n;    // alpha, beta where they are integers from 2 to 16, else 0
     // constant factors of the PPR expressions, formed on the host with the same operations
     // and order as in PPR_math.h / cz_kernels.h, so they are the same doubles
     double k_tn, k_tt;              // gam_n / deln, gam_t / delt
@@ -75,6 +105,10 @@ struct DevConsts {
     float lamf, muf;
     float m4f[16];
 };
+
+// 16 bytes at an 8-byte aligned place
+typedef float f32x4 __attribute__((ext_vector_type(4), aligned(8), may_alias));
+typedef double f64x2 __attribute__((ext_vector_type(2), aligned(8), may_alias));
 
 // ---- small vector helpers --------------------------------------------------------------------
 template <typename T>

@@ -299,57 +299,42 @@ __global__ __launch_bounds__(256) void k_tet_phase1(const int *__restrict__ ie, 
 // V (lam g~_i g~_j^T + mu g~_j g~_i^T + mu (g~_i . g~_j) I), and the mass block is m_ij I
 // (the supported form of M).
 template <typename T>
-struct TetIsoLoad;
+struct TetIso;
 
 template <>
-struct TetIsoLoad<float> {
+struct TetIso<float> {
     float4 gi, gj;   // (g~, V)
     int ij;
-    __device__ inline void load(const float *__restrict__ base, int tp, uint32_t code)
-    {
-        const uint32_t q = code_q(code);
-        const float4 *rec = (const float4 *)base + code_unit(code);
-        ij = (int)q;
-        gi = rec[(size_t)(q >> 2) * tp];
-        gj = rec[(size_t)(q & 3) * tp];
-    }
     __device__ inline void values(float w[9], float stiff, float mcoef) const
     {
         const float V = gi.w, c1 = stiff * V, cl = c1 * g_c.lamf, cu = c1 * g_c.muf;
-        const float dg = gi.x * gj.x + gi.y * gj.y + gi.z * gj.z;
-        const float dd = cu * dg + mcoef * V * g_c.m4f[ij];
+        // a table read by lane would wait for every load in flight; the consistent mass has two values
+        const float m = g_c.m_two ? ((ij >> 2) == (ij & 3) ? g_c.m_iif : g_c.m_ijf) : g_c.m4f[ij];
+        // products and sums fused as written, so that a block's FP32 value is the same in every kernel
+        const float dg = fmaf(gi.z, gj.z, fmaf(gi.x, gj.x, gi.y * gj.y));
+        const float dd = fmaf(mcoef * V, m, cu * dg);
         const float a[3] = {gi.x, gi.y, gi.z}, b[3] = {gj.x, gj.y, gj.z};
 #pragma unroll
         for (int k = 0; k < 3; k++)
 #pragma unroll
             for (int l = 0; l < 3; l++) {
-                float v = cl * a[k] * b[l] + cu * b[k] * a[l];
-                if (k == l) v += dd;
-                w[3 * k + l] = v;
+                const float v = fmaf(cl * a[k], b[l], cu * b[k] * a[l]);
+                w[3 * k + l] = k == l ? v + dd : v;
             }
     }
 };
 
 template <>
-struct TetIsoLoad<double> {
+struct TetIso<double> {
     double2 i0, i1, j0, j1;   // (g~x, g~y), (g~z, V)
     int ij;
-    __device__ inline void load(const double *__restrict__ base, int tp, uint32_t code)
-    {
-        const uint32_t q = code_q(code);
-        const double2 *rec = (const double2 *)base + (size_t)code_unit(code) * 2;
-        ij = (int)q;
-        i0 = rec[(size_t)(q >> 2) * tp * 2];
-        i1 = rec[(size_t)(q >> 2) * tp * 2 + 1];
-        j0 = rec[(size_t)(q & 3) * tp * 2];
-        j1 = rec[(size_t)(q & 3) * tp * 2 + 1];
-    }
     __device__ inline void values(double w[9], double stiff, double mcoef) const
     {
         const double V = i1.y, c1 = stiff * V, cl = c1 * g_c.lam, cu = c1 * g_c.mu;
         const double a[3] = {i0.x, i0.y, i1.x}, b[3] = {j0.x, j0.y, j1.x};
         const double dg = a[0] * b[0] + a[1] * b[1] + a[2] * b[2];
-        const double dd = cu * dg + mcoef * V * g_c.m4[ij];
+        const double m = g_c.m_two ? ((ij >> 2) == (ij & 3) ? g_c.m_ii : g_c.m_ij) : g_c.m4[ij];
+        const double dd = cu * dg + mcoef * V * m;
 #pragma unroll
         for (int k = 0; k < 3; k++)
 #pragma unroll

@@ -78,11 +78,12 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_fused(int nbf, const int *_
                                                            double *__restrict__ F, int ns, Stage sv,
                                                            double *__restrict__ tsum, int ilv)
 {
+    __shared__ __align__(16) char lds[vals_lds<L, KEYS, STAGE>()];
     int local;
     if (!split2(blockIdx.x, nbf, nchunks, ilv != 0, local))
         reduce_vec3<true, true>(local, nbf, foff, fcodes, fkeys, nfkeys, F, ns, 1, sv, tsum);
     else if (local < nchunks)
-        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, nlist, A, sv);
+        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, nlist, A, sv, lds);
 }
 
 // The CZ counters (workgroups [0, nbc); per specimen when cz_off is given: the CZs of specimen s
@@ -99,6 +100,8 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_rhs_fused(int nbf, int nbc,
         const int *__restrict__ damaged, const int *__restrict__ failed, int nc, int *__restrict__ counts,
         const int *__restrict__ cz_off, int nspec, int *__restrict__ spec_counts, Stage sv, int ilv)
 {
+    constexpr int BYTES = vals_lds<L, KEYS, STAGE>();
+    __shared__ __align__(16) char lds[BYTES];
     const int w = blockIdx.x;
     int local;
     if (w < nbc) {
@@ -106,9 +109,10 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_rhs_fused(int nbf, int nbc,
         else count_flags_n<KEYS>(w, nbc, damaged, failed, nc, counts);
     }
     else if (!split2(w - nbc, nbf, nchunks, ilv != 0, local))
-        reduce_force_rhs(local, nbf, foff, fcodes, fkeys, nfkeys, F, ns, node_row, roff, rcodes, cz_begin, b, sv);
+        reduce_force_rhs<KEYS, vals_stage<L, KEYS, STAGE>()>(local, nbf, foff, fcodes, fkeys, nfkeys, F, ns, node_row, roff, rcodes, cz_begin,
+                                      b, sv, lds);
     else if (local < nchunks)
-        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, nlist, A, sv);
+        reduce_vals<MIXED, ISO, false, L, KEYS, STAGE>(local, nchunks, off, codes, nullptr, nlist, A, sv, lds);
 }
 
 // rhs rows from the tet sums plus their CZ terms (workgroups [0, nbr)), then the CZ counters.
@@ -143,11 +147,12 @@ __global__ __launch_bounds__(KEYS) void k_contact_sums(int nb0, int nb1, const i
                                                        const int *__restrict__ rkeys, int nrkeys,
                                                        double *__restrict__ b, Stage sv)
 {
+    __shared__ __align__(16) char lds[vals_lds<L, KEYS, STAGE>()];
     const int w = blockIdx.x;
     if (w < nb0)
         reduce_vec3<true, false>(w, nb0, foff, fcodes, fkeys, nfkeys, F, ns, 1, sv, nullptr);
     else if (w < nb0 + nb1)
-        reduce_vals<MIXED, false, true, L, KEYS, STAGE>(w - nb0, nb1, voff, vcodes, vkeys, nlist, A, sv);
+        reduce_vals<MIXED, false, true, L, KEYS, STAGE>(w - nb0, nb1, voff, vcodes, vkeys, nlist, A, sv, lds);
     else
         reduce_vec3<true, false>(w - nb0 - nb1, gridDim.x - nb0 - nb1, roff, rcodes, rkeys, nrkeys, b, 1, 3, sv,
                                  nullptr);

@@ -191,6 +191,11 @@ constexpr int shape_value(int role, int c)
 }
 constexpr int shape_ncand(int role) { return role == ICF_SHAPE_ORDER ? 2 : 3; }
 constexpr int SHAPE_DEFAULT[NSHAPE] = {2, 2, 1, 2, 1};   // 256, 256, 8 lanes, 256, interleaved
+// What untuned launches use: the same, but node forces first.  Interleaved with the values they
+// gained 40 us on 256 specimens while both waited on memory; since they do not, the order costs up
+// to 9 us of 30 on 146,000 tets and nothing is left to hide (256 specimens: 621 first, 626
+// interleaved).
+constexpr int SHAPE_UNTUNED[NSHAPE] = {2, 2, 1, 2, 0};
 
 struct icf_ctx {
     int id = 0;
@@ -220,7 +225,8 @@ struct icf_ctx {
     unsigned *rep_host = nullptr, *rep_dev = nullptr, rep_seq = 0;
     int precision = ICF_FP64;
     DevConsts hc;
-    DevBuf tet_rhs, tet_tan, cz_rhs, cz_tan, ct, scan_tmp;
+    DevBuf tet_rhs, tan, cz_rhs, ct, scan_tmp;
+    uint32_t cz_word = 0;            // first 8-byte word of the CZs' records in `tan`
     DevBuf pat_a, pat_b;           // pattern build / broad phase / NL2set: 64-bit keys
     // the pattern's static part (elements and CZs): their distinct sorted keys, kept with a copy
     // of the node-id fields and altIds they came from; reused while that copy still matches
@@ -261,7 +267,9 @@ struct icf_ctx {
     // Per role: the candidate in use and, while tuning, the timings
     struct Tune {
         int ncand = NCAND;
-        int sel = CAND_DEFAULT_FP32;   // candidate in use
+        int sel = CAND_FP32;       // candidate in use
+        bool tuned = false;        // a tuning has chosen it
+        int untuned = CAND_UNTUNED;    // what launches use when it is neither tuned nor set
         bool active = false;       // timing the candidates in turn
         bool fixed = false;        // chosen by the caller (icf_set_chunk_keys / icf_set_shape)
         int turn = 0;              // launches started while tuning
@@ -585,6 +593,7 @@ int build_maps(icf_ctx *ctx, const std::vector<SlotMap *> &todo, SlotMap *mr, co
         }
         add_srcs(J, j, *m);
         J.nkeys[j] = m->nkeys;
+        J.vals[j] = m->target == TGT_VALS;
         J.cnt0[j] = keys;
         J.tile0[j + 1] = J.tile0[j] + blocks_for(m->nkeys, SCAN_TILE);
         J.sort0[j + 1] = J.sort0[j] + blocks_for(m->nkeys, 256);
@@ -908,7 +917,6 @@ template <typename F> struct OnLane {
     ~OnLane() { ctx->cur = ctx->stream; }
 };
 
-// reserve > n: only grow the staging buffers for `reserve` units
 // Plane stride of the tet staging records for n tets.
 int tet_plane(long long n) { return (int)((std::max(n, 1LL) + 63) / 64 * 64); }
 
@@ -922,18 +930,27 @@ bool stream_tet_staging(const icf_ctx *ctx, int n)
     return (size_t)tet_plane(n) * (rec + sizeof(double) * TET_RHS_REC) > STREAM_STAGING_BYTES;
 }
 
-int stage_tets(icf_ctx *ctx, const int *ie, const double *dn, int n, int es, int ns, int reserve = 0)
+// Staging buffers of a call over nt tets and nc CZs; their tangent records share one buffer.
+int reserve_stage(icf_ctx *ctx, int nt, int nc)
+{
+    const size_t val = ctx->precision == ICF_MIXED ? 4 : 8, rec = ctx->hc.iso ? TET_ISO_REC : TET_GEN_REC;
+    const size_t cap = (size_t)tet_plane(nt), tets = val * rec * cap;
+    if (int r = grow(ctx, ctx->tet_rhs, sizeof(double) * TET_RHS_REC * cap)) return r;
+    if (int r = grow(ctx, ctx->cz_rhs, sizeof(double) * CZ_RHS_REC * (size_t)std::max(nc, 1))) return r;
+    if (int r = grow(ctx, ctx->tan, tets + val * CZ_TAN_REC * (size_t)nc)) return r;
+    ctx->cz_word = (uint32_t)(tets / 8);
+    return 0;
+}
+void *cz_records(const icf_ctx *ctx) { return (double *)ctx->tan.p + ctx->cz_word; }
+
+void stage_tets(icf_ctx *ctx, const int *ie, const double *dn, int n, int es, int ns)
 {
     const bool mixed = ctx->precision == ICF_MIXED, iso = ctx->hc.iso != 0;
-    const size_t rec = iso ? TET_ISO_REC : TET_GEN_REC;
-    const size_t cap = (size_t)tet_plane(std::max(n, reserve));
-    if (int r = grow(ctx, ctx->tet_rhs, sizeof(double) * TET_RHS_REC * cap)) return r;
-    if (int r = grow(ctx, ctx->tet_tan, (mixed ? 4 : 8) * rec * cap)) return r;
-    if (n == 0) return 0;
+    if (n == 0) return;
     const int tp = ctx->tplane = tet_plane(n);
     dim3 g(blocks_for(n, 256)), b(256);
     double *sr = (double *)ctx->tet_rhs.p;
-    void *st = ctx->tet_tan.p;
+    void *st = ctx->tan.p;
     const bool so = stream_tet_staging(ctx, n);
 #define ICF_T1(MX, IS, NAME)                                                                                   \
     do {                                                                                                      \
@@ -945,25 +962,20 @@ int stage_tets(icf_ctx *ctx, const int *ie, const double *dn, int n, int es, int
     else if (iso) ICF_T1(false, true, "k_tet_phase1<fp64,iso>");
     else ICF_T1(false, false, "k_tet_phase1<fp64,gen>");
 #undef ICF_T1
-    return 0;
 }
 
-int stage_czs(icf_ctx *ctx, double *dcz, int *icz, const double *dn, int n, int cs, int ns, int reserve = 0)
+void stage_czs(icf_ctx *ctx, double *dcz, int *icz, const double *dn, int n, int cs, int ns)
 {
     const bool mixed = ctx->precision == ICF_MIXED;
-    const size_t cap = (size_t)std::max(std::max(n, reserve), 1);
-    if (int r = grow(ctx, ctx->cz_rhs, sizeof(double) * CZ_RHS_REC * cap)) return r;
-    if (int r = grow(ctx, ctx->cz_tan, (mixed ? 4 : 8) * CZ_TAN_REC * cap)) return r;
-    if (n == 0) return 0;
+    if (n == 0) return;
     const long long waves = (n + CZ_PER_WAVE - 1) / CZ_PER_WAVE;   // three lanes per CZ
     dim3 g(blocks_for(waves * 64, 256)), b(256);
     if (mixed)
         LAUNCH(ctx, "k_cz_phase1<mixed>", (k_cz_phase1<true>), g, b, dcz, icz, dn, n, cs, ns, (double *)ctx->cz_rhs.p,
-               ctx->cz_tan.p);
+               cz_records(ctx));
     else
         LAUNCH(ctx, "k_cz_phase1<fp64>", (k_cz_phase1<false>), g, b, dcz, icz, dn, n, cs, ns, (double *)ctx->cz_rhs.p,
-               ctx->cz_tan.p);
-    return 0;
+               cz_records(ctx));
 }
 
 // ---- autotuner of the launch shapes -----------------------------------------------------------
@@ -1003,6 +1015,7 @@ void tune_fold(icf_ctx *ctx, icf_ctx::Tune &t, int role_id)
     }
     if (t.active && (t.samples >= ctx->tune_rounds * t.ncand || t.turn >= 4 * ctx->tune_rounds * t.ncand)) {
         t.active = false;
+        t.tuned = true;
         for (int c = 0; c < t.ncand; c++)
             if (t.best[c] > 0 && (t.best[t.sel] == 0 || t.best[c] < t.best[t.sel])) t.sel = c;
         if (t.bucket >= 0) {
@@ -1022,6 +1035,7 @@ int tune_begin(icf_ctx *ctx, icf_ctx::Tune &t, int role_id, long long units, boo
             std::lock_guard<std::mutex> lk(g_shape_cache.mu);
             auto it = g_shape_cache.choice.find({ctx->device, role_id, ctx->precision, bucket});
             if (it != g_shape_cache.choice.end()) return it->second;
+            if (!t.tuned) return t.untuned;
         }
         return t.sel;
     }
@@ -1066,7 +1080,7 @@ void phase1_fused(icf_ctx *ctx, const int *ie, const double *dn, int nt, int es,
     const int nbc = nc ? (int)blocks_for((long long)(nc + CZ_PER_WAVE - 1) / CZ_PER_WAVE * 64, B) : 0;
     const dim3 g(std::max(interleave2_grid(nbt, nbc), 1)), b(B);
     double *tr = (double *)ctx->tet_rhs.p, *cr = (double *)ctx->cz_rhs.p;
-    void *tt = ctx->tet_tan.p, *ct = ctx->cz_tan.p;
+    void *tt = ctx->tan.p, *ct = cz_records(ctx);
     const int tp = ctx->tplane = tet_plane(nt);
     const bool so = stream_tet_staging(ctx, nt);
 #define ICF_P1(MX, IS, NAME)                                                                                      \
@@ -1203,10 +1217,10 @@ Stage make_stage(icf_ctx *ctx, double h)
 {
     Stage sv;
     sv.tet_rhs = (const double *)ctx->tet_rhs.p;
-    sv.tet_tan = ctx->tet_tan.p;
+    sv.tan = ctx->tan.p;
+    sv.cz_word = ctx->cz_word;
     sv.tplane = ctx->tplane;
     sv.cz_rhs = (const double *)ctx->cz_rhs.p;
-    sv.cz_tan = ctx->cz_tan.p;
     sv.ct_tan = ctx->ct.p;
     sv.ct_f = (const double *)ctx->ct_f.p;
     const DevConsts &c = ctx->hc;
@@ -1291,10 +1305,11 @@ int icf_create(int device, icf_ctx **out)
     if (e != hipSuccess) return (int)e;
     if (device >= ndev) return ICF_E_INVALID;
     icf_ctx *ctx = new icf_ctx();
-    for (auto &row : ctx->tune) row[1].sel = CAND_DEFAULT_FP64;   // FP64 staging roles
+    for (auto &row : ctx->tune) row[1].sel = CAND_FP64;   // FP64 staging roles
     for (int r = 0; r < NSHAPE; r++) {
         ctx->shape[r].ncand = shape_ncand(r);
         ctx->shape[r].sel = SHAPE_DEFAULT[r];
+        ctx->shape[r].untuned = SHAPE_UNTUNED[r];
     }
     ctx->id = g_next_ctx_id++;
     ctx->device = device;
@@ -1332,7 +1347,7 @@ int icf_destroy(icf_ctx *ctx)
     if (ctx->stream_c) (void)hipStreamSynchronize(ctx->stream_c);
     (void)hipStreamSynchronize(ctx->stream);
     for (SlotMap &m : ctx->maps) free_map(m);
-    DevBuf *bufs[] = {&ctx->tet_rhs, &ctx->tet_tan, &ctx->cz_rhs, &ctx->cz_tan, &ctx->ct,   &ctx->scan_tmp,
+    DevBuf *bufs[] = {&ctx->tet_rhs, &ctx->tan, &ctx->cz_rhs, &ctx->ct,   &ctx->scan_tmp,
                       &ctx->pat_a,   &ctx->pat_b,   &ctx->bp_f,   &ctx->bp_i, &ctx->bp_l, &ctx->bp_c,
                       &ctx->tsum,    &ctx->ct_f,    &ctx->adj.off, &ctx->adj.ids, &ctx->batch.d,
                       &ctx->patc.snap, &ctx->patc.keys, &ctx->bp_g, &ctx->map_cnt, &ctx->map_rank, &ctx->map_sums};
@@ -1423,11 +1438,20 @@ int icf_set_constants(icf_ctx *ctx, const icf_consts *c)
                         iso = c->M[(3 * i + k) * 12 + 3 * j + l] == (k == l ? mij : 0.0);
             }
         d.iso = iso ? 1 : 0;
+        d.m_two = 1;
+        d.m_ii = d.m4[0];
+        d.m_ij = d.m4[1];
+        d.m_iif = d.m4f[0];
+        d.m_ijf = d.m4f[1];
+        for (int k = 0; k < 16; k++) d.m_two = d.m_two && d.m4[k] == (k / 4 == k % 4 ? d.m_ii : d.m_ij);
         d.lam = lam;
         d.mu = mu;
         d.lamf = (float)lam;
         d.muf = (float)mu;
     }
+    auto small_int = [](double v) { return v >= 2 && v <= 16 && v == (double)(int)v ? (int)v : 0; };
+    d.alpha_n = small_int(c->alpha);
+    d.beta_n = small_int(c->beta);
     d.k_tn = c->gam_n / c->deln;
     d.k_tt = c->gam_t / c->delt;
     d.k_dnn = c->gam_n / (c->deln * c->deln);
@@ -1707,6 +1731,7 @@ int icf_set_autotune(icf_ctx *ctx, int rounds)
         icf_ctx::Tune &t = *tr.first;
         if (rounds == 0) {             // stop: fold what was timed, keep the fastest so far
             if (t.active) {
+                t.tuned = true;
                 tune_fold(ctx, t, tr.second);
                 for (int c = 0; c < t.ncand; c++)
                     if (t.best[c] > 0 && (t.best[t.sel] == 0 || t.best[c] < t.best[t.sel])) t.sel = c;
@@ -1830,8 +1855,9 @@ int icf_elem_force(icf_ctx *ctx, const int *ie, double *dn, double h, double *A,
                             {TGT_FORCE, -1, {{KIND_TET, ie, nElems, el_stride, EL_NODES, 4}}}};
     if (int r = get_maps(ctx, req)) return r;
     SlotMap *mv = req[0].map, *mr = req[1].map, *mf = req[2].map;
+    if (int r = reserve_stage(ctx, nElems, 0)) return r;
     Timer tm(ctx);
-    if (int r = stage_tets(ctx, ie, dn, nElems, el_stride, nd_stride)) return r;
+    stage_tets(ctx, ie, dn, nElems, el_stride, nd_stride);
     Stage st = make_stage(ctx, h);
     launch_vec3(ctx, mf, dn + (size_t)nd_stride * ND_F, nd_stride, 1, 1, st);
     launch_vals(ctx, mv, A, 1, st);
@@ -1855,8 +1881,9 @@ int icf_cz_force(icf_ctx *ctx, double *dcz, int *icz, double *dn, double *A, dou
                             {TGT_RHS, -1, {{KIND_CZ, icz, nCZs, cz_stride, CZI_ROWS, 6}}}};
     if (int r = get_maps(ctx, req)) return r;
     SlotMap *mv = req[0].map, *mr = req[1].map;
+    if (int r = reserve_stage(ctx, 0, nCZs)) return r;
     Timer tm(ctx);
-    if (int r = stage_czs(ctx, dcz, icz, dn, nCZs, cz_stride, nd_stride)) return r;
+    stage_czs(ctx, dcz, icz, dn, nCZs, cz_stride, nd_stride);
     Stage st = make_stage(ctx, h);
     launch_vals(ctx, mv, A, 1, st);
     launch_vec3(ctx, mr, b, 1, 3, 1, st);
@@ -2141,8 +2168,7 @@ static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride,
     if (tsum)
         if (int r = grow(ctx, ctx->tsum, sizeof(double) * 3 * (size_t)mf->nkeys)) return r;
     // buffers grow before any work is issued (growing synchronizes the context's stream)
-    if (int r = stage_tets(ctx, ie, dn, 0, el_stride, nd_stride, nElems)) return r;
-    if (int r = stage_czs(ctx, dcz, icz, dn, 0, cz_stride, nd_stride, nCZs)) return r;
+    if (int r = reserve_stage(ctx, nElems, nCZs)) return r;
     Timer tm(ctx);
     int *counts = ctx->small + 2;   // the two counts of GPU_Functionality.cs:474-475
     const int *dmg = icz ? icz + (size_t)cz_stride * CZI_TDAMAGED : nullptr;
@@ -2154,8 +2180,8 @@ static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride,
         phase1_fused(ctx, ie, dn, nElems, el_stride, nd_stride, dcz, icz, nCZs, cz_stride, counts);
     } else {
         LAUNCH(ctx, "k_fill_int", k_fill_int, dim3(1), dim3(64), counts, 2, 0);
-        if (int r = stage_tets(ctx, ie, dn, nElems, el_stride, nd_stride)) return r;
-        if (int r = stage_czs(ctx, dcz, icz, dn, nCZs, cz_stride, nd_stride)) return r;
+        stage_tets(ctx, ie, dn, nElems, el_stride, nd_stride);
+        stage_czs(ctx, dcz, icz, dn, nCZs, cz_stride, nd_stride);
     }
     Stage st = make_stage(ctx, h);
     double *F = dn + (size_t)nd_stride * ND_F;

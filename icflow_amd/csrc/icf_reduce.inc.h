@@ -64,6 +64,7 @@ struct MapJobs {
     long long at[MAX_MAP_SRCS];         // the source's place in `rank`
     int *snap[MAX_MAP_SRCS];            // copy of the source's fields, as they are counted
     int nkeys[MAX_JOBS];
+    bool vals[MAX_JOBS];                // keys are BCSR blocks
     long long cnt0[MAX_JOBS];           // the map's place in `cnt` (nkeys counts)
     unsigned tile0[MAX_JOBS + 1];       // first scan tile of a map
     unsigned sort0[MAX_JOBS + 1];       // first sorting workgroup of a map
@@ -208,7 +209,9 @@ __global__ __launch_bounds__(256) void k_map_fill(MapJobs J, const int *__restri
     const size_t i = (size_t)q * J.src[k].n + u;
     const int key = J.snap[k][i], j = J.job[k];
     if (key < 0 || key >= J.nkeys[j]) return;
-    J.codes[j][J.off[j][key] + rank[J.at[k] + i]] = make_code(J.src[k].kind, (uint32_t)u, (uint32_t)q);
+    const uint32_t kind = J.src[k].kind;
+    const uint32_t local = J.vals[j] && kind == KIND_CZ ? czv_code((uint32_t)q) : (uint32_t)q;
+    J.codes[j][J.off[j][key] + rank[J.at[k] + i]] = make_code(kind, (uint32_t)u, local);
 }
 
 __device__ inline void sort_codes(uint32_t *c, int b, int e)
@@ -272,57 +275,138 @@ constexpr int KEY_CANDS[NKC] = {64, 128, 256, 512};
 constexpr int STAGE_CANDS[NSC] = {2, 3};
 __host__ __device__ constexpr int cand_keys(int c) { return KEY_CANDS[c / NSC]; }
 __host__ __device__ constexpr int cand_stage(int c) { return STAGE_CANDS[c % NSC]; }
-constexpr int CAND_DEFAULT_FP32 = 2 * NSC + 0;           // 256 keys, 2 per key, until tuned
-constexpr int CAND_DEFAULT_FP64 = 2 * NSC + 1;           // 256 keys, 1.5 per key
+constexpr int CAND_FP32 = 2 * NSC + 0, CAND_FP64 = 2 * NSC + 1;   // a context's shape until tuned or set
+// Launches of roles that are neither tuned nor set take 128 keys, 3 FP32 or 1.5 FP64 contributions
+// per key.  Time of the fused value launch, and of the other shapes of 64 to 256 keys (us): 256
+// batched specimens mixed 621 (627-703), 779,000 tets FP64 190 (187-201), 309,000 tets FP64 65
+// (65-75), 146,000 tets mixed 30.0 (28.6-32.8).
+constexpr int CAND_UNTUNED = 1 * NSC + 1;
 template <typename L, int KEYS, int STAGE>
 __host__ __device__ constexpr int flat_cap() { return sizeof(L) == 4 ? STAGE * KEYS : STAGE * KEYS / 2; }
-__host__ __device__ constexpr int flat_cap_of(bool fp32, int keys, int stage)
-{
-    return fp32 ? stage * keys : stage * keys / 2;
-}
+// bytes of LDS of a value reduction: the staged contributions, then the list of long keys
+template <typename L, int KEYS, int STAGE>
+__host__ __device__ constexpr int vals_stage() { return flat_cap<L, KEYS, STAGE>() * 9 * (int)sizeof(L); }
+template <typename L, int KEYS, int STAGE>
+__host__ __device__ constexpr int vals_lds() { return vals_stage<L, KEYS, STAGE>() + 2 * KEYS + 4 * (KEYS / 64); }
 
 // Staged per-unit records of the current call.
 struct Stage {
     const double *tet_rhs;  // node part i of tet u at (i * tplane + u) * 3
-    const void *tet_tan;    // isotropic: node i's (g~, V) of tet u at record i * tplane + u
+    const void *tan;        // tangent records: tets (isotropic: node i's (g~, V) of tet u at record
+                            // i * tplane + u), and from 8-byte word cz_word on the CZs'
+    uint32_t cz_word;
     int tplane;             // tet plane stride (the staged tet count, rounded up to 64)
     const double *cz_rhs;
-    const void *cz_tan;
     const void *ct_tan;     // impact tangent blocks (float in mixed mode)
     const double *ct_f;     // impact forces
     double stiff, mcoef;   // tet LHS coefficients (element_kernels2.h:239-240)
 };
 
-__device__ inline const double *rhs_of(const Stage &sv, uint32_t code)
+// One contribution to a node force or rhs row.
+struct Part {
+    double x, y, z;
+};
+__device__ inline Part part_of(const Stage &sv, uint32_t code)
 {
     const uint32_t kind = code_kind(code), u = code_unit(code), q = code_q(code);
-    if (kind == KIND_TET) return sv.tet_rhs + ((size_t)q * sv.tplane + u) * 3;
-    if (kind == KIND_CZ) return sv.cz_rhs + (size_t)u * CZ_RHS_REC + 3 * q;
-    return sv.ct_f + (size_t)u * CT_F_REC + 3 * q;
+    const double *p;
+    bool neg = false;
+    if (kind == KIND_TET) p = sv.tet_rhs + ((size_t)q * sv.tplane + u) * 3;
+    else if (kind == KIND_CZ) {
+        neg = q >= 3;
+        p = sv.cz_rhs + (size_t)u * CZ_RHS_REC + 3 * (neg ? q - 3 : q);
+    } else p = sv.ct_f + (size_t)u * CT_F_REC + 3 * q;
+    const f64x2 v = *(const f64x2 *)p;
+    const double z = p[2];
+    return neg ? Part{-v.x, -v.y, -z} : Part{v.x, v.y, z};
 }
 
-// One contribution's 3x3 block, as the values that are added into the slot's FP64
-// accumulator (FP32 values in mixed mode for tets and CZs).
-template <bool MIXED, bool ISO, typename L>
+// The values of one isotropic tet or CZ contribution, loaded by the same instructions whichever it
+// is (a wave usually has both).  Places are counted in 8-byte words from the start of the tangent
+// records, tets' then CZs' (Stage::tan): 32 bits hold them for 2^24 units of each, and a place is a
+// few 24-bit products and one select.
+template <typename T>
+struct TanLoad;
+__device__ inline const double *tan_word(const Stage &sv, uint32_t at) { return (const double *)sv.tan + at; }
+// i * tplane + u, node i's place in the planes of tet u (tplane is a multiple of 64 up to 2^24)
+__device__ inline uint32_t tet_at(const Stage &sv, uint32_t i, uint32_t u)
+{
+    return (__umul24(i, (uint32_t)sv.tplane >> 6) << 6) + u;
+}
+template <>
+struct TanLoad<float> {
+    f32x4 a, b;      // tet: (g~_i, V), (g~_j, V); CZ: values 0-3 and 2-5 of the pair's six
+    __device__ inline void load(const Stage &sv, uint32_t code)
+    {
+        const uint32_t u = code_unit(code), cz = sv.cz_word + __umul24(u, CZ_TAN_REC / 2) + 3 * czv_pair(code);
+        const bool tet = code_kind(code) == KIND_TET;
+        a = *(const f32x4 *)tan_word(sv, tet ? 2 * tet_at(sv, code_q(code) >> 2, u) : cz);
+        b = *(const f32x4 *)tan_word(sv, tet ? 2 * tet_at(sv, code_q(code) & 3, u) : cz + 1);
+    }
+    __device__ inline void values(float w[9], uint32_t code, float stiff, float mcoef) const
+    {
+        if (code_kind(code) == KIND_TET) {
+            TetIso<float> t;
+            t.gi = make_float4(a.x, a.y, a.z, a.w);
+            t.gj = make_float4(b.x, b.y, b.z, b.w);
+            t.ij = (int)code_q(code);
+            t.values(w, stiff, mcoef);
+        } else {
+            const float c[6] = {a.x, a.y, a.z, a.w, b.z, b.w};
+            cz_spread(c, czv_neg(code), w);
+        }
+    }
+};
+template <>
+struct TanLoad<double> {
+    f64x2 a, b, c, d;   // tet: (g~_i, V), (g~_j, V); CZ: the pair's six values in a, b, c
+    __device__ inline void load(const Stage &sv, uint32_t code)
+    {
+        const uint32_t u = code_unit(code), cz = sv.cz_word + __umul24(u, CZ_TAN_REC) + 6 * czv_pair(code);
+        const bool tet = code_kind(code) == KIND_TET;
+        const double *p0 = tan_word(sv, tet ? 4 * tet_at(sv, code_q(code) >> 2, u) : cz);
+        const double *p1 = tan_word(sv, tet ? 4 * tet_at(sv, code_q(code) & 3, u) : cz + 2);
+        a = *(const f64x2 *)p0;
+        b = *(const f64x2 *)(p0 + 2);
+        c = *(const f64x2 *)p1;
+        d = *(const f64x2 *)(p1 + 2);
+    }
+    __device__ inline void values(double w[9], uint32_t code, double stiff, double mcoef) const
+    {
+        if (code_kind(code) == KIND_TET) {
+            TetIso<double> t;
+            t.i0 = make_double2(a.x, a.y);
+            t.i1 = make_double2(b.x, b.y);
+            t.j0 = make_double2(c.x, c.y);
+            t.j1 = make_double2(d.x, d.y);
+            t.ij = (int)code_q(code);
+            t.values(w, stiff, mcoef);
+        } else {
+            const double z[6] = {a.x, a.y, b.x, b.y, d.x, d.y};
+            cz_spread(z, czv_neg(code), w);
+        }
+    }
+};
+
+// One contribution's 3x3 block where tets have general records or the units are impacts, as the
+// values that are added into the slot's FP64 accumulator.
+template <bool MIXED, typename L>
 __device__ inline void contrib9(const Stage &sv, uint32_t code, L v[9])
 {
     using T = typename std::conditional<MIXED, float, double>::type;
-    const uint32_t kind = code_kind(code), u = code_unit(code), q = code_q(code);
     const T stiff = (T)sv.stiff, mcoef = (T)sv.mcoef;
-    if (kind == KIND_TET && ISO) {
-        TetIsoLoad<T> l;
-        l.load((const T *)sv.tet_tan, sv.tplane, code);
-        T w[9];
-        l.values(w, stiff, mcoef);
+    const uint32_t kind = code_kind(code), u = code_unit(code), q = code_q(code);
+    if (kind == KIND_CZ) {
+        const T *rec = (const T *)((const double *)sv.tan + sv.cz_word) + (size_t)u * CZ_TAN_REC + 6 * czv_pair(code);
+        T c[6];
 #pragma unroll
-        for (int k = 0; k < 9; k++) v[k] = (L)w[k];
+        for (int k = 0; k < 6; k++) c[k] = rec[k];
+        cz_spread(c, czv_neg(code), v);
         return;
     }
     double acc[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
     if (kind == KIND_TET)
-        tet_block_gen<T>(acc, (const T *)sv.tet_tan + (size_t)u * TET_GEN_REC, q >> 2, q & 3, stiff, mcoef);
-    else if (kind == KIND_CZ)
-        cz_block<T>(acc, (const T *)sv.cz_tan + (size_t)u * CZ_TAN_REC, q / 6, q % 6);
+        tet_block_gen<T>(acc, (const T *)sv.tan + (size_t)u * TET_GEN_REC, q >> 2, q & 3, stiff, mcoef);
     else
         contact_block<T>(acc, (const T *)sv.ct_tan + (size_t)u * CT_TAN_REC, q >> 2, q & 3);
 #pragma unroll
@@ -335,18 +419,30 @@ __device__ inline void contrib9(const Stage &sv, uint32_t code, L v[9])
 // own of the round from LDS in list order into an FP64 accumulator.  The values and their order
 // are those of a sequential loop over the key's list, so the result does not depend on the
 // chunking.
+//   A block on the diagonal has some 16 to 40 contributions, one off it 4 to 6, and each row of
+// about 8 blocks holds one of the former: a wave of one key per lane runs as long as its longest
+// and was idle for three quarters of the sums, half of the kernel's VALU instructions.  Keys with
+// more than VALS_LONG contributions are therefore listed and summed by teams of nine lanes, one
+// component each, which keep their sums across the rounds; the rest by one lane each, in at most
+// VALS_LONG steps.
+//   With isotropic tets the next round's gathers are in flight while one is summed, so nothing in
+// between may wait for loads (the mass factor is selected, not looked up).  Alone, the values of
+// 256 batched specimens (mixed) take 420 us, from 524 without teams, prefetch and word addresses
+// (1.05 GB written and read at least); those of 779,000 tets (FP64) 144 us, from 189.
 //   keys   null: list positions are keys; else keys[position] (accumulate mode)
 //   off    first code per list position
 //   ACC    add to A (single-kernel calls); otherwise overwrite, zero where nothing contributes
 // L is the staging type: float for tet and CZ blocks in mixed mode, double otherwise.
+constexpr int VALS_LONG = 8;
 template <bool MIXED, bool ISO, bool ACC, typename L, int KEYS, int STAGE>
 __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__restrict__ off,
-        const uint32_t *__restrict__ codes, const int *__restrict__ keys, int nlist, double *__restrict__ A, Stage sv)
+        const uint32_t *__restrict__ codes, const int *__restrict__ keys, int nlist, double *__restrict__ A, Stage sv,
+        void *smem)
 {
     constexpr int CAP = flat_cap<L, KEYS, STAGE>();
     static_assert(CAP * 9 * sizeof(L) >= KEYS * 9 * sizeof(double), "output staging fits the LDS");
     constexpr int PER = (CAP + KEYS - 1) / KEYS;
-    __shared__ L lds[CAP * 9];
+    L *lds = (L *)smem;
     const int p0 = xcd_remap(bid_, nb_) * KEYS;
     if (p0 >= nlist) return;
     const int p1 = min(p0 + KEYS, nlist);
@@ -355,52 +451,131 @@ __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__rest
     const int p = p0 + threadIdx.x;
     const bool live = p < p1;
     int s = 0, b = 0, e = 0;
-    double acc[9];
-#pragma unroll
-    for (int i = 0; i < 9; i++) acc[i] = 0.;
     if (live) {
         s = keys ? keys[p] : p;
         b = off[p];
         e = off[p + 1];
-        if (ACC) {   // the block's current values, also loaded before the contributions
-            const double *src = A + (size_t)s * 9;
-#pragma unroll
-            for (int i = 0; i < 9; i++) acc[i] = src[i];
-        }
     }
-    for (int c0 = cb; c0 < ce; c0 += CAP) {
-        const int c1 = min(c0 + CAP, ce);
-        // codes first (coalesced), then the contributions, so their loads overlap
-        uint32_t cd[PER];
+    // the long keys, in order
+    constexpr int WAVES = KEYS / 64, TEAMS = 7 * WAVES, SLOTS = 2;
+    auto *longs = (unsigned short *)((char *)smem + vals_stage<L, KEYS, STAGE>());
+    int *wcnt = (int *)((char *)smem + vals_stage<L, KEYS, STAGE>() + 2 * KEYS);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool lng = live && e - b > VALS_LONG;
+    const unsigned long long lm = __ballot(lng);
+    if (lane == 0) wcnt[wave] = __popcll(lm);
+    __syncthreads();
+    int at_long = __popcll(lm & ((1ULL << lane) - 1)), nlong = 0;
 #pragma unroll
-        for (int r = 0; r < PER; r++) {
-            const int i = c0 + threadIdx.x + r * KEYS;
-            cd[r] = i < c1 ? codes[i] : 0u;
-        }
-        if (c0 != cb) __syncthreads();   // the previous round's values have been added
+    for (int w = 0; w < WAVES; w++) {
+        if (w < wave) at_long += wcnt[w];
+        nlong += wcnt[w];
+    }
+    if (lng) longs[at_long] = (unsigned short)threadIdx.x;
+    const bool mine = live && (!lng || at_long >= TEAMS * SLOTS);   // summed by this thread alone
+    double acc[9];
 #pragma unroll
-        for (int r = 0; r < PER; r++) {
-            const int i = threadIdx.x + r * KEYS;
-            if (c0 + i < c1) {
-                L v[9];
-                contrib9<MIXED, ISO, L>(sv, cd[r], v);
+    for (int i = 0; i < 9; i++) acc[i] = 0.;
+    if (ACC && mine) {   // the block's current values, also loaded before the contributions
+        const double *src = A + (size_t)s * 9;
 #pragma unroll
-                for (int k = 0; k < 9; k++) lds[i * 9 + k] = v[k];
+        for (int i = 0; i < 9; i++) acc[i] = src[i];
+    }
+    __syncthreads();
+    // consecutive long keys go to one wave's teams, whose ranges then fall in the same rounds
+    const int team = lane / 9, comp = lane - 9 * team;
+    int tkey[SLOTS], tb[SLOTS], te[SLOTS];
+    double tacc[SLOTS];
+#pragma unroll
+    for (int q = 0; q < SLOTS; q++) {
+        const int j = (q * WAVES + wave) * 7 + team;
+        const bool on = team < 7 && j < nlong;
+        tkey[q] = on ? (int)longs[j] : -1;
+        tb[q] = on ? off[p0 + tkey[q]] : 0;
+        te[q] = on ? off[p0 + tkey[q] + 1] : 0;
+        tacc[q] = 0.;
+        if (ACC && on) tacc[q] = A[(size_t)keys[p0 + tkey[q]] * 9 + comp];
+    }
+    auto sum = [&](int c0, int c1) {      // the contributions of the round, each key's in order
+        if (mine) {
+            const int hi = min(e, c1) - c0;
+            for (int c = max(b, c0) - c0; c < hi; c++) {
+#pragma unroll
+                for (int k = 0; k < 9; k++) acc[k] += (double)lds[c * 9 + k];
             }
         }
-        __syncthreads();
-        const int hi = min(e, c1) - c0;
-        for (int c = max(b, c0) - c0; c < hi; c++) {
 #pragma unroll
-            for (int k = 0; k < 9; k++) acc[k] += (double)lds[c * 9 + k];
+        for (int q = 0; q < SLOTS; q++) {
+            const int hi = min(te[q], c1) - c0;
+            for (int c = max(tb[q], c0) - c0; c < hi; c++) tacc[q] += (double)lds[c * 9 + comp];
+        }
+    };
+    uint32_t cd[PER];
+    auto fetch = [&](int c0) {            // codes of the round at c0 (coalesced)
+#pragma unroll
+        for (int r = 0; r < PER; r++) {
+            const int i = c0 + (int)threadIdx.x + r * KEYS;
+            cd[r] = i < min(c0 + CAP, ce) ? codes[i] : CODE_NONE;
+        }
+    };
+    if constexpr (ISO) {
+        // the next round's gathers are under way while this one is summed, and the codes of the
+        // one after that
+        using T = typename std::conditional<MIXED, float, double>::type;
+        const T stiff = (T)sv.stiff, mcoef = (T)sv.mcoef;
+        TanLoad<T> ld[PER];
+        uint32_t at[PER];
+        auto gather = [&]() {
+#pragma unroll
+            for (int r = 0; r < PER; r++) {
+                at[r] = cd[r];
+                if (at[r] != CODE_NONE) ld[r].load(sv, at[r]);
+            }
+        };
+        fetch(cb);
+        gather();
+        fetch(cb + CAP);
+        for (int c0 = cb; c0 < ce; c0 += CAP) {
+            if (c0 != cb) __syncthreads();   // the previous round's values have been added
+#pragma unroll
+            for (int r = 0; r < PER; r++) {
+                if (at[r] == CODE_NONE) continue;
+                T w[9];
+                ld[r].values(w, at[r], stiff, mcoef);
+                L *v = lds + ((int)threadIdx.x + r * KEYS) * 9;
+#pragma unroll
+                for (int k = 0; k < 9; k++) v[k] = (L)w[k];
+            }
+            __syncthreads();
+            gather();
+            fetch(c0 + 2 * CAP);
+            sum(c0, min(c0 + CAP, ce));
+        }
+    } else {
+        for (int c0 = cb; c0 < ce; c0 += CAP) {
+            fetch(c0);
+            if (c0 != cb) __syncthreads();   // the previous round's values have been added
+#pragma unroll
+            for (int r = 0; r < PER; r++) {
+                if (cd[r] == CODE_NONE) continue;
+                L v[9];
+                contrib9<MIXED, L>(sv, cd[r], v);
+#pragma unroll
+                for (int k = 0; k < 9; k++) lds[((int)threadIdx.x + r * KEYS) * 9 + k] = v[k];
+            }
+            __syncthreads();
+            sum(c0, min(c0 + CAP, ce));
         }
     }
     if (ACC) {
-        if (live) {
+        if (mine) {
             double *dst = A + (size_t)s * 9;
 #pragma unroll
             for (int i = 0; i < 9; i++) dst[i] = acc[i];
         }
+#pragma unroll
+        for (int q = 0; q < SLOTS; q++)
+            if (tkey[q] >= 0) A[(size_t)keys[p0 + tkey[q]] * 9 + comp] = tacc[q];
         return;
     }
     // overwrite mode: the chunk's blocks A[p0 .. p1) are contiguous; write them through LDS
@@ -409,10 +584,13 @@ __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__rest
     // lines from the staged records the other chunks still gather
     double *out = reinterpret_cast<double *>(lds);
     __syncthreads();
-    if (live) {
+    if (mine) {
 #pragma unroll
         for (int k = 0; k < 9; k++) out[threadIdx.x * 9 + k] = acc[k];
     }
+#pragma unroll
+    for (int q = 0; q < SLOTS; q++)
+        if (tkey[q] >= 0) out[tkey[q] * 9 + comp] = tacc[q];
     __syncthreads();
     const int nout = (p1 - p0) * 9;
     double *dst = A + (size_t)p0 * 9;
@@ -424,7 +602,8 @@ __global__ __launch_bounds__(KEYS) void k_reduce_vals(const int *__restrict__ of
                                                       const int *__restrict__ keys, int nlist, double *__restrict__ A,
                                                       Stage sv)
 {
-    reduce_vals<MIXED, ISO, ACC, L, KEYS, STAGE>(blockIdx.x, gridDim.x, off, codes, keys, nlist, A, sv);
+    __shared__ __align__(16) char lds[vals_lds<L, KEYS, STAGE>()];
+    reduce_vals<MIXED, ISO, ACC, L, KEYS, STAGE>(blockIdx.x, gridDim.x, off, codes, keys, nlist, A, sv, lds);
 }
 
 // Phase 2 for rhs rows (b[row*3+k]) or node forces (dn[node + ns*(F+k)]): one thread per list
@@ -448,29 +627,20 @@ __device__ __forceinline__ void reduce_vec3(int bid_, int nb_, const int *__rest
     } else {
         a0 = a1 = a2 = 0.;
     }
-    auto part = [&](int c) { return rhs_of(sv, codes[c]); };
+    auto add = [&](const Part &v) {
+        a0 += v.x; a1 += v.y; a2 += v.z;
+        if (TSUM) { t0 += v.x; t1 += v.y; t2 += v.z; }
+    };
     int c = b;
     for (; c + 4 <= e; c += 4) {          // loads of four contributions in flight, added in order
-        const double *r0 = part(c), *r1 = part(c + 1);
-        const double *r2 = part(c + 2), *r3 = part(c + 3);
-        const double x0 = r0[0], y0 = r0[1], z0 = r0[2], x1 = r1[0], y1 = r1[1], z1 = r1[2];
-        const double x2 = r2[0], y2 = r2[1], z2 = r2[2], x3 = r3[0], y3 = r3[1], z3 = r3[2];
-        a0 += x0; a1 += y0; a2 += z0;
-        a0 += x1; a1 += y1; a2 += z1;
-        a0 += x2; a1 += y2; a2 += z2;
-        a0 += x3; a1 += y3; a2 += z3;
-        if (TSUM) {
-            t0 += x0; t1 += y0; t2 += z0;
-            t0 += x1; t1 += y1; t2 += z1;
-            t0 += x2; t1 += y2; t2 += z2;
-            t0 += x3; t1 += y3; t2 += z3;
-        }
+        const Part p0 = part_of(sv, codes[c]), p1 = part_of(sv, codes[c + 1]);
+        const Part p2 = part_of(sv, codes[c + 2]), p3 = part_of(sv, codes[c + 3]);
+        add(p0);
+        add(p1);
+        add(p2);
+        add(p3);
     }
-    for (; c < e; c++) {
-        const double *r = part(c);
-        a0 += r[0]; a1 += r[1]; a2 += r[2];
-        if (TSUM) { t0 += r[0]; t1 += r[1]; t2 += r[2]; }
-    }
+    for (; c < e; c++) add(part_of(sv, codes[c]));
     dst[0] = a0; dst[comp_stride] = a1; dst[2 * comp_stride] = a2;
     if (TSUM) {
         double *o = tsum + (size_t)s * 3;
@@ -484,45 +654,69 @@ __device__ __forceinline__ void reduce_vec3(int bid_, int nb_, const int *__rest
 // followed by the row's CZ contributions in list order (as reduce_rhs_tsum from that tet sum).
 // Used when every rhs row's tet contributions are its node's force list and every row has such
 // a node (the host checks both once per pair of maps).
+// The contributions of the workgroup's nodes are one run of codes; they come through LDS in rounds
+// of BYTES / 24, like those of reduce_vals: codes read as they lie, three or more gathers in
+// flight per lane, neighbouring lanes in neighbouring tets.  A lane walking its own node's list
+// fetched every line for 24 of its bytes: alone on 256 batched specimens 242 us and 67 for the rows,
+// 205 for both this way.
+template <int KEYS, int BYTES>
 __device__ __forceinline__ void reduce_force_rhs(int bid_, int nb_, const int *__restrict__ foff,
         const uint32_t *__restrict__ fcodes, const int *__restrict__ fkeys, int nfkeys, double *__restrict__ F,
         int ns, const int *__restrict__ node_row, const int *__restrict__ roff, const uint32_t *__restrict__ rcodes,
-        const int *__restrict__ cz_begin, double *__restrict__ rhs, Stage sv)
+        const int *__restrict__ cz_begin, double *__restrict__ rhs, Stage sv, void *smem)
 {
-    const int t = xcd_remap(bid_, nb_) * blockDim.x + threadIdx.x;
-    if (t >= nfkeys) return;
-    const int s = fkeys ? fkeys[t] : t;
-    const int b = foff[t], e = foff[t + 1];
-    const int r = node_row[s];
-    double *dst = F + s;
-    double a0 = dst[0], a1 = dst[ns], a2 = dst[2 * (size_t)ns], t0 = 0., t1 = 0., t2 = 0.;
-    auto part = [&](int c) { return rhs_of(sv, fcodes[c]); };
-    int c = b;
-    for (; c + 4 <= e; c += 4) {          // loads of four contributions in flight, added in order
-        const double *r0 = part(c), *r1 = part(c + 1);
-        const double *r2 = part(c + 2), *r3 = part(c + 3);
-        const double x0 = r0[0], y0 = r0[1], z0 = r0[2], x1 = r1[0], y1 = r1[1], z1 = r1[2];
-        const double x2 = r2[0], y2 = r2[1], z2 = r2[2], x3 = r3[0], y3 = r3[1], z3 = r3[2];
-        a0 += x0; a1 += y0; a2 += z0;
-        a0 += x1; a1 += y1; a2 += z1;
-        a0 += x2; a1 += y2; a2 += z2;
-        a0 += x3; a1 += y3; a2 += z3;
-        t0 += x0; t1 += y0; t2 += z0;
-        t0 += x1; t1 += y1; t2 += z1;
-        t0 += x2; t1 += y2; t2 += z2;
-        t0 += x3; t1 += y3; t2 += z3;
+    constexpr int PER = BYTES / 24 / KEYS, CAP = PER * KEYS;
+    static_assert(PER >= 1, "a contribution per lane");
+    double *lds = (double *)smem;
+    const int p0 = xcd_remap(bid_, nb_) * KEYS;
+    if (p0 >= nfkeys) return;
+    const int p1 = min(p0 + KEYS, nfkeys), cb = foff[p0], ce = foff[p1];
+    const int t = p0 + (int)threadIdx.x;
+    const bool live = t < p1;
+    int s = 0, b = 0, e = 0, r = -1;
+    double a0 = 0., a1 = 0., a2 = 0., t0 = 0., t1 = 0., t2 = 0.;
+    double *dst = F;
+    if (live) {
+        s = fkeys ? fkeys[t] : t;
+        b = foff[t];
+        e = foff[t + 1];
+        r = node_row[s];
+        dst = F + s;
+        a0 = dst[0]; a1 = dst[ns]; a2 = dst[2 * (size_t)ns];
     }
-    for (; c < e; c++) {
-        const double *q = part(c);
-        a0 += q[0]; a1 += q[1]; a2 += q[2];
-        t0 += q[0]; t1 += q[1]; t2 += q[2];
+    for (int c0 = cb; c0 < ce; c0 += CAP) {
+        const int c1 = min(c0 + CAP, ce);
+        Part v[PER];
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int i = c0 + (int)threadIdx.x + k * KEYS;
+            if (i < c1) v[k] = part_of(sv, fcodes[i]);
+        }
+        if (c0 != cb) __syncthreads();   // the previous round's parts have been added
+#pragma unroll
+        for (int k = 0; k < PER; k++) {
+            const int i = (int)threadIdx.x + k * KEYS;
+            if (c0 + i < c1) {
+                lds[3 * i] = v[k].x;
+                lds[3 * i + 1] = v[k].y;
+                lds[3 * i + 2] = v[k].z;
+            }
+        }
+        __syncthreads();
+        const int hi = min(e, c1) - c0;
+        for (int c = max(b, c0) - c0; c < hi; c++) {
+            const double x = lds[3 * c], y = lds[3 * c + 1], z = lds[3 * c + 2];
+            a0 += x; a1 += y; a2 += z;
+            t0 += x; t1 += y; t2 += z;
+        }
     }
+    if (!live) return;
     dst[0] = a0; dst[ns] = a1; dst[2 * (size_t)ns] = a2;
     if (r < 0) return;
     const int re = roff[r + 1];
     for (int k = cz_begin[r]; k < re; k++) {
-        const double *q = rhs_of(sv, rcodes[k]);
-        t0 += q[0]; t1 += q[1]; t2 += q[2];
+        const Part q = part_of(sv, rcodes[k]);
+        t0 += q.x; t1 += q.y; t2 += q.z;
     }
     double *o = rhs + (size_t)r * 3;
     o[0] = t0; o[1] = t1; o[2] = t2;
@@ -589,8 +783,8 @@ __device__ __forceinline__ void reduce_rhs_tsum(int bid_, int nb_, const int *__
     }
     const int e = off[r + 1];
     for (int c = cz_begin[r]; c < e; c++) {
-        const double *p = rhs_of(sv, codes[c]);
-        a0 += p[0]; a1 += p[1]; a2 += p[2];
+        const Part p = part_of(sv, codes[c]);
+        a0 += p.x; a1 += p.y; a2 += p.z;
     }
     double *o = out + (size_t)r * 3;
     o[0] = a0; o[1] = a1; o[2] = a2;

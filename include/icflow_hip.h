@@ -236,7 +236,8 @@ int icf_set_overlap(icf_ctx *ctx, int on);
  * shape is a key limit (the workgroup size: 64, 128, 256 or 512) and a staging size (stage =
  * 2 or 3 FP32 contributions per key, half as many FP64 ones); the ICF_CHUNK_CANDIDATES = 8
  * shapes are numbered c = 2 * (index of the key limit) + (stage - 2).  Until tuned: 256 keys,
- * stage 2 for FP32 staging, 3 for FP64.  There are four roles, r = 2 * accumulate + fp64:
+ * stage 2 for FP32 staging, 3 for FP64 (what icf_get_autotune reports; launches of a role that was
+ * never tuned or set may use another shape that the library finds better for their size).  There are four roles, r = 2 * accumulate + fp64:
  * overwrite maps (icf_assemble_elems_and_czs) and accumulate maps (icf_collision_response and
  * the single-kernel calls), each with FP32 (mixed) or FP64 staging.
  * icf_set_autotune(ctx, rounds > 0) starts tuning every role: its next launches take the
@@ -266,7 +267,7 @@ int icf_set_chunk_keys(icf_ctx *ctx, int accumulate, int fp64, int keys, int sta
  *                      values; 1 interleaved in rounds of eight workgroups (0, 1)
  * Every candidate gives the same results bit for bit.  icf_set_shape fixes a role's value on
  * this context (ICF_E_INVALID for other values); icf_get_shape reports the context's value
- * (the default until tuned or set), whether the role is still being tuned and the fastest
+ * (the default until tuned or set; a launch of such a role may use another), whether the role is still being tuned and the fastest
  * timing per candidate (best_ms[3], 0: not timed or no such candidate).  Finished tunings, of these roles and of the
  * value reductions, are kept by the library per device, role, precision and size class (units
  * of the launch to the next power of two); a context's launches of a role that it is neither
