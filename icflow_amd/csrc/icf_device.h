@@ -118,20 +118,93 @@ __device__ inline T dot3(const T *a, const T *b) { return a[0] * b[0] + a[1] * b
 // call makes anyway, so that no copy and no clearing launch is needed.  A word is set when it holds
 // the call's sequence number; the device copy of the words keeps all but the first few threads
 // that set one off the bus.
-constexpr int REPORT_WORDS = 16;
+constexpr int REPORT_WORDS = 32;
 struct Report {
     unsigned *dev, *host;
     unsigned seq;
     __device__ inline void set(int k) const
     {
-        if (__hip_atomic_load(dev + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == seq) return;
+        if (was(k)) return;
         __hip_atomic_store(dev + k, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(host + k, seq, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    // whether an earlier launch of the call set word k
+    __device__ inline bool was(int k) const
+    {
+        return __hip_atomic_load(dev + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == seq;
     }
     // a value, from one thread
     __device__ inline void put(int k, unsigned v) const
     {
         __hip_atomic_store(host + k, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+};
+
+// Sum over the 256 threads of the workgroup, in every thread.
+__device__ inline unsigned sum256(unsigned x, unsigned *part)
+{
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = x;
+    __syncthreads();
+    const unsigned t = part[0] + part[1] + part[2] + part[3];
+    __syncthreads();
+    return t;
+}
+
+// Exclusive scan over the 256 threads of the workgroup; total in every thread.
+template <typename T>
+__device__ inline T scan256(T v, T *part, T &total)
+{
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    T x = v;
+    for (int o = 1; o < 64; o <<= 1) {
+        const T y = __shfl_up(x, o);
+        if (lane >= o) x += y;
+    }
+    if (lane == 63) part[wave] = x;
+    __syncthreads();
+    T before = 0;
+    total = 0;
+    for (int w = 0; w < 4; w++) {
+        if (w < wave) before += part[w];
+        total += part[w];
+    }
+    __syncthreads();
+    return before + x - v;
+}
+
+// Where each workgroup's part of an ordered list starts, without a scan launch in between: a launch
+// leaves one count per workgroup and per GROUP workgroups (`groups`, zero before it), and in the
+// next one every workgroup adds up what lies before its own.  A library scan is two or three
+// launches of 4 to 7 us each for lists of any size that occurs here.
+struct Tiles {
+    static constexpr unsigned GROUP = 256;
+    unsigned *sums, *groups;
+    __host__ __device__ static unsigned ngroups(unsigned n) { return (n + GROUP - 1) / GROUP; }
+    // from one thread of workgroup w
+    __device__ inline void put(unsigned w, unsigned v) const
+    {
+        sums[w] = v;
+        if (v) atomicAdd(groups + w / GROUP, v);
+    }
+    // all 256 threads: the sum of the workgroups before w; of all n
+    __device__ inline unsigned before(unsigned w, unsigned *part) const
+    {
+        const unsigned g = w / GROUP, t = g * GROUP + threadIdx.x;
+        unsigned x = t < w ? sums[t] : 0u;
+        for (unsigned i = threadIdx.x; i < g; i += 256) x += groups[i];
+        return sum256(x, part);
+    }
+    __device__ inline unsigned total(unsigned n, unsigned *part) const
+    {
+        unsigned x = 0;
+        for (unsigned i = threadIdx.x; i < ngroups(n); i += 256) x += groups[i];
+        return sum256(x, part);
+    }
+    // all threads of one workgroup, in a launch before
+    __device__ inline void clear(unsigned n) const
+    {
+        for (unsigned i = threadIdx.x; i < ngroups(n); i += blockDim.x) groups[i] = 0u;
     }
 };
 

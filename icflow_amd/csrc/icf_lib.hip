@@ -228,12 +228,13 @@ struct icf_ctx {
     DevBuf tet_rhs, tan, cz_rhs, ct, scan_tmp;
     uint32_t cz_word = 0;            // first 8-byte word of the CZs' records in `tan`
     DevBuf pat_a, pat_b;           // pattern build / broad phase / NL2set: 64-bit keys
-    // the pattern's static part (elements and CZs): their distinct sorted keys, kept with a copy
-    // of the node-id fields and altIds they came from; reused while that copy still matches
+    DevBuf pat_cnt;                // pattern build: the impacts' pairs per row (zero in between)
+    // the pattern's static part (elements and CZs): its rows, kept with a copy of the node-id fields
+    // and altIds they came from; reused while that copy still matches
     struct PatCache {
         bool valid = false;
-        int nNodes = 0, nElems = 0, el_stride = 0, nCZs = 0, cz_stride = 0, N = 0, cb = 0, nkeys = 0;
-        DevBuf snap, keys;
+        int nNodes = 0, nElems = 0, el_stride = 0, nCZs = 0, cz_stride = 0, N = 0;
+        DevBuf snap, rows, cols;
     } patc;
     DevBuf bp_f, bp_i, bp_l;         // broad phase and NL2set scratch (doubles, ints, int64)
     DevBuf bp_c;                     // broad phase grid (cell counts, first sorted position per cell key)
@@ -1350,7 +1351,7 @@ int icf_destroy(icf_ctx *ctx)
     DevBuf *bufs[] = {&ctx->tet_rhs, &ctx->tan, &ctx->cz_rhs, &ctx->ct,   &ctx->scan_tmp,
                       &ctx->pat_a,   &ctx->pat_b,   &ctx->bp_f,   &ctx->bp_i, &ctx->bp_l, &ctx->bp_c,
                       &ctx->tsum,    &ctx->ct_f,    &ctx->adj.off, &ctx->adj.ids, &ctx->batch.d,
-                      &ctx->patc.snap, &ctx->patc.keys, &ctx->bp_g, &ctx->map_cnt, &ctx->map_rank, &ctx->map_sums};
+                      &ctx->patc.snap, &ctx->patc.rows, &ctx->patc.cols, &ctx->pat_cnt, &ctx->bp_g, &ctx->map_cnt, &ctx->map_rank, &ctx->map_sums};
     for (DevBuf *b : bufs)
         if (b->p) (void)hipFree(b->p);
     if (ctx->small) (void)hipFree(ctx->small);
@@ -2406,123 +2407,99 @@ int icf_build_pattern(icf_ctx *ctx, const int *altId, int nNodes, const int *ie,
         return fail(ctx, ICF_E_INVALID, "icf_build_pattern: invalid argument");
     if (ctx->capturing) return fail(ctx, ICF_E_CAPTURE, "icf_build_pattern returns a host value");
     *nnz = 0;
-    // the static part (elements, CZs) and the impacts; the static part's distinct keys are kept
-    // and reused while its node ids and the altIds are unchanged, so that a call with only new
-    // impacts sorts the impact keys and merges them in
-    PatSrc src[3] = {{ie, nElems, el_stride, EL_NODES, 4, 0, 0},
-                     {icz, nCZs, cz_stride, CZI_VRTS, 6, 0, (long long)nElems * pat_pairs(4, 0)},
-                     {icr, nImpacts, cr_stride, CR_NODES, 4, 1, 0}};
+    const PatSrc el{ie, nElems, el_stride, EL_NODES, 4, 0}, cz{icz, nCZs, cz_stride, CZI_VRTS, 6, 0},
+        im{icr, nImpacts, cr_stride, CR_NODES, 4, 1};
     const long long Ms = (long long)nElems * pat_pairs(4, 0) + (long long)nCZs * pat_pairs(6, 0);
     const long long Mi = (long long)nImpacts * pat_pairs(4, 1);
     if (Ms + Mi >= (1LL << 31) - 1)
         return fail(ctx, ICF_E_CAPACITY, "icf_build_pattern: 2^31 or more candidate pairs");
-    int *d_err = ctx->small + 1, *d_diff = ctx->small + 2;
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, d_err, 2, 0);
     int cb = 1;
     while ((1LL << cb) <= (long long)N) cb++;
     const PatFields pf{altId, nNodes, ie, nElems, el_stride, icz, nCZs, cz_stride};
     const long long nsnap = (long long)nNodes + 4LL * nElems + 6LL * nCZs;
     auto &pc = ctx->patc;
-    bool hit = pc.valid && pc.nNodes == nNodes && pc.nElems == nElems && pc.el_stride == el_stride &&
-               pc.nCZs == nCZs && pc.cz_stride == cz_stride && pc.N == N && pc.cb == cb;
-    if (hit && nsnap > 0) {
-        hipLaunchKernelGGL(k_pat_snap, dim3(blocks_for(nsnap, 256)), dim3(256), 0, ctx->stream, pf, nsnap,
-                           (int *)pc.snap.p, 1, d_diff);
-        int diff = 0;
-        HIPCHK(ctx, hipGetLastError());
-        HIPCHK(ctx, hipMemcpyAsync(&diff, d_diff, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        hit = diff == 0;
+    const bool kept = pc.valid && pc.nNodes == nNodes && pc.nElems == nElems && pc.el_stride == el_stride &&
+                      pc.nCZs == nCZs && pc.cz_stride == cz_stride && pc.N == N;
+    // scratch: keys and their distinct ones, or the impacts' pairs; counts per tile of keys or rows
+    const unsigned ktiles = blocks_for(Ms, PAT_TILE), rtiles = blocks_for(N, 256), tiles = std::max(ktiles, rtiles);
+    const size_t nr = (size_t)N, mi = (size_t)Mi, nt = (size_t)tiles + Tiles::ngroups(tiles);
+    const size_t keys = kept ? 0 : (size_t)Ms;
+    if (int r = grow(ctx, ctx->pat_a, std::max(sizeof(unsigned long long) * keys, sizeof(int2) * mi) + 1)) return r;
+    if (int r = grow(ctx, ctx->pat_b, std::max(sizeof(unsigned long long) * keys, sizeof(int) * 3 * mi) + 1)) return r;
+    if (int r = grow(ctx, ctx->bp_l, sizeof(int) * (2 * nr + nt + 2))) return r;
+    if (ctx->pat_cnt.bytes < sizeof(int) * nr) {
+        if (int r = grow(ctx, ctx->pat_cnt, sizeof(int) * nr)) return r;
+        HIPCHK(ctx, hipMemsetAsync(ctx->pat_cnt.p, 0, ctx->pat_cnt.bytes, ctx->stream));
     }
-    // sorted keys -> their distinct blocks, in order (flag, scan, compact); returns the count
-    auto distinct = [&](const unsigned long long *keys, long long M, unsigned long long *out, int *count) -> int {
-        if (int r = grow(ctx, ctx->bp_l, sizeof(int) * 2 * ((size_t)M + 1))) return r;
-        int *flag = (int *)ctx->bp_l.p, *pos = flag + M + 1;
-        size_t ub = 0;
-        HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, ub, flag, pos, (int)M + 1, ctx->stream));
-        if (int r = grow(ctx, ctx->scan_tmp, ub)) return r;
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, flag + M, 1, 0);
-        hipLaunchKernelGGL(k_pat_flag, dim3(blocks_for(M, 256)), dim3(256), 0, ctx->stream, keys, (int)M, cb, flag);
-        HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, ub, flag, pos, (int)M + 1, ctx->stream));
-        hipLaunchKernelGGL(k_pat_compact, dim3(blocks_for(M, 256)), dim3(256), 0, ctx->stream, keys, (int)M, flag,
-                           pos, out);
+    int *w = (int *)ctx->bp_l.p + 2 * nr, *rank = (int *)ctx->pat_b.p;
+    const Tiles tl{(unsigned *)w + 2, (unsigned *)w + 2 + tiles};
+    const PatExtra x{(int2 *)ctx->pat_a.p, rank, (int *)ctx->pat_cnt.p, (int *)ctx->bp_l.p, (int *)ctx->bp_l.p + nr,
+                     rank + mi, rank + 2 * mi, (unsigned *)w};
+    const dim3 b(256);
+    // The elements' and CZs' distinct blocks are kept and used while their node ids and the altIds
+    // are what they were, which the same launches find out; where they are not, all is built anew.
+    bool fresh = !kept;
+    Report rep;
+    for (;; fresh = true) {
+        rep = new_report(ctx);
+        if (fresh) {
+            pc.valid = false;
+            if (int r = grow(ctx, pc.rows, sizeof(int) * (nr + 1))) return r;
+            if (int r = grow(ctx, pc.cols, sizeof(int) * (size_t)Ms + 1)) return r;
+            if (int r = grow(ctx, pc.snap, sizeof(int) * (size_t)nsnap + 1)) return r;
+            if (int r = grow(ctx, ctx->pat_a, sizeof(unsigned long long) * (size_t)Ms + 1)) return r;
+            if (int r = grow(ctx, ctx->pat_b, sizeof(unsigned long long) * (size_t)Ms + 1)) return r;
+            auto *ka = (unsigned long long *)ctx->pat_a.p, *kb = (unsigned long long *)ctx->pat_b.p;
+            int *count = nullptr;
+            if (Ms > 0) {
+                count = w + 1;
+                size_t sb = 0;
+                HIPCHK(ctx, hipcub::DeviceRadixSort::SortKeys(nullptr, sb, ka, kb, (int)Ms, 0, 2 * cb, ctx->stream));
+                if (int r = grow(ctx, ctx->scan_tmp, sb)) return r;
+                hipLaunchKernelGGL(k_pat_emit, dim3(blocks_for(Ms, 256)), b, 0, ctx->stream, el, cz, altId, nNodes, N,
+                                   cb, ka, tl, ktiles, rep);
+                HIPCHK(ctx, hipcub::DeviceRadixSort::SortKeys(ctx->scan_tmp.p, sb, ka, kb, (int)Ms, 0, 2 * cb,
+                                                              ctx->stream));
+                hipLaunchKernelGGL(k_pat_count, dim3(ktiles), b, 0, ctx->stream, kb, Ms, cb, tl);
+                hipLaunchKernelGGL(k_pat_compact, dim3(ktiles), b, 0, ctx->stream, kb, Ms, cb, tl, ka, (int *)pc.cols.p,
+                                   count);
+            }
+            hipLaunchKernelGGL(k_pat_rows, dim3(blocks_for((long long)N + 1, 256)), b, 0, ctx->stream, ka, count, N, cb,
+                               (int *)pc.rows.p);
+            if (nsnap > 0)
+                hipLaunchKernelGGL(k_pat_snap, dim3(blocks_for(nsnap, 256)), b, 0, ctx->stream, pf, nsnap,
+                                   (int *)pc.snap.p);
+        }
+        const int *srow = (const int *)pc.rows.p, *scol = (const int *)pc.cols.p;
+        PatExtra xe = x;           // the buffers may have moved for the keys
+        xe.item = (int2 *)ctx->pat_a.p;
+        xe.rank = (int *)ctx->pat_b.p;
+        xe.raw = xe.rank + mi;
+        xe.cols = xe.raw + mi;
+        const unsigned cmp = fresh ? 0u : blocks_for(nsnap, 256), pairs = blocks_for(Mi, 256);
+        if (cmp + pairs)
+            hipLaunchKernelGGL(k_pat_extra, dim3(cmp + pairs), b, 0, ctx->stream, pf, nsnap, (const int *)pc.snap.p, cmp,
+                               im, nNodes, N, srow, scol, xe, tl, rtiles, rep);
+        if (Mi > 0 && N > 0) {
+            hipLaunchKernelGGL(k_pat_reserve, dim3(rtiles), b, 0, ctx->stream, N, xe);
+            hipLaunchKernelGGL(k_pat_fill, dim3(pairs), b, 0, ctx->stream, Mi, xe);
+            hipLaunchKernelGGL(k_pat_distinct, dim3(rtiles), b, 0, ctx->stream, N, xe, tl);
+        }
+        hipLaunchKernelGGL(k_pat_write, dim3(blocks_for((long long)N + 1, 256)), b, 0, ctx->stream, srow, scol, N,
+                           Mi > 0 && N > 0, xe, tl, rtiles, max_nnz, csr_rows, csr_cols, rep);
         HIPCHK(ctx, hipGetLastError());
-        HIPCHK(ctx, hipMemcpyAsync(count, pos + M, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        return 0;
-    };
-    auto sort_keys = [&](unsigned long long *in, unsigned long long *out, long long M) -> int {
-        size_t sb = 0;
-        HIPCHK(ctx, hipcub::DeviceRadixSort::SortKeys(nullptr, sb, in, out, (int)M, 0, 2 * cb, ctx->stream));
-        if (int r = grow(ctx, ctx->scan_tmp, sb)) return r;
-        HIPCHK(ctx, hipcub::DeviceRadixSort::SortKeys(ctx->scan_tmp.p, sb, in, out, (int)M, 0, 2 * cb, ctx->stream));
-        return 0;
-    };
-    if (!hit) {
-        pc.valid = false;
-        int nk = 0;
-        if (Ms > 0) {
-            if (int r = grow(ctx, ctx->pat_a, sizeof(unsigned long long) * (size_t)Ms)) return r;
-            if (int r = grow(ctx, ctx->pat_b, sizeof(unsigned long long) * (size_t)Ms)) return r;
-            if (int r = grow(ctx, pc.keys, sizeof(unsigned long long) * (size_t)Ms)) return r;
-            auto *a = (unsigned long long *)ctx->pat_a.p, *b = (unsigned long long *)ctx->pat_b.p;
-            for (int k = 0; k < 2; k++)
-                if (src[k].n)
-                    hipLaunchKernelGGL(k_pat_emit, dim3(blocks_for((long long)src[k].n * pat_pairs(src[k].K, 0), 256)),
-                                       dim3(256), 0, ctx->stream, src[k], altId, nNodes, N, cb, a, d_err);
-            if (int r = sort_keys(a, b, Ms)) return r;
-            if (int r = distinct(b, Ms, (unsigned long long *)pc.keys.p, &nk)) return r;
-        }
-        int err = 0;
-        HIPCHK(ctx, hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        if (err) return fail(ctx, ICF_E_INDEX, "icf_build_pattern: a node id or altId is out of range");
-        if (nsnap > 0) {
-            if (int r = grow(ctx, pc.snap, sizeof(int) * (size_t)nsnap)) return r;
-            hipLaunchKernelGGL(k_pat_snap, dim3(blocks_for(nsnap, 256)), dim3(256), 0, ctx->stream, pf, nsnap,
-                               (int *)pc.snap.p, 0, d_diff);
-            HIPCHK(ctx, hipGetLastError());
-        }
+        if (fresh || !reported(rep, PAT_DIFF)) break;
+    }
+    if (fresh && !reported(rep, PAT_ERR_STATIC)) {
         pc.nNodes = nNodes, pc.nElems = nElems, pc.el_stride = el_stride, pc.nCZs = nCZs;
-        pc.cz_stride = cz_stride, pc.N = N, pc.cb = cb, pc.nkeys = nk;
+        pc.cz_stride = cz_stride, pc.N = N;
         pc.valid = true;
     }
-    // the impacts' keys, sorted and merged into the static part's
-    int num = pc.nkeys;
-    const unsigned long long *uniq = (const unsigned long long *)pc.keys.p;
-    if (Mi > 0) {
-        const long long Mt = pc.nkeys + Mi;
-        if (int r = grow(ctx, ctx->pat_a, sizeof(unsigned long long) * (size_t)std::max(2 * Mi, Mt))) return r;
-        if (int r = grow(ctx, ctx->pat_b, sizeof(unsigned long long) * (size_t)Mt)) return r;
-        auto *a = (unsigned long long *)ctx->pat_a.p, *b = (unsigned long long *)ctx->pat_b.p;
-        hipLaunchKernelGGL(k_pat_emit, dim3(blocks_for(Mi, 256)), dim3(256), 0, ctx->stream, src[2], altId, nNodes, N,
-                           cb, a, d_err);
-        if (int r = sort_keys(a, a + Mi, Mi)) return r;
-        size_t mb = 0;
-        HIPCHK(ctx, hipcub::DeviceMerge::MergeKeys(nullptr, mb, (const unsigned long long *)pc.keys.p, pc.nkeys,
-                                                   (const unsigned long long *)(a + Mi), (int)Mi, b,
-                                                   ::rocprim::less<unsigned long long>(), ctx->stream));
-        if (int r = grow(ctx, ctx->scan_tmp, mb)) return r;
-        HIPCHK(ctx, hipcub::DeviceMerge::MergeKeys(ctx->scan_tmp.p, mb, (const unsigned long long *)pc.keys.p,
-                                                   pc.nkeys, (const unsigned long long *)(a + Mi), (int)Mi, b,
-                                                   ::rocprim::less<unsigned long long>(), ctx->stream));
-        if (int r = distinct(b, Mt, a, &num)) return r;
-        uniq = a;
-    }
-    int err = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&err, d_err, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (err) return fail(ctx, ICF_E_INDEX, "icf_build_pattern: a node id or altId is out of range");
-    const int n_nz = num;
-    *nnz = n_nz;
-    if (n_nz > max_nnz) return fail(ctx, ICF_E_CAPACITY, "icf_build_pattern: more blocks than max_nnz");
-    const unsigned long long *u = uniq;
-    if (n_nz > 0)
-        hipLaunchKernelGGL(k_pat_cols, dim3(blocks_for(n_nz, 256)), dim3(256), 0, ctx->stream, u, n_nz, cb, csr_cols);
-    hipLaunchKernelGGL(k_pat_rows, dim3(blocks_for((long long)N + 1, 256)), dim3(256), 0, ctx->stream, u, n_nz, N, cb,
-                       csr_rows);
-    HIPCHK(ctx, hipGetLastError());
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    if (reported(rep, PAT_ERR_STATIC) || reported(rep, PAT_ERR_IMPACT))
+        return fail(ctx, ICF_E_INDEX, "icf_build_pattern: a node id or altId is out of range");
+    *nnz = (int)((volatile unsigned *)rep.host)[PAT_NNZ];
+    if (*nnz > max_nnz) return fail(ctx, ICF_E_CAPACITY, "icf_build_pattern: more blocks than max_nnz");
     return 0;
 }
 

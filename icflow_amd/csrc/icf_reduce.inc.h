@@ -115,27 +115,6 @@ __device__ inline int tile_job(const MapJobs &J, int &k0)
     return j;
 }
 
-// Exclusive scan over the 256 threads of the workgroup; total in every thread.
-__device__ inline unsigned long long scan256(unsigned long long v, unsigned long long *part, unsigned long long &total)
-{
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    unsigned long long x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const unsigned long long y = __shfl_up(x, o);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) part[wave] = x;
-    __syncthreads();
-    unsigned long long before = 0;
-    total = 0;
-    for (int w = 0; w < 4; w++) {
-        if (w < wave) before += part[w];
-        total += part[w];
-    }
-    __syncthreads();
-    return before + x - v;
-}
-
 __global__ __launch_bounds__(256) void k_map_tiles(MapJobs J, const int *__restrict__ cnt,
                                                    unsigned long long *__restrict__ sums)
 {
