@@ -484,18 +484,28 @@ __global__ __launch_bounds__(256) void k_bp_place(const unsigned long long *__re
     }
 }
 
-// NL2set, pass 1: tuples per candidate pair (set bits of its mask).
-__global__ __launch_bounds__(256) void k_nl2_count(const int *__restrict__ masks, int nPairs, int *__restrict__ cnt)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nPairs) return;
-    cnt[i] = __popc((unsigned)masks[2LL * i] & 0xffu);
-}
-
-// Pass 2: the (node << 32 | tet) keys in insertion order (position o), each inserted into an
-// open-addressing table (linear probing, at most half full) that keeps the smallest
-// position of every key: its first occurrence.
+// NL2set: the distinct (node, tet) tuples of the candidate pairs' masks, in the order of their first
+// occurrence (pair, then bit).  Every tuple goes into an open-addressing table (linear probing)
+// that keeps its smallest place 8 * pair + bit; the places that are their tuple's smallest are
+// counted per 256 pairs and written behind the pairs before (Tiles).  Four launches and one wait, with
+// the table as large as the last call's distinct tuples ask for (a tuple without a slot is reported,
+// and the host repeats the call with a table for all).  With the tuples counted, scanned and listed
+// first it took 13 launches and two waits, 166 us a call on the 384,000-tet compression (1.66M
+// pairs, 416,000 bits) and 122 us on one of 3,072 tets; now 73 and 35.  Three chains of dependent
+// reads (masks, pairs and node ids, table) bound it: a pair has few bits, so the set bits of 256
+// pairs are gathered in LDS and taken by one thread each.
 constexpr unsigned long long NL2_EMPTY = ~0ULL;   // no key: node and tet ids are >= 0
+constexpr int NL2_FULL = 0, NL2_TOTAL = 17, NL2_NUM = 18;   // words of the report; the last two are values
+constexpr unsigned long long NL2_MAX = 1ULL << 28;          // tuples of one call, repeated ones counted
+// Four slots, read in one go: a search is one read almost always.
+struct alignas(64) Nl2Bucket {
+    unsigned long long key[4], place[4];
+};
+struct Nl2Table {
+    Nl2Bucket *bucket;
+    unsigned long long mask;      // buckets - 1
+    unsigned *bits;               // set bits per Tiles::GROUP workgroups, as Tiles keeps them
+};
 __device__ inline unsigned long long nl2_hash(unsigned long long k)
 {
     k ^= k >> 33;
@@ -503,68 +513,169 @@ __device__ inline unsigned long long nl2_hash(unsigned long long k)
     k ^= k >> 33;
     return k;
 }
-__global__ __launch_bounds__(256) void k_nl2_emit(const int *__restrict__ masks, const int *__restrict__ pairs,
-                                                  int nPairs, const int *__restrict__ ie, int es,
-                                                  const int *__restrict__ off, unsigned long long *__restrict__ key,
-                                                  unsigned long long *__restrict__ tkey, int *__restrict__ tpos,
-                                                  unsigned long long tmask)
+
+// bit 0-3: vertex s of B inside A; bits 4-7: vertex s-4 of A inside B
+__device__ inline unsigned long long nl2_key(const int *pairs, int i, int s, const int *ie, int es)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nPairs) return;
-    const int bits = masks[2LL * i] & 0xff;
-    if (!bits) return;
     const int tA = pairs[2LL * i], tB = pairs[2LL * i + 1];
-    int o = off[i];
-    for (int s = 0; s < 8; s++) {
-        if (!(bits & (1 << s))) continue;
-        // bits 0-3: vertex s of B inside A; bits 4-7: vertex s-4 of A inside B
-        const int node = s < 4 ? ie[tB + (size_t)es * s] : ie[tA + (size_t)es * (s - 4)];
-        const int tet = s < 4 ? tA : tB;
-        const unsigned long long k = ((unsigned long long)(unsigned)node << 32) | (unsigned)tet;
-        key[o] = k;
-        for (unsigned long long h = nl2_hash(k) & tmask;; h = (h + 1) & tmask) {
-            const unsigned long long prev = atomicCAS(&tkey[h], NL2_EMPTY, k);
-            if (prev == NL2_EMPTY || prev == k) {
-                atomicMin(&tpos[h], o);
-                break;
-            }
-        }
-        o++;
+    const int node = s < 4 ? ie[tB + (size_t)es * s] : ie[tA + (size_t)es * (s - 4)];
+    return ((unsigned long long)(unsigned)node << 32) | (unsigned)(s < 4 ? tA : tB);
+}
+
+// list[0 .. total) = 8 * thread + bit of the workgroup's set bits, in order; total in every thread.
+__device__ inline unsigned nl2_list(unsigned bits, unsigned short *list, unsigned *part)
+{
+    unsigned total, at = scan256((unsigned)__popc(bits), part, total);
+    for (; bits; bits &= bits - 1) list[at++] = (unsigned short)(threadIdx.x * 8 + (unsigned)__ffs(bits) - 1);
+    __syncthreads();
+    return total;
+}
+
+__global__ __launch_bounds__(256) void k_nl2_clear(Nl2Table t, Tiles tiles, unsigned ntiles)
+{
+    const unsigned long long h = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (h <= 4 * t.mask + 3) {
+        t.bucket[h / 4].key[h % 4] = NL2_EMPTY;
+        t.bucket[h / 4].place[h % 4] = ~0ULL;
+    }
+    if (blockIdx.x == 0) {
+        Tiles::clear(tiles.groups, ntiles);
+        Tiles::clear(t.bits, ntiles);
     }
 }
 
-// Pass 3: keep[o] = 1 where position o is its key's first occurrence (keep[n] = 0 is set by
-// the caller, so the exclusive scan of keep ends with the count).
-__global__ __launch_bounds__(256) void k_nl2_keep(const unsigned long long *__restrict__ key, int n,
-                                                  const unsigned long long *__restrict__ tkey,
-                                                  const int *__restrict__ tpos, unsigned long long tmask,
-                                                  int *__restrict__ keep)
+// A vertex belongs to some twenty tets, so a tuple comes up as often, mostly in neighbouring pairs:
+// those of the same 256 pairs are found in a small table in LDS first (a tuple that finds no slot
+// in it within 8 steps is taken for a new one), and only the others go to the large one.
+// firsts[i] = the bits of pair i that did.
+constexpr int NL2_LOCAL = 1024;
+constexpr unsigned short NL2_NONE = 0xffff;
+__global__ __launch_bounds__(256) void k_nl2_emit(const int *__restrict__ masks, const int *__restrict__ pairs,
+                                                  int nPairs, const int *__restrict__ ie, int es, Nl2Table t,
+                                                  unsigned long long probes, unsigned char *__restrict__ firsts,
+                                                  Report rep)
 {
-    const int o = blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= n) return;
-    const unsigned long long k = key[o];
-    unsigned long long h = nl2_hash(k) & tmask;
-    while (tkey[h] != k) h = (h + 1) & tmask;
-    keep[o] = tpos[h] == o ? 1 : 0;
+    __shared__ unsigned long long lkey[NL2_LOCAL];
+    __shared__ unsigned lplace[NL2_LOCAL], part[4], first[256];
+    __shared__ unsigned short list[2048], at[2048];
+    const int w = xcd_remap(blockIdx.x, gridDim.x), i0 = w * 256, i = i0 + (int)threadIdx.x;
+    for (int h = threadIdx.x; h < NL2_LOCAL; h += 256) {
+        lkey[h] = NL2_EMPTY;
+        lplace[h] = ~0u;
+    }
+    first[threadIdx.x] = 0u;
+    const unsigned total = nl2_list(i < nPairs ? (unsigned)masks[2LL * i] & 0xffu : 0u, list, part);
+    if (threadIdx.x == 0) Tiles::add(t.bits, (unsigned)w, total);
+    for (unsigned e = threadIdx.x; e < total; e += 256) {
+        const unsigned long long k = nl2_key(pairs, i0 + (list[e] >> 3), list[e] & 7, ie, es);
+        unsigned h = (unsigned)nl2_hash(k) % NL2_LOCAL;
+        unsigned short slot = NL2_NONE;
+        for (int n = 0; n < 8 && slot == NL2_NONE; n++, h = (h + 1) % NL2_LOCAL) {
+            const unsigned long long prev = atomicCAS(&lkey[h], NL2_EMPTY, k);
+            if (prev == NL2_EMPTY || prev == k) slot = (unsigned short)h;
+        }
+        if (slot != NL2_NONE) atomicMin(&lplace[slot], e);
+        at[e] = slot;
+    }
+    __syncthreads();
+    for (unsigned e = threadIdx.x; e < total; e += 256) {
+        const unsigned short slot = at[e];
+        if (slot != NL2_NONE && lplace[slot] != e) continue;
+        const int l = list[e] >> 3, s = list[e] & 7;
+        atomicOr(&first[l], 1u << s);
+        const unsigned long long k = slot != NL2_NONE ? lkey[slot] : nl2_key(pairs, i0 + l, s, ie, es);
+        const unsigned long long place = 8ULL * (unsigned)(i0 + l) + (unsigned)s;
+        unsigned long long h = nl2_hash(k) & t.mask;
+        bool done = false;
+        for (unsigned long long n = 0; n < probes && !done; n++, h = (h + 1) & t.mask) {
+            Nl2Bucket *b = t.bucket + h;
+            const Nl2Bucket was = *b;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (done) continue;
+                unsigned long long key = was.key[j];
+                if (key == NL2_EMPTY) {
+                    key = atomicCAS(&b->key[j], NL2_EMPTY, k);
+                    if (key == NL2_EMPTY) key = k;
+                }
+                done = key == k;
+                if (done && was.place[j] > place) atomicMin(&b->place[j], place);
+            }
+            if (n == 4 && !done && rep.is(NL2_FULL)) break;
+        }
+        if (!done) rep.set(NL2_FULL);
+    }
+    __syncthreads();
+    if (i < nPairs) firsts[i] = (unsigned char)first[threadIdx.x];
 }
 
-// nl2 rows 0-1: the kept keys at their places in first-occurrence order.
-__global__ __launch_bounds__(256) void k_nl2_write(const unsigned long long *__restrict__ key, int n,
-                                                   const int *__restrict__ keep, const int *__restrict__ dst,
-                                                   int *__restrict__ nl2, int ts)
+// kept[i], the bits of pair i that came first among their 256 pairs' -> those whose tuples occur
+// there first of all
+__global__ __launch_bounds__(256) void k_nl2_keep(const int *__restrict__ pairs, int nPairs,
+                                                  const int *__restrict__ ie, int es, Nl2Table t,
+                                                  unsigned char *__restrict__ kept, Tiles tiles, Report rep)
 {
-    const int o = blockIdx.x * blockDim.x + threadIdx.x;
-    if (o >= n || !keep[o]) return;
-    const int k = dst[o];
-    if (k >= ts) return;   // beyond the output's capacity: the caller reports the count
-    nl2[k] = (int)(key[o] >> 32);
-    nl2[k + (size_t)ts] = (int)(key[o] & 0xffffffffULL);
+    __shared__ unsigned short list[2048];
+    __shared__ unsigned part[4], keep[256];
+    if (rep.was(NL2_FULL)) return;
+    const int w = xcd_remap(blockIdx.x, gridDim.x), i0 = w * 256, i = i0 + (int)threadIdx.x;
+    keep[threadIdx.x] = 0u;
+    const unsigned total = nl2_list(i < nPairs ? kept[i] : 0u, list, part);
+    unsigned num = 0;
+    if (total) {
+        for (unsigned e = threadIdx.x; e < total; e += 256) {
+            const int l = list[e] >> 3, s = list[e] & 7;
+            const unsigned long long k = nl2_key(pairs, i0 + l, s, ie, es);
+            unsigned long long h = nl2_hash(k) & t.mask;
+            const unsigned long long place = 8ULL * (unsigned)(i0 + l) + (unsigned)s;
+            for (bool found = false; !found; h = (h + 1) & t.mask) {
+                const Nl2Bucket b = t.bucket[h];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    if (b.key[j] != k) continue;
+                    found = true;
+                    if (b.place[j] == place) {
+                        atomicOr(&keep[l], 1u << s);
+                        num++;
+                    }
+                }
+            }
+        }
+        num = sum256(num, part);
+        if (i < nPairs) kept[i] = (unsigned char)keep[threadIdx.x];
+    }
+    if (threadIdx.x == 0) tiles.put((unsigned)w, num);
 }
 
-__global__ void k_fill_u64(unsigned long long *__restrict__ p, long long n, unsigned long long v)
+// nl2 rows 0-1: the kept tuples at their places; those beyond ts are left out (the caller reports
+// the count).
+__global__ __launch_bounds__(256) void k_nl2_write(const unsigned char *__restrict__ kept,
+                                                   const int *__restrict__ pairs, int nPairs,
+                                                   const int *__restrict__ ie, int es, Nl2Table t, Tiles tiles,
+                                                   int *__restrict__ nl2, int ts, Report rep)
 {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+    __shared__ unsigned part[4];
+    __shared__ unsigned long long part8[4];
+    unsigned long long bits = 0, total;
+    for (unsigned g = threadIdx.x; g < Tiles::ngroups(gridDim.x); g += 256) bits += t.bits[(size_t)g * Tiles::STRIDE];
+    (void)scan256(bits, part8, total);
+    if (blockIdx.x == 0 && threadIdx.x == 0) rep.put(NL2_TOTAL, (unsigned)(total > NL2_MAX ? NL2_MAX + 1 : total));
+    if (rep.was(NL2_FULL) || total > NL2_MAX) return;
+    if (blockIdx.x == 0) {
+        const unsigned num = tiles.total(gridDim.x, part);
+        if (threadIdx.x == 0) rep.put(NL2_NUM, num);
+    }
+    if (tiles.sums[blockIdx.x] == 0) return;
+    const int i = blockIdx.x * 256 + (int)threadIdx.x;
+    unsigned m = i < nPairs ? kept[i] : 0u, all;
+    unsigned at = tiles.before(blockIdx.x, part);
+    at += scan256((unsigned)__popc(m), part, all);
+    for (; m; m &= m - 1, at++) {
+        if (at >= (unsigned)ts) break;
+        const unsigned long long k = nl2_key(pairs, i, __ffs(m) - 1, ie, es);
+        nl2[at] = (int)(k >> 32);
+        nl2[at + (size_t)ts] = (int)(k & 0xffffffffULL);
+    }
 }
 
 }  // namespace icf

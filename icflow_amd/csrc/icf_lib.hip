@@ -239,6 +239,7 @@ struct icf_ctx {
     DevBuf bp_f, bp_i, bp_l;         // broad phase and NL2set scratch (doubles, ints, int64)
     DevBuf bp_c;                     // broad phase grid (cell counts, first sorted position per cell key)
     DevBuf bp_g;                     // broad phase pair grouping (counts and starts per tet, ranks)
+    long long nl2_last = 0;          // distinct tuples of the last NL2set call
     long long bp_cap = 0;            // pair keys the broad phase's buffer holds (grows with use)
     DevBuf map_cnt, map_rank, map_sums;   // building slot maps: counts (zero in between), ranks, tile sums
     DevBuf tsum;                     // per-node tet sums of the fused call
@@ -2422,7 +2423,7 @@ int icf_build_pattern(icf_ctx *ctx, const int *altId, int nNodes, const int *ie,
                       pc.nCZs == nCZs && pc.cz_stride == cz_stride && pc.N == N;
     // scratch: keys and their distinct ones, or the impacts' pairs; counts per tile of keys or rows
     const unsigned ktiles = blocks_for(Ms, PAT_TILE), rtiles = blocks_for(N, 256), tiles = std::max(ktiles, rtiles);
-    const size_t nr = (size_t)N, mi = (size_t)Mi, nt = (size_t)tiles + Tiles::ngroups(tiles);
+    const size_t nr = (size_t)N, mi = (size_t)Mi, nt = (size_t)tiles + Tiles::group_words(tiles);
     const size_t keys = kept ? 0 : (size_t)Ms;
     if (int r = grow(ctx, ctx->pat_a, std::max(sizeof(unsigned long long) * keys, sizeof(int2) * mi) + 1)) return r;
     if (int r = grow(ctx, ctx->pat_b, std::max(sizeof(unsigned long long) * keys, sizeof(int) * 3 * mi) + 1)) return r;
@@ -2687,48 +2688,40 @@ int icf_nl2set(icf_ctx *ctx, const int *masks, const int *pairs, int nPairs, con
     *nOut = 0;
     if (nPairs == 0) return 0;
     if (int r = note_write(ctx, nl2, sizeof(int) * 2 * (size_t)tet_stride, "icf_nl2set")) return r;
-    if (int r = grow(ctx, ctx->bp_i, sizeof(int) * 2 * ((size_t)nPairs + 1))) return r;
-    int *cnt = (int *)ctx->bp_i.p, *off = cnt + nPairs + 1;
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, cnt + nPairs, 1, 0);
-    hipLaunchKernelGGL(k_nl2_count, dim3(blocks_for(nPairs, 256)), dim3(256), 0, ctx->stream, masks, nPairs, cnt);
-    size_t b1 = 0;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, b1, cnt, off, nPairs + 1, ctx->stream));
-    if (int r = grow(ctx, ctx->scan_tmp, b1)) return r;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, b1, cnt, off, nPairs + 1, ctx->stream));
-    int total = 0;
-    HIPCHK(ctx, hipMemcpyAsync(&total, off + nPairs, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (total == 0) return 0;
-    if (total > (1 << 28)) return fail(ctx, ICF_E_CAPACITY, "icf_nl2set: more than 2^28 tuples");
-    // the table: a power of two at least twice the tuples
-    unsigned long long H = 1;
-    while (H < 2ULL * (unsigned long long)total) H <<= 1;
-    if (int r = grow(ctx, ctx->pat_a, sizeof(unsigned long long) * ((size_t)total + H))) return r;
-    if (int r = grow(ctx, ctx->bp_l, sizeof(int) * ((size_t)H + 2 * (size_t)total + 2))) return r;
-    auto *key = (unsigned long long *)ctx->pat_a.p, *tkey = key + total;
-    int *tpos = (int *)ctx->bp_l.p, *keep = tpos + H, *dst = keep + total + 1;
-    hipLaunchKernelGGL(k_fill_u64, dim3(blocks_for((long long)H, 256)), dim3(256), 0, ctx->stream, tkey, (long long)H,
-                       NL2_EMPTY);
-    hipLaunchKernelGGL(k_fill_int, dim3(blocks_for((long long)H, 256)), dim3(256), 0, ctx->stream, tpos, (int)H,
-                       INT_MAX);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, ctx->stream, keep + total, 1, 0);
-    hipLaunchKernelGGL(k_nl2_emit, dim3(blocks_for(nPairs, 256)), dim3(256), 0, ctx->stream, masks, pairs, nPairs, ie,
-                       el_all_stride, off, key, tkey, tpos, H - 1);
-    hipLaunchKernelGGL(k_nl2_keep, dim3(blocks_for(total, 256)), dim3(256), 0, ctx->stream, key, total, tkey, tpos,
-                       H - 1, keep);
-    size_t s1 = 0;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, s1, keep, dst, total + 1, ctx->stream));
-    if (int r = grow(ctx, ctx->scan_tmp, s1)) return r;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, s1, keep, dst, total + 1, ctx->stream));
-    // the tuples that fit are written before the count is read, so one wait serves both
-    hipLaunchKernelGGL(k_nl2_write, dim3(blocks_for(total, 256)), dim3(256), 0, ctx->stream, key, total, keep, dst,
-                       nl2, tet_stride);
-    int num = 0;
-    HIPCHK(ctx, hipGetLastError());
-    HIPCHK(ctx, hipMemcpyAsync(&num, dst + total, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    *nOut = num;
-    if (num > tet_stride) return fail(ctx, ICF_E_CAPACITY, "icf_nl2set: more tuples than tet_stride");
+    const unsigned nb = blocks_for(nPairs, 256);
+    const size_t ng = Tiles::group_words(nb);
+    if (int r = grow(ctx, ctx->bp_i, (size_t)nPairs)) return r;
+    if (int r = grow(ctx, ctx->bp_l, sizeof(unsigned) * ((size_t)nb + 2 * ng))) return r;
+    auto *w = (unsigned *)ctx->bp_l.p;
+    const Tiles tl{w, w + nb};
+    auto *kept = (unsigned char *)ctx->bp_i.p;
+    // the table: a power of two at least twice the last call's distinct tuples (a quarter more) or one
+    // for 16 pairs; a tuple without a slot in 16 buckets asks for another round with room for all
+    unsigned long long need = std::max({2048LL, ctx->nl2_last + ctx->nl2_last / 4, (long long)nPairs / 16});
+    for (int round = 0;; round++) {
+        unsigned long long H = 1;
+        while (H < 2ULL * need) H <<= 1;
+        if (int r = grow(ctx, ctx->pat_a, sizeof(Nl2Bucket) * (H / 4))) return r;
+        const Nl2Table t{(Nl2Bucket *)ctx->pat_a.p, H / 4 - 1, w + nb + ng};
+        const Report rep = new_report(ctx);
+        hipLaunchKernelGGL(k_nl2_clear, dim3(blocks_for((long long)H, 256)), dim3(256), 0, ctx->stream, t, tl, nb);
+        hipLaunchKernelGGL(k_nl2_emit, dim3(nb), dim3(256), 0, ctx->stream, masks, pairs, nPairs, ie, el_all_stride, t,
+                           round ? H / 4 : 16ULL, kept, rep);
+        hipLaunchKernelGGL(k_nl2_keep, dim3(nb), dim3(256), 0, ctx->stream, pairs, nPairs, ie, el_all_stride, t, kept,
+                           tl, rep);
+        hipLaunchKernelGGL(k_nl2_write, dim3(nb), dim3(256), 0, ctx->stream, kept, pairs, nPairs, ie, el_all_stride, t, tl,
+                           nl2, tet_stride, rep);
+        HIPCHK(ctx, hipGetLastError());
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        const volatile unsigned *got = rep.host;
+        need = got[NL2_TOTAL];
+        if (need > NL2_MAX) return fail(ctx, ICF_E_CAPACITY, "icf_nl2set: more than 2^28 tuples");
+        if (reported(rep, NL2_FULL)) continue;
+        *nOut = (int)got[NL2_NUM];
+        ctx->nl2_last = *nOut;
+        break;
+    }
+    if (*nOut > tet_stride) return fail(ctx, ICF_E_CAPACITY, "icf_nl2set: more tuples than tet_stride");
     return 0;
 }
 

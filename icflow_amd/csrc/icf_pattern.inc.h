@@ -73,7 +73,7 @@ __global__ __launch_bounds__(256) void k_pat_emit(PatSrc el, PatSrc cz, const in
                                                   int cb, unsigned long long *__restrict__ keys, Tiles tiles,
                                                   unsigned ntiles, Report rep)
 {
-    if (blockIdx.x == 0) tiles.clear(ntiles);
+    if (blockIdx.x == 0) Tiles::clear(tiles.groups, ntiles);
     const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const long long Me = (long long)el.n * pat_pairs(4, 0), M = Me + (long long)cz.n * pat_pairs(6, 0);
     if (t >= M) return;
@@ -192,7 +192,7 @@ __global__ __launch_bounds__(256) void k_pat_extra(PatFields f, long long nfield
         return;
     }
     if (blockIdx.x == nsnap) {
-        tiles.clear(ntiles);
+        Tiles::clear(tiles.groups, ntiles);
         if (threadIdx.x == 0) *x.cursor = 0u;
     }
     const long long t = (long long)(blockIdx.x - nsnap) * blockDim.x + threadIdx.x;
