@@ -271,7 +271,7 @@ struct icf_ctx {
         int ncand = NCAND;
         int sel = CAND_FP32;       // candidate in use
         bool tuned = false;        // a tuning has chosen it
-        int untuned = CAND_UNTUNED;    // what launches use when it is neither tuned nor set
+        int untuned = -1;              // what launches use when it is neither tuned nor set; -1: by their size
         bool active = false;       // timing the candidates in turn
         bool fixed = false;        // chosen by the caller (icf_set_chunk_keys / icf_set_shape)
         int turn = 0;              // launches started while tuning
@@ -1057,7 +1057,8 @@ void tune_end(icf_ctx *ctx, icf_ctx::Tune &t)
 // value-reduction roles: ids 0-3
 int tune_begin(icf_ctx *ctx, bool acc, bool fp64, long long keys)
 {
-    return tune_begin(ctx, ctx->tune[acc][fp64], 2 * acc + fp64, keys);
+    const int c = tune_begin(ctx, ctx->tune[acc][fp64], 2 * acc + fp64, keys);
+    return c >= 0 ? c : keys <= VALS_SMALL ? CAND_SMALL : CAND_UNTUNED;
 }
 void tune_end(icf_ctx *ctx, bool acc, bool fp64) { tune_end(ctx, ctx->tune[acc][fp64]); }
 
@@ -1102,7 +1103,7 @@ void phase1_fused(icf_ctx *ctx, const int *ie, const double *dn, int nt, int es,
     shape_end(ctx, ICF_SHAPE_PHASE1);
 }
 
-// Calls f(integral_constant<cand_keys(c)>, integral_constant<cand_stage(c)>).
+// Calls f(integral_constant<cand_keys(c)>, integral_constant<cand_stage(c)>), or the small shape.
 template <typename F>
 void with_cand(int c, F &&f)
 {
@@ -1116,7 +1117,8 @@ void with_cand(int c, F &&f)
     case 4: f(integral_constant<int, cand_keys(4)>(), integral_constant<int, cand_stage(4)>()); break;
     case 5: f(integral_constant<int, cand_keys(5)>(), integral_constant<int, cand_stage(5)>()); break;
     case 6: f(integral_constant<int, cand_keys(6)>(), integral_constant<int, cand_stage(6)>()); break;
-    default: f(integral_constant<int, cand_keys(7)>(), integral_constant<int, cand_stage(7)>()); break;
+    case 7: f(integral_constant<int, cand_keys(7)>(), integral_constant<int, cand_stage(7)>()); break;
+    default: f(integral_constant<int, SMALL_KEYS>(), integral_constant<int, SMALL_STAGE>()); break;
     }
 }
 

@@ -263,6 +263,9 @@ constexpr int CAND_FP32 = 2 * NSC + 0, CAND_FP64 = 2 * NSC + 1;   // a context's
 // batched specimens mixed 621 (627-703), 779,000 tets FP64 190 (187-201), 309,000 tets FP64 65
 // (65-75), 146,000 tets mixed 30.0 (28.6-32.8).
 constexpr int CAND_UNTUNED = 1 * NSC + 1;
+// ... and where that leaves most of the chip idle, one wave of 64 keys with room for all of their
+// contributions.
+constexpr int CAND_SMALL = NCAND, SMALL_KEYS = 64, SMALL_STAGE = 16, VALS_SMALL = 1 << 17;
 template <typename L, int KEYS, int STAGE>
 __host__ __device__ constexpr int flat_cap() { return sizeof(L) == 4 ? STAGE * KEYS : STAGE * KEYS / 2; }
 // bytes of LDS of a value reduction: the staged contributions, then the list of long keys
@@ -489,6 +492,7 @@ __device__ __forceinline__ void reduce_vals(int bid_, int nb_, const int *__rest
 #pragma unroll
         for (int q = 0; q < SLOTS; q++) {
             const int hi = min(te[q], c1) - c0;
+#pragma unroll 4
             for (int c = max(tb[q], c0) - c0; c < hi; c++) tacc[q] += (double)lds[c * 9 + comp];
         }
     };
@@ -647,7 +651,7 @@ __device__ __forceinline__ void reduce_force_rhs(int bid_, int nb_, const int *_
         int ns, const int *__restrict__ node_row, const int *__restrict__ roff, const uint32_t *__restrict__ rcodes,
         const int *__restrict__ cz_begin, double *__restrict__ rhs, Stage sv, void *smem)
 {
-    constexpr int PER = BYTES / 24 / KEYS, CAP = PER * KEYS;
+    constexpr int PER = BYTES / 24 / KEYS < 12 ? BYTES / 24 / KEYS : 12, CAP = PER * KEYS;
     static_assert(PER >= 1, "a contribution per lane");
     double *lds = (double *)smem;
     const int p0 = xcd_remap(bid_, nb_) * KEYS;
@@ -686,6 +690,7 @@ __device__ __forceinline__ void reduce_force_rhs(int bid_, int nb_, const int *_
         }
         __syncthreads();
         const int hi = min(e, c1) - c0;
+#pragma unroll 4
         for (int c = max(b, c0) - c0; c < hi; c++) {
             const double x = lds[3 * c], y = lds[3 * c + 1], z = lds[3 * c + 2];
             a0 += x; a1 += y; a2 += z;
@@ -695,10 +700,21 @@ __device__ __forceinline__ void reduce_force_rhs(int bid_, int nb_, const int *_
     if (!live) return;
     dst[0] = a0; dst[ns] = a1; dst[2 * (size_t)ns] = a2;
     if (r < 0) return;
+    // six contributions of CZs in flight, as many as a row mostly has
+    constexpr int CZS = 6;
     const int re = roff[r + 1];
-    for (int k = cz_begin[r]; k < re; k++) {
-        const Part q = part_of(sv, rcodes[k]);
-        t0 += q.x; t1 += q.y; t2 += q.z;
+    for (int k = cz_begin[r]; k < re; k += CZS) {
+        uint32_t cd[CZS];
+        Part q[CZS];
+#pragma unroll
+        for (int i = 0; i < CZS; i++) cd[i] = rcodes[min(k + i, re - 1)];
+#pragma unroll
+        for (int i = 0; i < CZS; i++) q[i] = part_of(sv, cd[i]);
+#pragma unroll
+        for (int i = 0; i < CZS; i++)
+            if (k + i < re) {
+                t0 += q[i].x; t1 += q[i].y; t2 += q[i].z;
+            }
     }
     double *o = rhs + (size_t)r * 3;
     o[0] = t0; o[1] = t1; o[2] = t2;
