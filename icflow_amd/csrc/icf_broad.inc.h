@@ -20,102 +20,130 @@ namespace icf {
 
 constexpr int BP_DIRS = 12;
 
-// Bounds of the k-DOP pass, kept as order-preserving integer images of the doubles so that
-// atomicMin / atomicMax on them are exact: {largest AABB extent, min of the AABB minimum
-// corners (x, y, z), max of the same (x, y, z)}.
-constexpr int BP_NBOUNDS = 7;
-__host__ __device__ inline unsigned long long bp_ord(double v)
+// Words of a call's report: a node id is out of range, positions are not finite, the grid has more
+// cells than the buffers; and values: the grid's cells with and without margin, the pairs, the
+// candidates of the fullest region.
+constexpr int BP_BAD = 0, BP_NONFINITE = 1, BP_BIG = 2, BP_G = 19, BP_NCELL = 20, BP_NV = 21, BP_CAND = 22;
+
+// Clears what the launches of one search count into.
+__global__ __launch_bounds__(256) void k_bp_clear(int *__restrict__ count, int ncount, int *__restrict__ acount,
+                                                  int nacount, unsigned long long *__restrict__ total, int ntotal,
+                                                  Tiles ct, unsigned nct, Tiles at, unsigned nat)
 {
-    unsigned long long u;
-    memcpy(&u, &v, sizeof(u));
-    return (u >> 63) ? ~u : (u | 0x8000000000000000ULL);
-}
-__host__ __device__ inline double bp_unord(unsigned long long u)
-{
-    u = (u >> 63) ? (u & 0x7fffffffffffffffULL) : ~u;
-    double v;
-    memcpy(&v, &u, sizeof(v));
-    return v;
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < ncount) count[i] = 0;
+    if (i < nacount) acount[i] = 0;
+    if (i < ntotal) total[i] = 0ULL;
+    if (blockIdx.x == 0) {
+        Tiles::clear(ct.groups, nct);
+        Tiles::clear(at.groups, nat);
+    }
 }
 
-__global__ void k_bp_bounds_init(unsigned long long *__restrict__ b)
-{
-    const int k = threadIdx.x;
-    // min slots start high, max slots low; slot BP_NBOUNDS is the bad-node-id flag
-    if (k <= BP_NBOUNDS) b[k] = (k >= 1 && k <= 3) ? ~0ULL : 0ULL;
-}
-
-// Tet t's 12-direction k-DOP (lo l, hi h) from its 4 nodes' current positions; false if a
-// node id is out of range.  Both kernels below compute it with this code, so their values agree
-// bit for bit.
-__device__ inline bool bp_tet_kdop(const double *__restrict__ dn, int ns, const int *__restrict__ ie, int es, int t,
-                                   int nNodesBound, double l[BP_DIRS], double h[BP_DIRS])
+// The 12 planes' value at a point, d a constant.
+__device__ inline double bp_plane(int d, double x, double y, double z)
 {
 #pragma clang fp contract(off)
-#pragma unroll
-    for (int d = 0; d < BP_DIRS; d++) {
-        l[d] = 1e300;
-        h[d] = -1e300;
+    switch (d) {
+    case 0: return x;
+    case 1: return y;
+    case 2: return z;
+    case 3: return x + y;
+    case 4: return x + z;
+    case 5: return y + z;
+    case 6: return x - y;
+    case 7: return x - z;
+    case 8: return y - z;
+    case 9: return x + y - z;
+    case 10: return x + z - y;
+    default: return y + z - x;
     }
+}
+
+// Current positions of tet t's 4 nodes; false if a node id is out of range.
+__device__ inline bool bp_tet_nodes(const double *__restrict__ dn, int ns, const int *__restrict__ ie, int es, int t,
+                                    double p[4][3])
+{
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int n = ie[t + (size_t)es * v];
-        if (n < 0 || (nNodesBound > 0 && n >= nNodesBound)) return false;
-        const double x = dn[n + (size_t)ns * ND_XC], y = dn[n + (size_t)ns * (ND_XC + 1)],
-                     z = dn[n + (size_t)ns * (ND_XC + 2)];
-        const double p[BP_DIRS] = {x, y, z, x + y, x + z, y + z, x - y, x - z, y - z, x + y - z, x + z - y, y + z - x};
+        if (n < 0 || n >= ns) return false;
 #pragma unroll
-        for (int d = 0; d < BP_DIRS; d++) {
-            l[d] = fmin(l[d], p[d]);
-            h[d] = fmax(h[d], p[d]);
-        }
+        for (int k = 0; k < 3; k++) p[v][k] = dn[n + (size_t)ns * (ND_XC + k)];
     }
     return true;
 }
 
-// Per surface tet: the minimum corner of its AABB (the k-DOP's first three lo planes, which
-// bin it into the grid), and the block's contribution to the bounds (one atomic per bound per
-// block).  k_bp_sorted computes the whole k-DOP again rather than reading 24 planes back.
-__global__ __launch_bounds__(256) void k_bp_kdop(const double *__restrict__ dn, int ns, const int *__restrict__ ie,
-                                                 int es, int nT, double *__restrict__ lo,
-                                                 unsigned long long *__restrict__ bounds, int nNodesBound)
+// The tet's extent (l, h) in direction d, a constant.  All launches below compute it with this code, so
+// their values agree bit for bit.
+__device__ inline void bp_extent(int d, const double p[4][3], double &l, double &h)
 {
-#pragma clang fp contract(off)
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    double b[BP_NBOUNDS] = {0, 1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
-    if (t < nT) {
-        double l[BP_DIRS], h[BP_DIRS];
-        if (!bp_tet_kdop(dn, ns, ie, es, t, nNodesBound, l, h)) {
-            atomicMax(&bounds[BP_NBOUNDS], 1ULL);
-        } else {
+    l = 1e300;
+    h = -1e300;
 #pragma unroll
-            for (int d = 0; d < 3; d++) lo[(size_t)d * nT + t] = l[d];
-            b[0] = fmax(h[0] - l[0], fmax(h[1] - l[1], h[2] - l[2]));
-#pragma unroll
-            for (int k = 0; k < 3; k++) b[1 + k] = b[4 + k] = l[k];
-        }
+    for (int v = 0; v < 4; v++) {
+        const double x = bp_plane(d, p[v][0], p[v][1], p[v][2]);
+        l = fmin(l, x);
+        h = fmax(h, x);
     }
-    // block reduction: across the wave, then the block's waves through LDS
-    __shared__ double part[256 / 64][BP_NBOUNDS];
+}
+
+// Bounds of the k-DOPs: {largest AABB extent, min of the AABB minimum corners (x, y, z), max of the
+// same}, one set per workgroup; BP_BLOCKS of them at most, each taking every so many tets.
+constexpr int BP_NBOUNDS = 7, BP_BLOCKS = 256;
+__device__ inline bool bp_is_max(int k) { return k == 0 || k >= 4; }
+__device__ inline void bp_bounds256(double b[BP_NBOUNDS], double part[4][BP_NBOUNDS])
+{
 #pragma unroll
     for (int k = 0; k < BP_NBOUNDS; k++) {
-        double v = b[k];
         for (int o = 32; o > 0; o >>= 1) {
-            const double w = __shfl_xor(v, o);
-            v = (k == 0 || k >= 4) ? fmax(v, w) : fmin(v, w);
+            const double w = __shfl_xor(b[k], o);
+            b[k] = bp_is_max(k) ? fmax(b[k], w) : fmin(b[k], w);
         }
-        b[k] = v;
+        if (__lane_id() == 0) part[threadIdx.x >> 6][k] = b[k];
     }
-    const int wave = threadIdx.x >> 6;
-    if (__lane_id() == 0)
-        for (int k = 0; k < BP_NBOUNDS; k++) part[wave][k] = b[k];
     __syncthreads();
+#pragma unroll
+    for (int k = 0; k < BP_NBOUNDS; k++)
+        for (int w = 0; w < 4; w++) b[k] = bp_is_max(k) ? fmax(b[k], part[w][k]) : fmin(b[k], part[w][k]);
+}
+
+// Per surface tet: the minimum corner of its AABB (the k-DOP's first three lo planes, which
+// bin it into the grid), and the workgroup's bounds.  (With one atomic per bound and 256 tets the
+// 9,700 atomics of 353,000 tets, one after the other on one cache line, made it 40 us, now 18.)  k_bp_sorted
+// computes the whole k-DOP.
+__global__ __launch_bounds__(256) void k_bp_kdop(const double *__restrict__ dn, int ns, const int *__restrict__ ie,
+                                                 int es, int nT, double *__restrict__ lo, double *__restrict__ bounds,
+                                                 Report rep)
+{
+#pragma clang fp contract(off)
+    __shared__ double part[4][BP_NBOUNDS];
+    double b[BP_NBOUNDS] = {0, 1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
+    bool bad = false;
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < nT; t += gridDim.x * 256) {
+        double p[4][3], l[3], h[3];
+        if (!bp_tet_nodes(dn, ns, ie, es, t, p)) {
+            bad = true;
+            continue;
+        }
+#pragma unroll
+        for (int d = 0; d < 3; d++) bp_extent(d, p, l[d], h[d]);
+#pragma unroll
+        for (int d = 0; d < 3; d++) lo[(size_t)d * nT + t] = l[d];
+        b[0] = fmax(b[0], fmax(h[0] - l[0], fmax(h[1] - l[1], h[2] - l[2])));
+#pragma unroll
+        for (int k = 0; k < 3; k++) {
+            b[1 + k] = fmin(b[1 + k], l[k]);
+            b[4 + k] = fmax(b[4 + k], l[k]);
+        }
+    }
+    if (bad) rep.set(BP_BAD);
+    bp_bounds256(b, part);
     if (threadIdx.x < BP_NBOUNDS) {
-        const int k = threadIdx.x;
-        double v = part[0][k];
-        for (int w = 1; w < (int)(blockDim.x >> 6); w++) v = (k == 0 || k >= 4) ? fmax(v, part[w][k]) : fmin(v, part[w][k]);
-        if (k == 0 || k >= 4) atomicMax(&bounds[k], bp_ord(v));
-        else atomicMin(&bounds[k], bp_ord(v));
+        double v = b[0];
+#pragma unroll
+        for (int k = 1; k < BP_NBOUNDS; k++) v = (int)threadIdx.x == k ? b[k] : v;
+        bounds[(size_t)blockIdx.x * BP_NBOUNDS + threadIdx.x] = v;
     }
 }
 
@@ -124,11 +152,59 @@ __global__ __launch_bounds__(256) void k_bp_kdop(const double *__restrict__ dn, 
 // one below and one above in y and z -- so that the neighbour rows a cell reads never wrap.
 // Cell (x, y, z) of the margin grid has the linear key x + gx (y + gy z).  Tets are binned
 // by the cell of their AABB's minimum corner; with cs >= every extent, overlapping tets lie
-// in the same or neighbouring cells.
+// in the same or neighbouring cells.  It lies in device memory: the launches are sized by what the
+// last search found (with room for more), and do nothing where it does not fit (ok == 0).
 struct BpGrid {
-    double cs, org[3];
-    int n[3], gx, gy, gz;
+    double cs, org[3], invq;
+    int n[3], gx, gy, gz, G, ncell, ok;
 };
+
+// A k-DOP plane in whole steps of cs / BP_STEPS from the grid's origin, modulo 2^16.  The steps do not
+// decrease with the plane, so lo <= hi of two tets means that the steps' difference hi - lo is not
+// negative, and in 16 bits that is its sign: tets of neighbouring cells are at most 3 cs apart along
+// an axis, 9 cs along a sum of three, 18,432 steps.  (Where rounding of the planes could add
+// to that, positions beyond 2^40 cs, all steps are 0, and every pair is left to the exact test.)
+constexpr double BP_STEPS = 2048;
+__device__ inline unsigned bp_step(double plane, double org, double invq)
+{
+#pragma clang fp contract(off)
+    if (invq == 0) return 0u;
+    const double t = floor((plane - org) * invq);
+    return (unsigned)(int)(t - 65536.0 * floor(t * (1.0 / 65536.0)));
+}
+
+// The grid of these bounds: cells at least the largest extent, coarsened (any size >= the extents
+// finds the same pairs) until the margin grid has at most 2^24 cells.  False if they are not finite.
+__device__ inline bool bp_make_grid(const double b[BP_NBOUNDS], BpGrid &g)
+{
+#pragma clang fp contract(off)
+    double span[3];
+    for (int k = 0; k < 3; k++) {
+        g.org[k] = b[1 + k];
+        span[k] = b[4 + k] - b[1 + k];
+        if (!isfinite(g.org[k]) || !isfinite(span[k])) return false;
+    }
+    g.cs = b[0] > 0 ? b[0] * 1.000001 : 1.0;
+    for (;;) {
+        double cells = 1;
+        for (int k = 0; k < 3; k++) {
+            const double c = floor(span[k] / g.cs) + 1;
+            g.n[k] = c < (double)(1 << 24) ? (int)c : (1 << 24);
+            cells *= (double)g.n[k] + (k == 0 ? 3 : 2);
+        }
+        if (cells <= (double)(1 << 24)) break;
+        g.cs *= 1.25;
+    }
+    double far = 0;
+    for (int k = 0; k < 3; k++) far = fmax(far, fmax(fabs(b[1 + k]), fabs(b[4 + k])));
+    g.invq = isfinite(g.cs) && far <= g.cs * 1099511627776.0 ? BP_STEPS / g.cs : 0.0;
+    g.gx = g.n[0] + 3;
+    g.gy = g.n[1] + 2;
+    g.gz = g.n[2] + 2;
+    g.G = g.gx * g.gy * g.gz;
+    g.ncell = g.n[0] * g.n[1] * g.n[2];
+    return true;
+}
 
 // The rank of this lane's key among all ranks taken from count[key] (bumped atomically), for
 // lanes with on set (-1 for the others): one atomicAdd per run of consecutive such lanes with
@@ -155,14 +231,38 @@ __device__ inline int run_rank(bool on, unsigned key, int *__restrict__ count)
     return on ? base + lane - h : -1;
 }
 
-// Per tet: its cell key and its rank among the tets of its cell (count[key] is bumped
+// The grid, made by every workgroup from the nb sets of bounds and left in *grid by the first; per
+// tet: its cell key and its rank among the tets of its cell (count[key] is bumped
 // atomically, so the order within a cell varies from call to call; the pairs do not).
-__global__ __launch_bounds__(256) void k_bp_cell(const double *__restrict__ lo, int nT, BpGrid g,
-                                                 unsigned *__restrict__ key, int *__restrict__ rank,
-                                                 int *__restrict__ count)
+__global__ __launch_bounds__(256) void k_bp_cell(const double *__restrict__ lo, int nT,
+                                                 const double *__restrict__ bounds, int nb, int capG, int capC,
+                                                 BpGrid *__restrict__ grid, unsigned *__restrict__ key,
+                                                 int *__restrict__ rank, int *__restrict__ count, Report rep)
 {
+    __shared__ double part[4][BP_NBOUNDS];
+    __shared__ BpGrid g;
+    double b[BP_NBOUNDS] = {0, 1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
+    if ((int)threadIdx.x < nb) {
+#pragma unroll
+        for (int k = 0; k < BP_NBOUNDS; k++) b[k] = bounds[(size_t)threadIdx.x * BP_NBOUNDS + k];
+    }
+    bp_bounds256(b, part);
+    if (threadIdx.x == 0) {
+        const bool bad = rep.was(BP_BAD), finite = !bad && bp_make_grid(b, g);
+        g.ok = finite && g.G <= capG && g.ncell <= capC;
+        if (blockIdx.x == 0) {
+            *grid = g;
+            if (!bad && !finite) rep.set(BP_NONFINITE);
+            if (finite && !g.ok) rep.set(BP_BIG);
+            if (finite) {
+                rep.put(BP_G, (unsigned)g.G);
+                rep.put(BP_NCELL, (unsigned)g.ncell);
+            }
+        }
+    }
+    __syncthreads();
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nT) return;
+    if (!g.ok || t >= nT) return;
     int c[3];
 #pragma unroll
     for (int a = 0; a < 3; a++) {
@@ -174,37 +274,109 @@ __global__ __launch_bounds__(256) void k_bp_cell(const double *__restrict__ lo, 
     rank[t] = run_rank(true, k, count);   // neighbouring tets of a mesh often share a cell
 }
 
+// out[0 .. n] = exclusive scan of v[0 .. n) in two launches (n: the grid's cells when grid is given, which
+// the launches cover); the second puts the sum into word `word` of the report when not negative.
+constexpr int BP_ITEMS = 8, BP_TILE = 256 * BP_ITEMS;
+__global__ __launch_bounds__(256) void k_bp_tiles(const int *__restrict__ v, int n, const BpGrid *__restrict__ grid,
+                                                  Tiles tiles)
+{
+    __shared__ unsigned part[4];
+    if (!grid->ok) return;
+    if (n < 0) n = grid->G;
+    const int k0 = (int)blockIdx.x * BP_TILE;
+    if (k0 >= n) return;
+    unsigned x = 0;
+    for (int r = 0; r < BP_ITEMS; r++) {
+        const int k = k0 + r * 256 + (int)threadIdx.x;
+        if (k < n) x += (unsigned)v[k];
+    }
+    x = sum256(x, part);
+    if (threadIdx.x == 0) tiles.put(blockIdx.x, x);
+}
+__global__ __launch_bounds__(256) void k_bp_scan(const int *__restrict__ v, int n, const BpGrid *__restrict__ grid,
+                                                 Tiles tiles, int *__restrict__ out, int word, Report rep)
+{
+    __shared__ unsigned part[4];
+    if (!grid->ok) return;
+    if (n < 0) n = grid->G;
+    const int k0 = (int)blockIdx.x * BP_TILE;
+    if (k0 >= n) return;
+    unsigned run = tiles.before(blockIdx.x, part), total;
+    for (int r = 0; r < BP_ITEMS; r++) {
+        const int k = k0 + r * 256 + (int)threadIdx.x;
+        const unsigned at = run + scan256(k < n ? (unsigned)v[k] : 0u, part, total);
+        run += total;
+        if (k < n) out[k] = (int)at;
+    }
+    if (k0 + BP_TILE >= n && threadIdx.x == 0) {
+        out[n] = (int)run;
+        if (word >= 0) rep.put(word, run);
+    }
+}
+
 // The k-DOPs and node ids in cell order (a counting sort: first[key] is the exclusive scan
 // of the cell counts): tet t goes to position j = first[key[t]] + rank[t], so that the tets
 // of one cell, and of neighbouring cells, are adjacent in memory for the pair search.  Per
-// position: the tet (sidx), the k-DOP as (lo, hi) pairs per direction (skd, 24 doubles), the
-// node ids (snode), and the k-DOP in FP32 rounded outward, lo down and hi up (sk32: 12 lo then
-// 12 hi): a prefilter that never rejects a pair whose FP64 k-DOPs overlap.  first[L] for
-// L = 0 .. G is then the first position of the cells with keys >= L.
-__global__ __launch_bounds__(256) void k_bp_sorted(const double *__restrict__ dn, int ns, int nNodesBound, int nT,
+// position: the tet (sidx), the k-DOP in steps with the node ids (srec), the k-DOP as (lo, hi) pairs
+// per direction (skd) and in FP32 rounded outward, lo down and hi up (sk32: 12 lo then 12 hi): steps
+// and FP32 never reject a pair whose FP64 k-DOPs overlap.  first[L] for L = 0 .. G is then the first position of the cells with keys >= L.
+struct alignas(64) BpTet {
+    uint4 lo, mid, hi;      // lo of directions 0-7; lo 8-11, hi 0-3; hi 4-11: two to a word
+    int4 node;
+};
+__global__ __launch_bounds__(256) void k_bp_sorted(const double *__restrict__ dn, int ns, int nT,
                                                    const unsigned *__restrict__ key,
                                                    const int *__restrict__ rank, const int *__restrict__ first,
-                                                   const int *__restrict__ ie, int es, int *__restrict__ sidx,
-                                                   double2 *__restrict__ skd, int4 *__restrict__ snode,
+                                                   const int *__restrict__ ie, int es,
+                                                   const BpGrid *__restrict__ grid, int *__restrict__ sidx,
+                                                   BpTet *__restrict__ srec, double2 *__restrict__ skd,
                                                    float4 *__restrict__ sk32)
 {
+#pragma clang fp contract(off)
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nT) return;
+    if (t >= nT || !grid->ok) return;
     const int j = first[key[t]] + rank[t];
     sidx[j] = t;
-    double l[BP_DIRS], h[BP_DIRS];
-    (void)bp_tet_kdop(dn, ns, ie, es, t, nNodesBound, l, h);   // node ids checked by k_bp_kdop
+    double p[4][3];
+    (void)bp_tet_nodes(dn, ns, ie, es, t, p);   // node ids checked by k_bp_kdop
+    const double x = grid->org[0], y = grid->org[1], z = grid->org[2], invq = grid->invq;
     float f[2 * BP_DIRS];
+    unsigned q[BP_DIRS];
 #pragma unroll
     for (int d = 0; d < BP_DIRS; d++) {
-        skd[(size_t)j * BP_DIRS + d] = make_double2(l[d], h[d]);
-        f[d] = __double2float_rd(l[d]);
-        f[BP_DIRS + d] = __double2float_ru(h[d]);
+        double l, h;
+        bp_extent(d, p, l, h);
+        skd[(size_t)j * BP_DIRS + d] = make_double2(l, h);
+        f[d] = __double2float_rd(l);
+        f[BP_DIRS + d] = __double2float_ru(h);
+        const double o = bp_plane(d, x, y, z);
+        const unsigned ql = bp_step(l, o, invq), qh = bp_step(h, o, invq);
+        q[d / 2] = d % 2 ? q[d / 2] | ql << 16 : ql;
+        q[6 + d / 2] = d % 2 ? q[6 + d / 2] | qh << 16 : qh;
     }
-    snode[j] = make_int4(ie[t], ie[t + (size_t)es], ie[t + 2 * (size_t)es], ie[t + 3 * (size_t)es]);
+    BpTet r;
+    r.lo = make_uint4(q[0], q[1], q[2], q[3]);
+    r.mid = make_uint4(q[4], q[5], q[6], q[7]);
+    r.hi = make_uint4(q[8], q[9], q[10], q[11]);
+    r.node = make_int4(ie[t], ie[t + (size_t)es], ie[t + 2 * (size_t)es], ie[t + 3 * (size_t)es]);
+    srec[j] = r;
 #pragma unroll
-    for (int q = 0; q < 6; q++)
-        sk32[(size_t)j * 6 + q] = make_float4(f[4 * q], f[4 * q + 1], f[4 * q + 2], f[4 * q + 3]);
+    for (int k = 0; k < 6; k++)
+        sk32[(size_t)j * 6 + k] = make_float4(f[4 * k], f[4 * k + 1], f[4 * k + 2], f[4 * k + 3]);
+}
+
+// The sign bits (0x80008000) of hi - lo over the 12 directions, both ways; 0 where all overlap.
+typedef short s16x2 __attribute__((ext_vector_type(2)));
+__device__ inline unsigned bp_sub(unsigned a, unsigned b)
+{
+    return __builtin_bit_cast(unsigned, (s16x2)(__builtin_bit_cast(s16x2, a) - __builtin_bit_cast(s16x2, b)));
+}
+__device__ inline unsigned bp_apart(const BpTet &a, const BpTet &b)
+{
+    unsigned x = bp_sub(b.mid.z, a.lo.x) | bp_sub(b.mid.w, a.lo.y) | bp_sub(b.hi.x, a.lo.z) | bp_sub(b.hi.y, a.lo.w);
+    x |= bp_sub(b.hi.z, a.mid.x) | bp_sub(b.hi.w, a.mid.y) | bp_sub(a.mid.z, b.lo.x) | bp_sub(a.mid.w, b.lo.y);
+    x |= bp_sub(a.hi.x, b.lo.z) | bp_sub(a.hi.y, b.lo.w) | bp_sub(a.hi.z, b.mid.x) | bp_sub(a.hi.w, b.mid.y);
+    return x & 0x80008000u;
 }
 
 // A wave's LDS writes made visible to the wave's other lanes (no workgroup barrier).
@@ -215,15 +387,17 @@ __device__ inline void bp_wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// The pair search, first pass: one wave per cell of the grid's interior; the waves of a
-// workgroup meet only at its start.  The candidates are the cell's own tets and those of the 13 neighbouring cells
+// The pair search, first pass: one wave per cell of the grid's interior and slice of its tets; the
+// waves of a workgroup meet only at its start.  The candidates are the cell's own tets and those of the 13 neighbouring cells
 // with a larger key (each pair of cells visited once): 5 runs of consecutive keys -- (x, x+1)
 // of the cell's own row, and the rows (x-1 .. x+1) at (y+1, z), (y-1, z+1), (y, z+1),
 // (y+1, z+1) -- hence 5 ranges of sorted positions; in the first range only larger positions
-// pair up.  The 64 lanes hold 64 candidates at a time (FP32 k-DOP and node ids in registers,
-// loaded coalesced); the cell's own tets, BPW_OWN at a time, are staged in the wave's LDS and
-// read by all lanes at once.  A pair passes if its outward-rounded FP32 k-DOPs overlap in all
-// 12 directions and (when asked) the tets share no node.  The passing (own, candidate)
+// pair up.  The 64 lanes hold 64 candidates at a time, loaded coalesced; the own tets, BPW_OWN at a
+// time, are staged in the wave's LDS and read by all lanes at once.  The 24 comparisons of a pair
+// are 12 subtractions of two 16-bit steps each (bp_apart); the pairs that pass gather in a list
+// and are taken 64 at a time, one per lane, through the node ids (most of them share a node, and
+// are not wanted).  In FP32 with the ids compared for all pairs, 40 comparisons each with a ballot of
+// its own, 353,000 tets (1.66M pairs pass) took 264 us; now 152.  The passing (own, candidate)
 // positions collect in the wave's LDS buffer and leave in batches, one atomicAdd on the
 // counter of the workgroup's buffer region per batch (positions beyond the region's capacity
 // are only counted; the caller then grows the buffer and searches again).  What a wave holds at its end leaves with the rest of its workgroup's:
@@ -231,8 +405,16 @@ __device__ inline void bp_wave_sync()
 // (the reservations on the one counter, one per wave, took a quarter of the kernel's time).
 // Two waves per workgroup: a workgroup's LDS stays allocated until its slowest wave ends, and
 // the work per cell varies several-fold, so with four waves the resident waves averaged about
-// two per SIMD.  The second pass applies the exact FP64 test.
-constexpr int BPW_WAVES = 2, BPW_OWN = 16, BPW_BUF = 256;
+// two per SIMD.  Where the grid has too few cells to fill the chip, several waves share a cell's
+// tets, four at a time in turn (3,300 tets: 82 us with one wave per cell, now 12).  The second
+// pass applies the exact FP64 test.
+constexpr int BPW_WAVES = 2, BPW_OWN = 16, BPW_BUF = 128, BPW_LIST = 128;
+struct BpWave {
+    BpTet own[BPW_OWN];
+    int4 node[64];                      // of the candidates
+    unsigned long long buf[BPW_BUF];
+    unsigned short list[BPW_LIST];      // own << 6 | candidate
+};
 // The candidate buffer is split into BP_PARTS regions of cap / BP_PARTS entries, each with its
 // own counter (BP_PART_STRIDE counters apart, so that no two share a cache line): workgroup w
 // appends to region w mod BP_PARTS, which spreads the reservations over as many addresses.
@@ -248,17 +430,16 @@ __device__ inline long long bp_slot(long long cap, const unsigned long long *__r
     return o < (n < capP ? n : capP) ? (long long)blockIdx.y * capP + o : -1;
 }
 
-// One wave's cell of the pair search (k_bp_cellwave): on return, cnt pairs are left in buf.
-__device__ inline void bp_cell_pairs(const float4 *__restrict__ sk32, const int4 *__restrict__ snode,
-                                     int exclude_shared, const BpGrid &g, const int *__restrict__ first,
-                                     unsigned long long *__restrict__ total, unsigned long long *__restrict__ out,
-                                     long long cap, int i, float4 (*ow)[7], unsigned long long *buf, int lane,
+// One wave's cell and slice of the pair search (k_bp_cellwave): on return, cnt pairs are left in buf.
+__device__ inline void bp_cell_pairs(const BpTet *__restrict__ srec, int exclude_shared, const BpGrid &g,
+                                     const int *__restrict__ first, unsigned long long *__restrict__ total, unsigned long long *__restrict__ out,
+                                     long long cap, int i, int slice, int slices, int chunk, BpWave &W, int lane,
                                      unsigned long long below, int &cnt)
 {
     const int x = i % g.n[0] + 1, y = (i / g.n[0]) % g.n[1] + 1, z = i / (g.n[0] * g.n[1]) + 1;
     const int L = x + g.gx * (y + g.gy * z);
     const int s0 = first[L], s1 = first[L + 1];
-    if (s0 == s1) return;
+    if (s0 + slice * chunk >= s1) return;
     const int gxy = g.gx * g.gy;
     const int r_lo[5] = {s0, first[L - 1 + g.gx], first[L - 1 - g.gx + gxy], first[L - 1 + gxy],
                          first[L - 1 + g.gx + gxy]};
@@ -275,21 +456,14 @@ __device__ inline void bp_cell_pairs(const float4 *__restrict__ sk32, const int4
         if (lane == 0) base = atomicAdd(total, (unsigned long long)cnt);
         base = __shfl(base, 0);
         for (int q = lane; q < cnt; q += 64)
-            if (base + q < (unsigned long long)cap) out[base + q] = buf[q];
+            if (base + q < (unsigned long long)cap) out[base + q] = W.buf[q];
         bp_wave_sync();
         cnt = 0;
     };
-    for (int a0 = s0; a0 < s1; a0 += BPW_OWN) {
-        const int na = min(BPW_OWN, s1 - a0);
+    for (int a0 = s0 + slice * chunk; a0 < s1; a0 += slices * chunk) {
+        const int na = min(chunk, s1 - a0);
         bp_wave_sync();   // the previous own tets are no longer read
-        if (lane < na) {
-#pragma unroll
-            for (int q = 0; q < 6; q++) ow[lane][q] = sk32[(size_t)(a0 + lane) * 6 + q];
-            const int4 n4 = snode[a0 + lane];
-            ow[lane][6] = make_float4(__int_as_float(n4.x), __int_as_float(n4.y), __int_as_float(n4.z),
-                                      __int_as_float(n4.w));
-        }
-        bp_wave_sync();
+        if (lane < na) W.own[lane] = srec[a0 + lane];
         for (int k0 = 0; k0 < K; k0 += 64) {
             const int k = k0 + lane;
             const bool valid = k < K;
@@ -300,80 +474,77 @@ __device__ inline void bp_cell_pairs(const float4 *__restrict__ sk32, const int4
                     jb = r_lo[r] + (k - r_pre[r]);
                     own_row = r == 0;
                 }
-            float c[2 * BP_DIRS];
-#pragma unroll
-            for (int q = 0; q < 6; q++) {
-                const float4 v = sk32[(size_t)jb * 6 + q];
-                c[4 * q] = v.x;
-                c[4 * q + 1] = v.y;
-                c[4 * q + 2] = v.z;
-                c[4 * q + 3] = v.w;
-            }
-            const int4 cn = snode[jb];
-            for (int ia = 0; ia < na; ia++) {
-                const int ja = a0 + ia;
-                float a[2 * BP_DIRS];
-#pragma unroll
-                for (int q = 0; q < 6; q++) {
-                    const float4 v = ow[ia][q];
-                    a[4 * q] = v.x;
-                    a[4 * q + 1] = v.y;
-                    a[4 * q + 2] = v.z;
-                    a[4 * q + 3] = v.w;
-                }
-                const float4 an4 = ow[ia][6];
-                // the wave's mask of passing lanes, one ballot per comparison (each a compare
-                // into a mask and a scalar AND)
-                unsigned long long mk = __ballot(valid & (!own_row | (jb > ja)));
-#pragma unroll
-                for (int d = 0; d < BP_DIRS; d++) {
-                    mk &= ~__ballot(a[d] > c[BP_DIRS + d]);
-                    mk &= ~__ballot(a[BP_DIRS + d] < c[d]);
-                }
+            // what comes after the positions of the candidate is larger than every own tet's but the
+            // first range's
+            const int after = own_row ? jb : INT_MAX;
+            const BpTet c = srec[jb];
+            W.node[lane] = c.node;
+            bp_wave_sync();
+            int nlist = 0;
+            auto take = [&](int m) {      // the list's first m <= 64 pairs
+                bp_wave_sync();
+                const unsigned e = W.list[lane < m ? lane : 0];
+                const int ia = (int)(e >> 6), l = (int)(e & 63);
+                const int pb = __shfl(jb, l);
+                bool hit = lane < m;
                 if (exclude_shared) {
-                    const int an[4] = {__float_as_int(an4.x), __float_as_int(an4.y), __float_as_int(an4.z),
-                                       __float_as_int(an4.w)};
-                    const int m[4] = {cn.x, cn.y, cn.z, cn.w};
+                    const int4 p = W.own[ia].node, q = W.node[l];
+                    const int an[4] = {p.x, p.y, p.z, p.w}, bn[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
                     for (int j2 = 0; j2 < 4; j2++)
 #pragma unroll
-                        for (int j1 = 0; j1 < 4; j1++) mk &= ~__ballot(m[j2] == an[j1]);
+                        for (int j1 = 0; j1 < 4; j1++) hit &= bn[j2] != an[j1];
                 }
-                if (mk == 0) continue;
-                const bool hit = (mk >> lane) & 1;
-                if (hit) buf[cnt + __popcll(mk & below)] = ((unsigned long long)ja << 32) | (unsigned)jb;
+                const unsigned long long mk = __ballot(hit);
+                if (hit) W.buf[cnt + __popcll(mk & below)] = ((unsigned long long)(a0 + ia) << 32) | (unsigned)pb;
                 cnt += __popcll(mk);
+                // the rest of the list to its front
+                const unsigned short rest = W.list[min(m + lane, BPW_LIST - 1)];
+                bp_wave_sync();
+                nlist -= m;
+                if (lane < nlist) W.list[lane] = rest;
                 if (cnt > BPW_BUF - 64) flush();
+            };
+            for (int ia = 0; ia < na; ia++) {
+                const bool near = valid & (after > a0 + ia) & (bp_apart(W.own[ia], c) == 0);
+                const unsigned long long mk = __ballot(near);
+                if (mk == 0) continue;
+                if (near) W.list[nlist + __popcll(mk & below)] = (unsigned short)(ia << 6 | lane);
+                nlist += __popcll(mk);
+                if (nlist >= 64) take(64);
             }
+            if (nlist) take(nlist);
+            bp_wave_sync();   // the candidates are no longer read
         }
     }
 }
 
-// At most 80 registers, for 6 waves per SIMD (88 otherwise: 5 waves; a 12-byte spill; forcing
-// 8 waves spills 100 bytes and doubles the time).
-__global__ __launch_bounds__(64 * BPW_WAVES) __attribute__((amdgpu_waves_per_eu(6))) void k_bp_cellwave(const float4 *__restrict__ sk32,
-                                                                const int4 *__restrict__ snode, int exclude_shared,
-                                                                BpGrid g, const int *__restrict__ first,
+__global__ __launch_bounds__(64 * BPW_WAVES) void k_bp_cellwave(const BpTet *__restrict__ srec,
+                                                                int exclude_shared,
+                                                                const BpGrid *__restrict__ grid, int slices, int chunk,
+                                                                const int *__restrict__ first,
                                                                 unsigned long long *__restrict__ total,
                                                                 unsigned long long *__restrict__ out, long long cap)
 {
-    __shared__ float4 own[BPW_WAVES][BPW_OWN][7];
-    __shared__ unsigned long long pbuf[BPW_WAVES][BPW_BUF];
+    __shared__ BpWave waves[BPW_WAVES];
     __shared__ int wcnt[BPW_WAVES], done;
+    if (!grid->ok) return;
+    const BpGrid g = *grid;
     const int wave = threadIdx.x >> 6, lane = __lane_id();
     if (threadIdx.x == 0) done = 0;
     __syncthreads();
     const unsigned long long below = (1ULL << lane) - 1;
-    unsigned long long *buf = pbuf[wave];
     int cnt = 0;
-    const int ncell = g.n[0] * g.n[1] * g.n[2];
-    const int i = (int)blockIdx.x * BPW_WAVES + wave;
+    // the slices of a cell are neighbouring waves; runs of 64 workgroups stay on one XCD, whose L2 then
+    // holds the tets of neighbouring cells
+    const int run = (int)blockIdx.x / 512 * 512, in = (int)blockIdx.x - run;
+    const int w = (run + in % 8 * 64 + in / 8) * BPW_WAVES + wave, i = w / slices;
     const long long capP = cap / BP_PARTS;
     const int part = (int)(blockIdx.x % BP_PARTS);
     total += (size_t)part * BP_PART_STRIDE;
     out += (size_t)part * capP;
-    if (i < ncell) bp_cell_pairs(sk32, snode, exclude_shared, g, first, total, out, capP, i, own[wave], buf, lane,
-                                 below, cnt);
+    if (i < g.ncell) bp_cell_pairs(srec, exclude_shared, g, first, total, out, capP, i, w % slices, slices, chunk, waves[wave],
+                                   lane, below, cnt);
     // the workgroup's last wave out writes every wave's remaining pairs
     if (lane == 0) wcnt[wave] = cnt;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
@@ -384,15 +555,15 @@ __global__ __launch_bounds__(64 * BPW_WAVES) __attribute__((amdgpu_waves_per_eu(
     int pre[BPW_WAVES + 1];
     pre[0] = 0;
 #pragma unroll
-    for (int w = 0; w < BPW_WAVES; w++) pre[w + 1] = pre[w] + wcnt[w];
+    for (int v = 0; v < BPW_WAVES; v++) pre[v + 1] = pre[v] + wcnt[v];
     if (pre[BPW_WAVES] == 0) return;
     unsigned long long base = 0;
     if (lane == 0) base = atomicAdd(total, (unsigned long long)pre[BPW_WAVES]);
     base = __shfl(base, 0);
 #pragma unroll
-    for (int w = 0; w < BPW_WAVES; w++)
-        for (int q = lane; q < wcnt[w]; q += 64)
-            if (base + pre[w] + q < (unsigned long long)capP) out[base + pre[w] + q] = pbuf[w][q];
+    for (int v = 0; v < BPW_WAVES; v++)
+        for (int q = lane; q < wcnt[v]; q += 64)
+            if (base + pre[v] + q < (unsigned long long)capP) out[base + pre[v] + q] = waves[v].buf[q];
 }
 
 // The pair search, second pass: per candidate (own, candidate) position pair of the first
@@ -453,8 +624,14 @@ __global__ __launch_bounds__(256) void k_bp_scatter(const unsigned long long *__
                                                     const int *__restrict__ rank,
                                                     const unsigned long long *__restrict__ ncand, long long cap,
                                                     const int *__restrict__ start,
-                                                    unsigned long long *__restrict__ grp)
+                                                    unsigned long long *__restrict__ grp, Report rep)
 {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+        // the fullest region decides whether the buffer held every candidate
+        unsigned long long most = 0;
+        for (int q = 0; q < BP_PARTS; q++) most = max(most, ncand[(size_t)q * BP_PART_STRIDE]);
+        rep.put(BP_CAND, (unsigned)min(most, 0xffffffffULL));
+    }
     const long long i = bp_slot(cap, ncand);
     if (i < 0) return;
     const int r = rank[i];
@@ -467,11 +644,13 @@ __global__ __launch_bounds__(256) void k_bp_scatter(const unsigned long long *__
 // smaller than its own (the b's of a group are distinct), so the pairs come out in (a, b)
 // order; those below max_pairs are written.
 __global__ __launch_bounds__(256) void k_bp_place(const unsigned long long *__restrict__ grp,
-                                                  const int *__restrict__ start, int nT, long long max_pairs,
+                                                  const int *__restrict__ start, int nT,
+                                                  const BpGrid *__restrict__ grid, long long max_pairs,
                                                   int *__restrict__ pairs)
 {
+    if (!grid->ok) return;
     const long long p = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (long long)start[nT]) return;
+    if (p >= (long long)start[nT]) return;   // at most the places of the buffer
     const unsigned long long v = grp[p];
     const int a = (int)(v >> 32), b = (int)(v & 0xffffffffULL);
     const int s = start[a], e = start[a + 1];

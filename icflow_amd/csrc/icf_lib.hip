@@ -240,6 +240,7 @@ struct icf_ctx {
     DevBuf bp_c;                     // broad phase grid (cell counts, first sorted position per cell key)
     DevBuf bp_g;                     // broad phase pair grouping (counts and starts per tet, ranks)
     long long nl2_last = 0;          // distinct tuples of the last NL2set call
+    long long bp_cells = 0, bp_inner = 0;   // cells of the last search's grid, with and without margin
     long long bp_cap = 0;            // pair keys the broad phase's buffer holds (grows with use)
     DevBuf map_cnt, map_rank, map_sums;   // building slot maps: counts (zero in between), ranks, tile sums
     DevBuf tsum;                     // per-node tet sums of the fused call
@@ -2563,117 +2564,99 @@ int icf_broad_phase(icf_ctx *ctx, const double *dn, int nd_stride, const int *ie
     if (nTets == 0) return 0;
     const int nT = nTets;
     if (nT > (1 << 23)) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: more than 2^23 surface tets");
-    // scratch: lo, hi (12 nT each), bounds (7), cell-ordered k-DOPs in FP64 (24 nT) and FP32
-    // (12 nT doubles' worth)
-    if (int r = grow(ctx, ctx->bp_f, sizeof(double) * ((size_t)60 * nT + 8))) return r;
-    if (int r = grow(ctx, ctx->bp_i, sizeof(int) * (8 * (size_t)nT + 4))) return r;
-    if (int r = grow(ctx, ctx->bp_l, sizeof(long long) * BP_PARTS * BP_PART_STRIDE)) return r;
-    double *lo = (double *)ctx->bp_f.p, *hi = lo + (size_t)12 * nT;
-    auto *bounds = (unsigned long long *)(hi + (size_t)12 * nT);
-    double2 *skd = (double2 *)(hi + (size_t)12 * nT + 8);          // 12 double2 = 24 doubles per tet
-    float4 *sk32 = (float4 *)(hi + (size_t)36 * nT + 8);           // 6 float4 = 12 doubles per tet
+    // scratch: in cell order the records (8 nT doubles' worth), k-DOPs in FP64 (24 nT) and FP32 (12 nT); minimum
+    // corners (3 nT), bounds, grid
+    const int nb = std::min<int>(blocks_for(nT, 256), BP_BLOCKS);
+    const size_t nbounds = (size_t)BP_BLOCKS * BP_NBOUNDS, ngrid = (sizeof(BpGrid) + 7) / 8;
+    if (int r = grow(ctx, ctx->bp_f, sizeof(double) * ((size_t)47 * nT + nbounds + ngrid))) return r;
+    if (int r = grow(ctx, ctx->bp_i, sizeof(int) * 3 * (size_t)nT)) return r;
+    BpTet *srec = (BpTet *)ctx->bp_f.p;
+    double2 *skd = (double2 *)(srec + nT);                         // 12 double2 = 24 doubles per tet
+    float4 *sk32 = (float4 *)(skd + (size_t)BP_DIRS * nT);         // 6 float4 = 12 doubles per tet
+    double *lo = (double *)ctx->bp_f.p + (size_t)44 * nT, *bounds = lo + (size_t)3 * nT;
+    BpGrid *grid = (BpGrid *)(bounds + nbounds);
     auto *key = (unsigned *)ctx->bp_i.p;
     int *rank = (int *)(key + nT), *sidx = rank + nT;
-    int4 *snode = (int4 *)(sidx + nT + ((4 - ((3 * nT) & 3)) & 3));   // 4 nT ints, 16-byte aligned
-    hipLaunchKernelGGL(k_bp_bounds_init, dim3(1), dim3(64), 0, ctx->stream, bounds);
-    hipLaunchKernelGGL(k_bp_kdop, dim3(blocks_for(nT, 256)), dim3(256), 0, ctx->stream, dn, nd_stride, ie,
-                       el_all_stride, nT, lo, bounds, nd_stride);
-    unsigned long long hb[BP_NBOUNDS + 1];
-    HIPCHK(ctx, hipGetLastError());
-    HIPCHK(ctx, hipMemcpyAsync(hb, bounds, sizeof(hb), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-    if (hb[BP_NBOUNDS]) return fail(ctx, ICF_E_INDEX, "icf_broad_phase: bad node id");
-    // the grid: cells at least the largest extent, coarsened (any size >= the extents finds
-    // the same pairs) until the margin grid has at most 2^24 cells
-    BpGrid g;
-    const double ext = bp_unord(hb[0]);
-    double span[3];
-    for (int k = 0; k < 3; k++) {
-        g.org[k] = bp_unord(hb[1 + k]);
-        span[k] = bp_unord(hb[4 + k]) - g.org[k];
-        if (!std::isfinite(g.org[k]) || !std::isfinite(span[k]))
-            return fail(ctx, ICF_E_INVALID, "icf_broad_phase: non-finite node positions");
-    }
-    g.cs = ext > 0 ? ext * 1.000001 : 1.0;
-    for (;;) {
-        double cells = 1;
-        for (int k = 0; k < 3; k++) {
-            const double c = std::floor(span[k] / g.cs) + 1;
-            g.n[k] = c < (double)(1 << 24) ? (int)c : (1 << 24);
-            cells *= (double)g.n[k] + (k == 0 ? 3 : 2);
-        }
-        if (cells <= (double)(1 << 24)) break;
-        g.cs *= 1.25;
-    }
-    g.gx = g.n[0] + 3;
-    g.gy = g.n[1] + 2;
-    g.gz = g.n[2] + 2;
-    const int G = g.gx * g.gy * g.gz;
-    // cell counts, their exclusive scan (first), and the tets' cell-ordered copies
-    if (int r = grow(ctx, ctx->bp_c, sizeof(int) * 2 * ((size_t)G + 1))) return r;
-    int *count = (int *)ctx->bp_c.p, *first = count + G + 1;
-    size_t b3 = 0;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, b3, count, first, G + 1, ctx->stream));
-    if (int r = grow(ctx, ctx->scan_tmp, b3)) return r;
-    hipLaunchKernelGGL(k_fill_int, dim3(blocks_for((long long)G + 1, 256)), dim3(256), 0, ctx->stream, count, G + 1,
-                       0);
-    hipLaunchKernelGGL(k_bp_cell, dim3(blocks_for(nT, 256)), dim3(256), 0, ctx->stream, lo, nT, g, key, rank, count);
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, b3, count, first, G + 1, ctx->stream));
-    hipLaunchKernelGGL(k_bp_sorted, dim3(blocks_for(nT, 256)), dim3(256), 0, ctx->stream, dn, nd_stride, nd_stride,
-                       nT, key, rank,
-                       first, ie, el_all_stride, sidx, skd, snode, sk32);
-    // candidate pairs per cell (FP32 prefilter), collected in LDS and appended in batches; the
-    // exact test; the passing pairs grouped by a (a counting sort) and placed by their rank of b
-    // within the group: the pairs in (a, b) order.  The launches after the search take the
-    // candidate count from device memory (their grids cover the buffer), so one read-back at
-    // the end serves all; a second round only when the candidates outgrew the buffer.
-    const int ncell = g.n[0] * g.n[1] * g.n[2];
-    auto *tot = (unsigned long long *)ctx->bp_l.p;
+    // Every launch takes the grid from device memory and what it counts from there too, so one wait at
+    // the end serves all (with two, library scans, copies of the counts and the slower search a call took
+    // 219 us on 3,300 tets and 546 on 353,000, now 75 and 345); the launches and buffers are as large as the last search's grid and candidates ask
+    // for, and a search whose do not fit is repeated with what it found.
+    const long long cells = ctx->bp_cells ? ctx->bp_cells : 8192, inner = ctx->bp_inner ? ctx->bp_inner : 4096;
+    long long capG = cells + cells / 4 + 64, capC = inner + inner / 4 + 64;
     // at least 64 places per region, so that every region's grid row has a workgroup
     long long cap = std::max<long long>({ctx->bp_cap, 4LL * nT, 64LL * BP_PARTS});
-    size_t b5 = 0;
-    HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(nullptr, b5, (int *)nullptr, (int *)nullptr, nT + 1, ctx->stream));
-    if (int r = grow(ctx, ctx->scan_tmp, b5)) return r;
+    const unsigned atiles = blocks_for(nT, BP_TILE);
     long long ncand = 0;
-    int nv = 0;
-    for (int pass = 0; pass < 2; pass++) {
+    bool grown = false;
+    for (;;) {
         if (cap >= (1LL << 31)) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: more than 2^31 candidate pairs");
+        const unsigned ctiles = blocks_for(capG, BP_TILE);
+        const size_t ntotal = (size_t)BP_PARTS * BP_PART_STRIDE, nct = ctiles + Tiles::group_words(ctiles);
+        const size_t nw = nct + atiles + Tiles::group_words(atiles);
+        if (int r = grow(ctx, ctx->bp_l, sizeof(long long) * ntotal + sizeof(unsigned) * nw)) return r;
+        if (int r = grow(ctx, ctx->bp_c, sizeof(int) * 2 * ((size_t)capG + 1))) return r;
         if (int r = grow(ctx, ctx->pat_a, sizeof(unsigned long long) * (size_t)cap)) return r;
         if (int r = grow(ctx, ctx->pat_b, sizeof(unsigned long long) * (size_t)cap)) return r;
         if (int r = grow(ctx, ctx->bp_g, sizeof(int) * (2 * ((size_t)nT + 1) + (size_t)cap))) return r;
+        auto *tot = (unsigned long long *)ctx->bp_l.p;
+        auto *w = (unsigned *)(tot + ntotal);
+        const Tiles ct{w, w + ctiles}, at{w + nct, w + nct + atiles};
+        int *count = (int *)ctx->bp_c.p, *first = count + capG + 1;   // per cell, and their exclusive scan
         int *acount = (int *)ctx->bp_g.p, *start = acount + nT + 1, *rnk = start + nT + 1;
         auto *pa = (unsigned long long *)ctx->pat_a.p, *grp = (unsigned long long *)ctx->pat_b.p;
-        hipLaunchKernelGGL(k_fill_int, dim3(blocks_for(2 * BP_PARTS * BP_PART_STRIDE, 256)), dim3(256), 0,
-                           ctx->stream, (int *)tot, 2 * BP_PARTS * BP_PART_STRIDE, 0);
-        hipLaunchKernelGGL(k_fill_int, dim3(blocks_for((long long)nT + 1, 256)), dim3(256), 0, ctx->stream, acount,
-                           nT + 1, 0);
-        hipLaunchKernelGGL(k_bp_cellwave, dim3((ncell + BPW_WAVES - 1) / BPW_WAVES), dim3(64 * BPW_WAVES), 0,
-                           ctx->stream, sk32, snode, exclude_shared, g, first, tot, pa, cap);
+        const Report rep = new_report(ctx);
+        const dim3 b(256), tets(blocks_for(nT, 256));
+        hipLaunchKernelGGL(k_bp_clear, dim3(blocks_for(std::max<long long>({capG + 1, nT + 1LL, (long long)ntotal}), 256)),
+                           b, 0, ctx->stream, count, (int)(capG + 1), acount, nT + 1, tot, (int)ntotal, ct, ctiles, at,
+                           atiles);
+        hipLaunchKernelGGL(k_bp_kdop, dim3(nb), b, 0, ctx->stream, dn, nd_stride, ie, el_all_stride, nT, lo, bounds, rep);
+        hipLaunchKernelGGL(k_bp_cell, tets, b, 0, ctx->stream, lo, nT, bounds, nb, (int)capG, (int)capC, grid, key, rank,
+                           count, rep);
+        hipLaunchKernelGGL(k_bp_tiles, dim3(ctiles), b, 0, ctx->stream, count, -1, grid, ct);
+        hipLaunchKernelGGL(k_bp_scan, dim3(ctiles), b, 0, ctx->stream, count, -1, grid, ct, first, -1, rep);
+        hipLaunchKernelGGL(k_bp_sorted, tets, b, 0, ctx->stream, dn, nd_stride, nT, key, rank, first, ie, el_all_stride,
+                           grid, sidx, srec, skd, sk32);
+        // candidate pairs per cell (FP32 prefilter), collected in LDS and appended in batches; the
+        // exact test; the passing pairs grouped by a (a counting sort) and placed by their rank of b
+        // within the group: the pairs in (a, b) order.  The launches after the search take the
+        // candidate count from device memory (their grids cover the buffer).  Below 16,384 cells several
+        // waves share one.
+        const int slices = (int)std::min<long long>(16, std::max(1LL, 20480 / capC));
+        hipLaunchKernelGGL(k_bp_cellwave, dim3(blocks_for(capC * slices, 512 * BPW_WAVES) * 512), dim3(64 * BPW_WAVES), 0,
+                           ctx->stream, srec, exclude_shared, grid, slices, slices > 1 ? 4 : BPW_OWN, first, tot,
+                           pa, cap);
         const dim3 gparts(blocks_for(cap / BP_PARTS, 256), BP_PARTS);   // a grid row per region
-        hipLaunchKernelGGL(k_bp_exact, gparts, dim3(256), 0, ctx->stream, skd, sk32, sidx, tot,
-                           cap, pa, rnk, acount);
-        HIPCHK(ctx, hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, b5, acount, start, nT + 1, ctx->stream));
-        hipLaunchKernelGGL(k_bp_scatter, gparts, dim3(256), 0, ctx->stream, pa, rnk, tot, cap,
-                           start, grp);
+        hipLaunchKernelGGL(k_bp_exact, gparts, b, 0, ctx->stream, skd, sk32, sidx, tot, cap, pa, rnk, acount);
+        hipLaunchKernelGGL(k_bp_tiles, dim3(atiles), b, 0, ctx->stream, acount, nT, grid, at);
+        hipLaunchKernelGGL(k_bp_scan, dim3(atiles), b, 0, ctx->stream, acount, nT, grid, at, start, BP_NV, rep);
+        hipLaunchKernelGGL(k_bp_scatter, gparts, b, 0, ctx->stream, pa, rnk, tot, cap, start, grp, rep);
         if (max_pairs > 0)
-            hipLaunchKernelGGL(k_bp_place, dim3(blocks_for(cap, 256)), dim3(256), 0, ctx->stream, grp, start, nT,
-                               max_pairs, pairs);
-        std::vector<unsigned long long> got((size_t)BP_PARTS * BP_PART_STRIDE);
+            hipLaunchKernelGGL(k_bp_place, dim3(blocks_for(cap, 256)), b, 0, ctx->stream, grp, start, nT, grid, max_pairs,
+                               pairs);
         HIPCHK(ctx, hipGetLastError());
-        HIPCHK(ctx, hipMemcpyAsync(got.data(), tot, sizeof(unsigned long long) * got.size(), hipMemcpyDeviceToHost,
-                                   ctx->stream));
-        HIPCHK(ctx, hipMemcpyAsync(&nv, start + nT, sizeof(nv), hipMemcpyDeviceToHost, ctx->stream));
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
-        // the fullest region decides whether the buffer held every candidate
-        ncand = 0;
-        for (int q = 0; q < BP_PARTS; q++) ncand = std::max(ncand, (long long)got[(size_t)q * BP_PART_STRIDE]);
-        if (ncand <= cap / BP_PARTS) break;
-        if (pass == 1) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: pair count changed between two searches");
+        const volatile unsigned *got = rep.host;
+        if (reported(rep, BP_BAD)) return fail(ctx, ICF_E_INDEX, "icf_broad_phase: bad node id");
+        if (reported(rep, BP_NONFINITE))
+            return fail(ctx, ICF_E_INVALID, "icf_broad_phase: non-finite node positions");
+        ctx->bp_cells = got[BP_G];
+        ctx->bp_inner = got[BP_NCELL];
+        if (reported(rep, BP_BIG)) {
+            capG = std::max(capG, ctx->bp_cells + ctx->bp_cells / 4);
+            capC = std::max(capC, ctx->bp_inner + ctx->bp_inner / 4);
+            continue;
+        }
+        ncand = got[BP_CAND];
+        if (ncand <= cap / BP_PARTS) {
+            *nOut = got[BP_NV];
+            break;
+        }
+        if (grown) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: pair count changed between two searches");
+        grown = true;
         cap = BP_PARTS * (ncand + ncand / 4);
     }
     ctx->bp_cap = std::max(ctx->bp_cap, BP_PARTS * (ncand + ncand / 4));
-    *nOut = (long long)nv;
-    if ((long long)nv > max_pairs) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: more pairs than max_pairs");
+    if (*nOut > max_pairs) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: more pairs than max_pairs");
     return 0;
 }
 
