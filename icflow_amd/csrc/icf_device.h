@@ -119,6 +119,8 @@ __device__ inline T dot3(const T *a, const T *b) { return a[0] * b[0] + a[1] * b
 // the call's sequence number; the device copy of the words keeps all but the first few threads
 // that set one off the bus.
 constexpr int REPORT_WORDS = 32;
+constexpr int CZ_DAMAGED = 23, CZ_FAILED = 24;      // values: the CZ counts of an assembly
+constexpr int REPORT_SPECS = 1024;                  // behind the words, two counts of as many specimens
 struct Report {
     unsigned *dev, *host;
     unsigned seq;

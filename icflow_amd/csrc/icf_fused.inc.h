@@ -48,7 +48,7 @@ __device__ inline bool split2(int w, int na, int nb, bool ilv, int &local)
 }
 
 // Phase 1 of the fused call: tets (nbt workgroups) interleaved with CZs (nbc).  Workgroup 0 also
-// clears the two CZ counters that the last launch of the call adds up.
+// clears the two CZ counters that the last launch of the call adds up, and their ticket.
 template <bool MIXED, bool ISO, bool NT>
 __global__ __launch_bounds__(256) void k_phase1_fused(int nbt, int nbc, const int *__restrict__ ie,
                                                       const double *__restrict__ dn, int nt, int tp, int es, int ns,
@@ -57,7 +57,7 @@ __global__ __launch_bounds__(256) void k_phase1_fused(int nbt, int nbc, const in
                                                       double *__restrict__ cz_rhs, void *__restrict__ cz_tan,
                                                       int *__restrict__ counts)
 {
-    if (blockIdx.x == 0 && threadIdx.x < 2) counts[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 4 && threadIdx.x != 2) counts[threadIdx.x] = 0;
     int local;
     if (!interleave2(blockIdx.x, nbt, nbc, local))
         tet_phase1<MIXED, ISO, NT>(local, nbt, ie, dn, nt, tp, es, ns, tet_rhs, tet_tan);
@@ -98,15 +98,15 @@ __global__ __launch_bounds__(KEYS) void k_vals_force_rhs_fused(int nbf, int nbc,
         double *__restrict__ F, int ns, const int *__restrict__ node_row, const int *__restrict__ roff,
         const uint32_t *__restrict__ rcodes, const int *__restrict__ cz_begin, double *__restrict__ b,
         const int *__restrict__ damaged, const int *__restrict__ failed, int nc, int *__restrict__ counts,
-        const int *__restrict__ cz_off, int nspec, int *__restrict__ spec_counts, Stage sv, int ilv)
+        const int *__restrict__ cz_off, int nspec, int *__restrict__ spec_counts, Stage sv, int ilv, Report rep)
 {
     constexpr int BYTES = vals_lds<L, KEYS, STAGE>();
     __shared__ __align__(16) char lds[BYTES];
     const int w = blockIdx.x;
     int local;
     if (w < nbc) {
-        if (cz_off) count_flags_spec<KEYS>(w, nbc, damaged, failed, cz_off, nspec, spec_counts, counts);
-        else count_flags_n<KEYS>(w, nbc, damaged, failed, nc, counts);
+        if (cz_off) count_flags_spec<KEYS>(w, nbc, damaged, failed, cz_off, nspec, spec_counts, counts, rep);
+        else count_flags_n<KEYS>(w, nbc, damaged, failed, nc, counts, rep);
     }
     else if (!split2(w - nbc, nbf, nchunks, ilv != 0, local))
         reduce_force_rhs<KEYS, vals_stage<L, KEYS, STAGE>()>(local, nbf, foff, fcodes, fkeys, nfkeys, F, ns, node_row, roff, rcodes, cz_begin,

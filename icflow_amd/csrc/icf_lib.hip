@@ -802,7 +802,7 @@ struct Timer {
             return 0;
         }
         HIPCHK(ctx, hipEventRecord(ctx->ev1, ctx->stream));
-        HIPCHK(ctx, hipEventSynchronize(ctx->ev1));
+        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         float ms = 0;
         HIPCHK(ctx, hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
         ctx->last_ms = ms;
@@ -1155,10 +1155,11 @@ bool vals_force_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const SlotMap 
 
 // The second half of the fused call as one launch: node forces with the rhs rows, the CZ
 // counters and the BCSR values (overwrite).  False unless the rhs map's rows each have their
-// tet node (merge_ok) and the value map is an overwrite map.
+// tet node (merge_ok) and the value map is an overwrite map.  The counters go to `rep` too unless its
+// host words are null.
 bool vals_force_rhs_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const SlotMap *mf, double *F, int ns,
                           const SlotMap *mr, double *b, const int *dmg, const int *fld, int nCZs, int *counts,
-                          const Stage &st)
+                          const Stage &st, const Report &rep)
 {
     if (mv->keys || !mr->merge_ok || !mr->node_row) return false;
     if (mv->nlaunch == 0 && mf->nlaunch == 0 && nCZs == 0) return true;
@@ -1179,7 +1180,7 @@ bool vals_force_rhs_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const Slot
 #define ICF_VFR(MX, IS, L, NAME)                                                                                   \
     LAUNCH(ctx, NAME, (k_vals_force_rhs_fused<MX, IS, L, K, S>), g, bl, nbf, nbc, mv->loff, mv->codes, mv->nlaunch, \
            nch, A, mf->loff, mf->codes, mf->keys, mf->nlaunch, F, ns, mr->node_row, mr->off, mr->codes, mr->cz_begin, \
-           b, dmg, fld, nCZs, counts, per_spec ? bt.cz_off : nullptr, bt.n, bt.spec_counts, st, ilv)
+           b, dmg, fld, nCZs, counts, per_spec ? bt.cz_off : nullptr, bt.n, bt.spec_counts, st, ilv, rep)
         if (mixed && iso) ICF_VFR(true, true, float, "k_vals_force_rhs<mixed,iso>");
         else if (mixed) ICF_VFR(true, false, float, "k_vals_force_rhs<mixed,gen>");
         else if (iso) ICF_VFR(false, true, double, "k_vals_force_rhs<fp64,iso>");
@@ -1332,10 +1333,11 @@ int icf_create(int device, icf_ctx **out)
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev0);
     if (e == hipSuccess) e = hipEventCreate(&ctx->ev1);
     if (e == hipSuccess) e = hipMalloc(&ctx->small, 16 * sizeof(int));
+    const size_t rep_bytes = (REPORT_WORDS + 2 * REPORT_SPECS) * sizeof(unsigned);
     if (e == hipSuccess) e = hipMalloc(&ctx->rep_dev, REPORT_WORDS * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(ctx->rep_dev, 0, REPORT_WORDS * sizeof(unsigned));
-    if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->rep_host, REPORT_WORDS * sizeof(unsigned), hipHostMallocMapped);
-    if (e == hipSuccess) memset(ctx->rep_host, 0, REPORT_WORDS * sizeof(unsigned));
+    if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->rep_host, rep_bytes, hipHostMallocMapped);
+    if (e == hipSuccess) memset(ctx->rep_host, 0, rep_bytes);
     if (e == hipSuccess) e = scratch_for_device(device, (void **)&ctx->noalloc);
     if (e != hipSuccess) {
         delete ctx;
@@ -2190,7 +2192,12 @@ static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride,
     }
     Stage st = make_stage(ctx, h);
     double *F = dn + (size_t)nd_stride * ND_F;
-    if (tsum && fuse && vals_force_rhs_fused(ctx, mv, A, mf, F, nd_stride, mr, b, dmg, fld, nCZs, counts, st)) {
+    // a blocking call's counters come back with its wait
+    const bool tell = (nCZDamaged || nCZFailed || ctx->batch.spec_counts) && ctx->blocking && !ctx->capturing;
+    const Report rep = tell ? new_report(ctx) : Report{};
+    bool told = false;
+    if (tsum && fuse && vals_force_rhs_fused(ctx, mv, A, mf, F, nd_stride, mr, b, dmg, fld, nCZs, counts, st, rep)) {
+        told = tell && nCZs > 0;
         // done: node forces with the rhs rows, the counts and the BCSR values in one launch
     } else if (tsum) {
         // BCSR values and node forces (keeping each node's tet sum), then the rhs rows from
@@ -2221,8 +2228,13 @@ static int assemble_impl(icf_ctx *ctx, const int *ie, int nElems, int el_stride,
     if (int r = tm.finish()) return r;
     if ((nCZDamaged || nCZFailed) && ctx->blocking && !ctx->capturing) {
         int sums[2] = {0, 0};
-        HIPCHK(ctx, hipMemcpyAsync(sums, ctx->small + 2, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        if (told) {
+            sums[0] = (int)((volatile unsigned *)rep.host)[CZ_DAMAGED];
+            sums[1] = (int)((volatile unsigned *)rep.host)[CZ_FAILED];
+        } else if (nCZs) {
+            HIPCHK(ctx, hipMemcpyAsync(sums, ctx->small + 2, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        }
         if (nCZDamaged) *nCZDamaged = sums[0];
         if (nCZFailed) *nCZFailed = sums[1];
     }
@@ -2323,8 +2335,12 @@ int icf_assemble_batched(icf_ctx *ctx, const icf_worklist *wl, const int *ie, in
     if (int r = ln.done()) return r;
     if ((nCZDamaged || nCZFailed) && ctx->blocking && !ctx->capturing) {
         std::vector<int> c(2 * (size_t)n);
-        HIPCHK(ctx, hipMemcpyAsync(c.data(), cnt, sizeof(int) * c.size(), hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        if (nC && B.spec_counted && n <= REPORT_SPECS) {
+            for (size_t k = 0; k < c.size(); k++) c[k] = (int)((volatile unsigned *)ctx->rep_host)[REPORT_WORDS + k];
+        } else {
+            HIPCHK(ctx, hipMemcpyAsync(c.data(), cnt, sizeof(int) * c.size(), hipMemcpyDeviceToHost, ctx->stream));
+            HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+        }
         for (int k = 0; k < n; k++) {
             if (nCZDamaged) nCZDamaged[k] = c[2 * (size_t)k];
             if (nCZFailed) nCZFailed[k] = c[2 * (size_t)k + 1];

@@ -876,10 +876,28 @@ __device__ __forceinline__ void count_flags(int bid_, int nb_, const int *__rest
     }
 }
 
+// One thread of each of nb workgroups adds its counts; the last of them reports the totals when asked to
+// (rep.host; out[3] is zero before), so that the host has them after the wait of its call: a copy
+// and a second wait took 15 us of a call of 50.  A thread's tickets follow its sums because it waits for them.
+__device__ inline void add_counts(int *out, int d, int f, int nb, const Report &rep)
+{
+    if (!rep.host) {
+        if (d) atomicAdd(out, d);
+        if (f) atomicAdd(out + 1, f);
+        return;
+    }
+    const int d0 = atomicAdd(out, d), f0 = atomicAdd(out + 1, f);
+    int one = 1;
+    asm volatile("" : "+v"(one) : "v"(d0), "v"(f0));
+    if (atomicAdd(out + 3, one) != nb - 1) return;
+    rep.put(CZ_DAMAGED, (unsigned)__hip_atomic_load(out, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    rep.put(CZ_FAILED, (unsigned)__hip_atomic_load(out + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
 // count_flags for workgroups of NT threads (a multiple of 64, at most 1024).
 template <int NT>
 __device__ __forceinline__ void count_flags_n(int bid_, int nb_, const int *__restrict__ damaged,
-        const int *__restrict__ failed, int n, int *__restrict__ out)
+        const int *__restrict__ failed, int n, int *__restrict__ out, const Report &rep)
 {
     __shared__ int part[2][NT / 64];
     int d = 0, f = 0;
@@ -902,8 +920,7 @@ __device__ __forceinline__ void count_flags_n(int bid_, int nb_, const int *__re
             d += part[0][w];
             f += part[1][w];
         }
-        if (d) atomicAdd(out, d);
-        if (f) atomicAdd(out + 1, f);
+        add_counts(out, d, f, nb_, rep);
     }
 }
 
@@ -912,7 +929,7 @@ __device__ __forceinline__ void count_flags_n(int bid_, int nb_, const int *__re
 template <int NT>
 __device__ __forceinline__ void count_flags_spec(int bid_, int nb_, const int *__restrict__ damaged,
         const int *__restrict__ failed, const int *__restrict__ cz_off, int nspec, int *__restrict__ spec,
-        int *__restrict__ out)
+        int *__restrict__ out, const Report &rep)
 {
     __shared__ int part[2][NT / 64];
     int td = 0, tf = 0;
@@ -939,15 +956,16 @@ __device__ __forceinline__ void count_flags_spec(int bid_, int nb_, const int *_
             }
             spec[2 * s] = d;
             spec[2 * s + 1] = f;
+            if (rep.host && nspec <= REPORT_SPECS) {
+                rep.put(REPORT_WORDS + 2 * s, (unsigned)d);
+                rep.put(REPORT_WORDS + 2 * s + 1, (unsigned)f);
+            }
             td += d;
             tf += f;
         }
         __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        if (td) atomicAdd(out, td);
-        if (tf) atomicAdd(out + 1, tf);
-    }
+    if (threadIdx.x == 0) add_counts(out, td, tf, nb_, rep);
 }
 
 __global__ __launch_bounds__(256) void k_count_flags(const int *__restrict__ damaged, const int *__restrict__ failed,
