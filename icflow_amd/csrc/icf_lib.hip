@@ -120,6 +120,7 @@ struct SlotMap {
     int nkeys = 0;                 // keys counted; without fixed_nkeys at least the largest key + 1
     // grow-only buffers, kept when the map is built anew
     DevBuf b_off, b_codes, b_keys, b_loff, b_snap;
+    DevBuf b_off2;                 // offsets of slots that moved; changes places with b_off
     int *off = nullptr;            // nkeys + 1
     uint32_t *codes = nullptr;
     int *keys = nullptr;           // accumulate mode: the keys with contributions (null: all keys)
@@ -140,6 +141,7 @@ struct SlotMap {
     // touched the fields (suspect) the map is kept if they still compare equal
     std::vector<int *> snap;
     bool suspect = false;
+    bool changed = false;          // suspect, and the fields are known to be others
     bool built = false;
 };
 
@@ -356,14 +358,15 @@ int grow(icf_ctx *ctx, DevBuf &b, size_t bytes)
 
 void free_map(SlotMap &m)
 {
-    for (DevBuf *b : {&m.b_off, &m.b_codes, &m.b_keys, &m.b_loff, &m.b_snap, &m.b_row_node, &m.b_cz_begin, &m.b_node_row}) {
+    for (DevBuf *b : {&m.b_off, &m.b_off2, &m.b_codes, &m.b_keys, &m.b_loff, &m.b_snap, &m.b_row_node, &m.b_cz_begin, &m.b_node_row}) {
         if (b->p) (void)hipFree(b->p);
         *b = DevBuf();
     }
 }
 
 // Maps whose key fields overlap [lo, hi): dropped when the memory goes away (erase), else
-// marked suspect, to be compared against their snapshot before the next use.
+// marked suspect, to be compared against their snapshot before the next use (or not, where the
+// fields are known to have changed).
 bool map_keys_overlap(const SlotMap &m, uintptr_t lo, uintptr_t hi)
 {
     if (!m.built) return false;
@@ -375,7 +378,7 @@ bool map_keys_overlap(const SlotMap &m, uintptr_t lo, uintptr_t hi)
     return false;
 }
 
-void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = false)
+void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = false, bool changed = false)
 {
     if (ctx->adj.valid && ctx->adj.lo < hi && lo < ctx->adj.hi) {
         ctx->adj.valid = false;
@@ -390,6 +393,7 @@ void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = fal
             it = ctx->maps.erase(it);
         } else {
             if (hit) it->suspect = true;
+            if (hit && changed) it->changed = true;
             ++it;
         }
     }
@@ -636,7 +640,7 @@ int build_maps(icf_ctx *ctx, const std::vector<SlotMap *> &todo, SlotMap *mr, co
         over[j] = reported(rep, MAP_ERR + j);
         m->nlaunch = m->fixed_nkeys < 0 ? (int)((volatile unsigned *)rep.host)[MAP_NLIST + j] : m->nkeys;
         m->id = ++ctx->next_map_id;
-        m->suspect = false;
+        m->suspect = m->changed = false;
         m->built = !over[j];
     }
     if (mr) {
@@ -644,6 +648,49 @@ int build_maps(icf_ctx *ctx, const std::vector<SlotMap *> &todo, SlotMap *mr, co
         mr->tsum_ok = mr->nkeys > 0 && !reported(rep, LINK_ERR);
         mr->merge_ok = mr->tsum_ok && mf->nkeys > 0 && !reported(rep, LINK_ERR + 1);
     }
+    return 0;
+}
+
+// The new offsets of an overwrite value map (m.nkeys keys, nold before) whose slots may only have
+// moved (k_map_move); one wait.  `moved` tells whether they had; if not, the map is to be built.
+int move_map(icf_ctx *ctx, SlotMap &m, int nold, bool &moved)
+{
+    MapJobs J{};
+    J.njob = 1;
+    add_srcs(J, 0, m);
+    J.nkeys[0] = m.nkeys;
+    J.tile0[1] = blocks_for(m.nkeys, SCAN_TILE);
+    if (int r = grow(ctx, m.b_off2, sizeof(int) * ((size_t)m.nkeys + 1))) return r;
+    if (int r = grow(ctx, ctx->map_rank, sizeof(int) * (size_t)std::max(nold, 1))) return r;
+    if (int r = grow(ctx, ctx->map_sums, sizeof(unsigned long long) * std::max(J.tile0[1], 1u))) return r;
+    const size_t cnt_bytes = sizeof(int) * (size_t)std::max(m.nkeys, 1);
+    if (ctx->map_cnt.bytes < cnt_bytes) {
+        if (int r = grow(ctx, ctx->map_cnt, cnt_bytes)) return r;
+        HIPCHK(ctx, hipMemsetAsync(ctx->map_cnt.p, 0, ctx->map_cnt.bytes, ctx->stream));
+    }
+    int *cnt = (int *)ctx->map_cnt.p, *to = (int *)ctx->map_rank.p, *now = (int *)m.b_off2.p;
+    auto *sums = (unsigned long long *)ctx->map_sums.p;
+    J.off[0] = now;
+    const unsigned places = J.nsrc ? J.blk0[J.nsrc] : 0, olds = blocks_for(nold, 256);
+    const Report rep = new_report(ctx);
+    const dim3 b(256);
+    if (places) hipLaunchKernelGGL(k_map_move, dim3(places), b, 0, ctx->stream, J, to, rep);
+    if (places + olds)
+        hipLaunchKernelGGL(k_map_moved, dim3(places + olds), b, 0, ctx->stream, J, places, to, m.off, nold, cnt, rep);
+    if (J.tile0[1]) hipLaunchKernelGGL(k_map_tiles, dim3(J.tile0[1]), b, 0, ctx->stream, J, cnt, sums);
+    hipLaunchKernelGGL(k_map_scan, dim3(1), b, 0, ctx->stream, J, sums, rep);
+    if (J.tile0[1]) hipLaunchKernelGGL(k_map_offsets, dim3(J.tile0[1]), b, 0, ctx->stream, J, cnt, sums);
+    if (olds) hipLaunchKernelGGL(k_map_runs, dim3(olds), b, 0, ctx->stream, to, m.off, nold, now, rep);
+    HIPCHK(ctx, hipGetLastError());
+    HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
+    moved = !reported(rep, MAP_MOVED);
+    if (!moved) return 0;
+    std::swap(m.b_off, m.b_off2);
+    m.off = m.loff = now;
+    m.nlaunch = m.nkeys;
+    m.id = ++ctx->next_map_id;
+    m.suspect = m.changed = false;
+    m.built = true;
     return 0;
 }
 
@@ -675,11 +722,25 @@ int get_maps(icf_ctx *ctx, std::vector<MapReq> &req, const MapSrc *tet = nullptr
         if (r.map && r.map->suspect) {
             if (ctx->capturing)
                 return fail(ctx, ICF_E_CAPTURE, "a slot map must be checked during capture: run the call once uncaptured");
-            add_srcs(S, i, *r.map);
-            checked = true;
         }
     }
-    if (!ctx->capturing && (checked || !std::all_of(req.begin(), req.end(), [](const MapReq &r) { return r.map; })))
+    // Suspect maps are compared with their fields, except those known to have changed and, beside
+    // those, maps of fewer fields than they have: building them too costs less than a wait of its own
+    // (15 us a call).
+    long long changed = 0, unsure = 0;
+    for (MapReq &r : req) {
+        if (!r.map || !r.map->suspect) continue;
+        long long n = 0;
+        for (const SrcKey &s : r.srcs) n += src_fields(s);
+        (r.map->changed ? changed : unsure) += n;
+    }
+    for (int i = 0; i < nreq; i++) {
+        SlotMap *m = req[i].map;
+        if (!m || !m->suspect || m->changed || unsure < changed) continue;
+        add_srcs(S, i, *m);
+        checked = true;
+    }
+    if (!ctx->capturing && (!std::all_of(req.begin(), req.end(), [](const MapReq &r) { return r.map && !r.map->suspect; })))
         if (int r = lane_barrier(ctx)) return r;      // fields may have been written on the other lane
     if (checked) {
         const Report rep = new_report(ctx);
@@ -687,9 +748,11 @@ int get_maps(icf_ctx *ctx, std::vector<MapReq> &req, const MapSrc *tet = nullptr
         HIPCHK(ctx, hipGetLastError());
         HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
         for (int i = 0; i < nreq; i++)
-            if (req[i].map && req[i].map->suspect && !reported(rep, SNAP_DIFF + i)) req[i].map->suspect = false;
+            if (req[i].map && req[i].map->suspect && !reported(rep, SNAP_DIFF + i) && !req[i].map->changed)
+                req[i].map->suspect = false;
     }
     std::vector<SlotMap *> todo, first;
+    int nold = -1;                     // keys of the last of them if its slots may only have moved
     for (MapReq &r : req) {
         if (r.map && !r.map->suspect) continue;
         if (ctx->capturing)
@@ -715,9 +778,11 @@ int get_maps(icf_ctx *ctx, std::vector<MapReq> &req, const MapSrc *tet = nullptr
             }
         }
         SlotMap &m = *r.map;
+        nold = m.built && m.target == TGT_VALS && m.fixed_nkeys >= 0 && m.srcs == r.srcs ? m.nkeys : -1;
         if (m.built) bump(ctx);
         m.built = false;
         m.suspect = true;              // until it is built
+        m.changed = true;
         m.tsum_with = -1;
         m.target = r.target;
         m.fixed_nkeys = r.fixed_nkeys;
@@ -758,6 +823,11 @@ int get_maps(icf_ctx *ctx, std::vector<MapReq> &req, const MapSrc *tet = nullptr
     if (todo.empty() && !mr) return 0;
     bool over[MAX_JOBS] = {};
     int err = first.empty() ? 0 : size_keys(first);
+    if (!err && todo.size() == 1 && !mr && nold >= 0) {
+        bool moved = false;
+        err = move_map(ctx, *todo[0], nold, moved);
+        if (moved) return 0;
+    }
     if (!err) err = build_maps(ctx, todo, mr, mf, tet, over);
     std::vector<SlotMap *> again;
     bool bad = false;
@@ -2556,7 +2626,7 @@ int icf_pack_pcsr(icf_ctx *ctx, const int *altId, int nNodes, const int *csr_row
                         hi = (uintptr_t)(p.base + (size_t)p.stride * (row0 + K));
         for (int f = 0; f < 2; f++) {
             const uintptr_t a = f ? mid : lo, b = f ? hi : mid;
-            if (err || reported(rep, PACK_CHANGED + 2 * k + f)) invalidate_range(ctx, a, b);
+            if (err || reported(rep, PACK_CHANGED + 2 * k + f)) invalidate_range(ctx, a, b, false, !err);
             else touch_range(ctx, a, b);
         }
     }

@@ -49,11 +49,11 @@ __global__ __launch_bounds__(256) void k_map_maxkey(MapSrc s, int *__restrict__ 
 // sums, their scan, offsets with the lists of keys that have contributions, fill, sort.  Every
 // buffer is sized by what it could hold, so nothing waits for a count; the host reads the number
 // of keys to visit and the errors from the report, after one wait.  A Newton loop with contact
-// builds four maps in each iteration (the impacts change, and with them every slot), a step in
-// which CZs failed three: with the chunk tables of the value reductions laid out on the host and
-// allocations in between this took 16.9 + 6.5 ms in an iteration of the 384,000-tet compression,
-// 0.38 + 0.11 ms as it is.  The atomics of the count bound it (5.8M contributions), then the scattered
-// stores of the fill.
+// builds the impacts' three maps in each iteration (the impacts change), and the first one of a step in
+// which CZs failed those of the elements and CZs: with the chunk tables of the value reductions
+// laid out on the host and allocations in between the collision response of the 384,000-tet
+// compression took 6.7 ms, 0.18 ms as it is, the assembly after CZs failed on the 15,360-tet beam 1.0
+// ms, now 0.17.  The atomics of the count bound large maps, the six launches small ones.
 constexpr int MAX_JOBS = 3, MAX_MAP_SRCS = 6;
 constexpr int SCAN_ITEMS = 8, SCAN_TILE = 256 * SCAN_ITEMS;
 struct MapJobs {
@@ -79,9 +79,9 @@ static_assert(MAP_NLIST + MAX_JOBS <= REPORT_WORDS, "report words");
 // Source, unit and field of this thread; false beyond the units.  All fields of 256 units are taken
 // by neighbouring workgroups of one XCD, which so keeps the lines of their keys in its L2 (fields after
 // fields, dealt over all XCDs, the count took 254 us for 5.8M contributions, now 229, the fill 98, now 62).
-__device__ inline bool map_place(const MapJobs &J, int &k, int &u, int &q)
+__device__ inline bool map_place(const MapJobs &J, int &k, int &u, int &q, unsigned nb = gridDim.x)
 {
-    unsigned b = (unsigned)xcd_remap(blockIdx.x, gridDim.x);
+    unsigned b = (unsigned)xcd_remap(blockIdx.x, (int)nb);
     k = 0;
     while (k + 1 < J.nsrc && b >= J.blk0[k + 1]) k++;
     b -= J.blk0[k];
@@ -233,6 +233,57 @@ __global__ __launch_bounds__(256) void k_map_sort(MapJobs J)
     if (e > b) sort_codes(lds, b - c0, e - c0);
     __syncthreads();
     for (int i = threadIdx.x; i < c1 - c0; i += 256) codes[c0 + i] = lds[i];
+}
+
+// ---- slots that only moved -------------------------------------------------------------------
+// A Newton iteration with contact has the units of the last one, but other impacts' blocks between
+// theirs: every slot moves up or down, their order stays, and with it the codes.  Then the map needs
+// new offsets alone: moved[old slot] = new slot is taken from the fields, all fields are held
+// against it, the lengths of the runs go to the new slots, and their scan has to put each run
+// where it was (which also shows that no two slots became one); anything else is reported, and the map is
+// built from the fields.  No atomics, no sort, and the codes are not written: the assembly of an
+// iteration of the 384,000-tet compression takes 254 us instead of 492, of one with 44,574 tets 96
+// instead of 157.  Two passes over 5.8M fields bound it.
+constexpr int MAP_MOVED = 3;        // word of the report: not so
+__global__ __launch_bounds__(256) void k_map_move(MapJobs J, int *__restrict__ moved, Report rep)
+{
+    int k, u, q;
+    if (!map_place(J, k, u, q)) return;
+    const MapSrc &s = J.src[k];
+    const int old = J.snap[k][(size_t)q * s.n + u], key = s.base[u + (size_t)s.stride * (s.field0 + q)];
+    if ((old < 0) != (key < 0) || key >= J.nkeys[0]) rep.set(MAP_MOVED);
+    else if (old >= 0 && moved[old] != key) moved[old] = key;
+}
+
+// Workgroups below `places` compare the fields and copy them; the others take the runs of the old slots.
+__global__ __launch_bounds__(256) void k_map_moved(MapJobs J, unsigned places, const int *__restrict__ moved,
+                                                   const int *__restrict__ off, int nold, int *__restrict__ cnt,
+                                                   Report rep)
+{
+    if (rep.was(MAP_MOVED)) return;
+    if (blockIdx.x >= places) {
+        const int k = (int)(blockIdx.x - places) * 256 + (int)threadIdx.x;
+        const int n = k < nold ? off[k + 1] - off[k] : 0;
+        if (n) cnt[moved[k]] = n;
+        return;
+    }
+    int k, u, q;
+    if (!map_place(J, k, u, q, places)) return;
+    const MapSrc &s = J.src[k];
+    const size_t i = (size_t)q * s.n + u;
+    const int old = J.snap[k][i], key = s.base[u + (size_t)s.stride * (s.field0 + q)];
+    if (old < 0) return;
+    if (moved[old] != key) rep.set(MAP_MOVED);
+    if (old != key) J.snap[k][i] = key;
+}
+
+__global__ __launch_bounds__(256) void k_map_runs(const int *__restrict__ moved, const int *__restrict__ off, int nold,
+                                                  const int *__restrict__ now, Report rep)
+{
+    if (rep.was(MAP_MOVED)) return;
+    const int k = blockIdx.x * 256 + (int)threadIdx.x;
+    if (k >= nold || off[k] == off[k + 1]) return;
+    if (now[moved[k]] != off[k] || now[moved[k] + 1] != off[k + 1]) rep.set(MAP_MOVED);
 }
 
 // Whether a source's fields still are what the map was built from.
