@@ -283,13 +283,12 @@ __global__ __launch_bounds__(256) void k_bp_tiles(const int *__restrict__ v, int
     __shared__ unsigned part[4];
     if (!grid->ok) return;
     if (n < 0) n = grid->G;
-    const int k0 = (int)blockIdx.x * BP_TILE;
-    if (k0 >= n) return;
+    if ((int)blockIdx.x * BP_TILE >= n) return;
+    const int k0 = (int)blockIdx.x * BP_TILE + (int)threadIdx.x * BP_ITEMS;
     unsigned x = 0;
-    for (int r = 0; r < BP_ITEMS; r++) {
-        const int k = k0 + r * 256 + (int)threadIdx.x;
-        if (k < n) x += (unsigned)v[k];
-    }
+#pragma unroll
+    for (int r = 0; r < BP_ITEMS; r++)
+        if (k0 + r < n) x += (unsigned)v[k0 + r];
     x = sum256(x, part);
     if (threadIdx.x == 0) tiles.put(blockIdx.x, x);
 }
@@ -299,18 +298,24 @@ __global__ __launch_bounds__(256) void k_bp_scan(const int *__restrict__ v, int 
     __shared__ unsigned part[4];
     if (!grid->ok) return;
     if (n < 0) n = grid->G;
-    const int k0 = (int)blockIdx.x * BP_TILE;
-    if (k0 >= n) return;
-    unsigned run = tiles.before(blockIdx.x, part), total;
+    if ((int)blockIdx.x * BP_TILE >= n) return;
+    const int k0 = (int)blockIdx.x * BP_TILE + (int)threadIdx.x * BP_ITEMS;
+    unsigned c[BP_ITEMS], x = 0, total;
+#pragma unroll
     for (int r = 0; r < BP_ITEMS; r++) {
-        const int k = k0 + r * 256 + (int)threadIdx.x;
-        const unsigned at = run + scan256(k < n ? (unsigned)v[k] : 0u, part, total);
-        run += total;
-        if (k < n) out[k] = (int)at;
+        c[r] = k0 + r < n ? (unsigned)v[k0 + r] : 0u;
+        x += c[r];
     }
-    if (k0 + BP_TILE >= n && threadIdx.x == 0) {
-        out[n] = (int)run;
-        if (word >= 0) rep.put(word, run);
+    const unsigned run = tiles.before(blockIdx.x, part);
+    unsigned at = run + scan256(x, part, total);
+#pragma unroll
+    for (int r = 0; r < BP_ITEMS; r++) {
+        if (k0 + r < n) out[k0 + r] = (int)at;
+        at += c[r];
+    }
+    if ((int)(blockIdx.x + 1) * BP_TILE >= n && threadIdx.x == 0) {
+        out[n] = (int)(run + total);
+        if (word >= 0) rep.put(word, run + total);
     }
 }
 

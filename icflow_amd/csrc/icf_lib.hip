@@ -602,7 +602,7 @@ int build_maps(icf_ctx *ctx, const std::vector<SlotMap *> &todo, SlotMap *mr, co
         J.nkeys[j] = m->nkeys;
         J.vals[j] = m->target == TGT_VALS;
         J.cnt0[j] = keys;
-        J.tile0[j + 1] = J.tile0[j] + blocks_for(m->nkeys, SCAN_TILE);
+        J.tile0[j + 1] = J.tile0[j] + std::max(blocks_for(m->nkeys, SCAN_TILE), 1u);
         J.sort0[j + 1] = J.sort0[j] + blocks_for(m->nkeys, 256);
         J.off[j] = m->off;
         J.codes[j] = m->codes;
@@ -625,9 +625,8 @@ int build_maps(icf_ctx *ctx, const std::vector<SlotMap *> &todo, SlotMap *mr, co
     if (J.njob) {
         const dim3 b(256);
         if (places) hipLaunchKernelGGL(k_map_count, dim3(places), b, 0, ctx->stream, J, cnt, rank, rep);
-        if (tiles) hipLaunchKernelGGL(k_map_tiles, dim3(tiles), b, 0, ctx->stream, J, cnt, sums);
-        hipLaunchKernelGGL(k_map_scan, dim3(1), b, 0, ctx->stream, J, sums, rep);
-        if (tiles) hipLaunchKernelGGL(k_map_offsets, dim3(tiles), b, 0, ctx->stream, J, cnt, sums);
+        hipLaunchKernelGGL(k_map_tiles, dim3(tiles), b, 0, ctx->stream, J, cnt, sums);
+        hipLaunchKernelGGL(k_map_offsets, dim3(tiles), b, 0, ctx->stream, J, cnt, sums, rep);
         if (places) hipLaunchKernelGGL(k_map_fill, dim3(places), b, 0, ctx->stream, J, rank);
         if (sorts) hipLaunchKernelGGL(k_map_sort, dim3(sorts), b, 0, ctx->stream, J);
     }
@@ -659,7 +658,7 @@ int move_map(icf_ctx *ctx, SlotMap &m, int nold, bool &moved)
     J.njob = 1;
     add_srcs(J, 0, m);
     J.nkeys[0] = m.nkeys;
-    J.tile0[1] = blocks_for(m.nkeys, SCAN_TILE);
+    J.tile0[1] = std::max(blocks_for(m.nkeys, SCAN_TILE), 1u);
     if (int r = grow(ctx, m.b_off2, sizeof(int) * ((size_t)m.nkeys + 1))) return r;
     if (int r = grow(ctx, ctx->map_rank, sizeof(int) * (size_t)std::max(nold, 1))) return r;
     if (int r = grow(ctx, ctx->map_sums, sizeof(unsigned long long) * std::max(J.tile0[1], 1u))) return r;
@@ -677,9 +676,8 @@ int move_map(icf_ctx *ctx, SlotMap &m, int nold, bool &moved)
     if (places) hipLaunchKernelGGL(k_map_move, dim3(places), b, 0, ctx->stream, J, to, rep);
     if (places + olds)
         hipLaunchKernelGGL(k_map_moved, dim3(places + olds), b, 0, ctx->stream, J, places, to, m.off, nold, cnt, rep);
-    if (J.tile0[1]) hipLaunchKernelGGL(k_map_tiles, dim3(J.tile0[1]), b, 0, ctx->stream, J, cnt, sums);
-    hipLaunchKernelGGL(k_map_scan, dim3(1), b, 0, ctx->stream, J, sums, rep);
-    if (J.tile0[1]) hipLaunchKernelGGL(k_map_offsets, dim3(J.tile0[1]), b, 0, ctx->stream, J, cnt, sums);
+    hipLaunchKernelGGL(k_map_tiles, dim3(J.tile0[1]), b, 0, ctx->stream, J, cnt, sums);
+    hipLaunchKernelGGL(k_map_offsets, dim3(J.tile0[1]), b, 0, ctx->stream, J, cnt, sums, rep);
     if (olds) hipLaunchKernelGGL(k_map_runs, dim3(olds), b, 0, ctx->stream, to, m.off, nold, now, rep);
     HIPCHK(ctx, hipGetLastError());
     HIPCHK(ctx, hipStreamSynchronize(ctx->stream));
@@ -1129,7 +1127,7 @@ void tune_end(icf_ctx *ctx, icf_ctx::Tune &t)
 int tune_begin(icf_ctx *ctx, bool acc, bool fp64, long long keys)
 {
     const int c = tune_begin(ctx, ctx->tune[acc][fp64], 2 * acc + fp64, keys);
-    return c >= 0 ? c : keys <= VALS_SMALL ? CAND_SMALL : CAND_UNTUNED;
+    return c >= 0 ? c : !acc && keys <= VALS_SMALL ? CAND_SMALL : CAND_UNTUNED;
 }
 void tune_end(icf_ctx *ctx, bool acc, bool fp64) { tune_end(ctx, ctx->tune[acc][fp64]); }
 

@@ -44,7 +44,7 @@ __global__ __launch_bounds__(256) void k_map_maxkey(MapSrc s, int *__restrict__ 
 }
 
 // ---- building slot maps ----------------------------------------------------------------------
-// The maps a call needs and does not have are built together, in six launches and without a word
+// The maps a call needs and does not have are built together, in five launches and without a word
 // from the host in between: count (each contribution also takes its rank among its key's), block
 // sums, their scan, offsets with the lists of keys that have contributions, fill, sort.  Every
 // buffer is sized by what it could hold, so nothing waits for a count; the host reads the number
@@ -53,7 +53,7 @@ __global__ __launch_bounds__(256) void k_map_maxkey(MapSrc s, int *__restrict__ 
 // which CZs failed those of the elements and CZs: with the chunk tables of the value reductions
 // laid out on the host and allocations in between the collision response of the 384,000-tet
 // compression took 6.7 ms, 0.18 ms as it is, the assembly after CZs failed on the 15,360-tet beam 1.0
-// ms, now 0.17.  The atomics of the count bound large maps, the six launches small ones.
+// ms, now 0.17.  The atomics of the count bound large maps, the five launches small ones.
 constexpr int MAX_JOBS = 3, MAX_MAP_SRCS = 6;
 constexpr int SCAN_ITEMS = 8, SCAN_TILE = 256 * SCAN_ITEMS;
 struct MapJobs {
@@ -66,7 +66,7 @@ struct MapJobs {
     int nkeys[MAX_JOBS];
     bool vals[MAX_JOBS];                // keys are BCSR blocks
     long long cnt0[MAX_JOBS];           // the map's place in `cnt` (nkeys counts)
-    unsigned tile0[MAX_JOBS + 1];       // first scan tile of a map
+    unsigned tile0[MAX_JOBS + 1];       // first scan tile of a map (one at least)
     unsigned sort0[MAX_JOBS + 1];       // first sorting workgroup of a map
     int *off[MAX_JOBS];                 // nkeys + 1: first code of each key
     uint32_t *codes[MAX_JOBS];
@@ -118,69 +118,64 @@ __device__ inline int tile_job(const MapJobs &J, int &k0)
     return j;
 }
 
+// Eight consecutive keys per thread, so that a tile takes one scan over its threads.
 __global__ __launch_bounds__(256) void k_map_tiles(MapJobs J, const int *__restrict__ cnt,
                                                    unsigned long long *__restrict__ sums)
 {
     __shared__ unsigned long long part[4];
     int k0;
     const int j = tile_job(J, k0);
+    k0 += (int)threadIdx.x * SCAN_ITEMS;
     unsigned long long v = 0, total;
-    for (int r = 0; r < SCAN_ITEMS; r++) {
-        const int k = k0 + r * 256 + (int)threadIdx.x;
-        if (k < J.nkeys[j]) v += scan_item(cnt[J.cnt0[j] + k]);
-    }
+#pragma unroll
+    for (int r = 0; r < SCAN_ITEMS; r++)
+        if (k0 + r < J.nkeys[j]) v += scan_item(cnt[J.cnt0[j] + k0 + r]);
     (void)scan256(v, part, total);
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-// One workgroup: each map's tile sums become the tiles' starts; the totals end the offsets.
-__global__ __launch_bounds__(256) void k_map_scan(MapJobs J, unsigned long long *__restrict__ sums, Report rep)
-{
-    __shared__ unsigned long long part[4];
-    for (int j = 0; j < J.njob; j++) {
-        unsigned long long run = 0, total;
-        for (unsigned t0 = J.tile0[j]; t0 < J.tile0[j + 1]; t0 += 256) {
-            const unsigned t = t0 + threadIdx.x;
-            const unsigned long long v = t < J.tile0[j + 1] ? sums[t] : 0ULL;
-            const unsigned long long x = scan256(v, part, total);
-            if (t < J.tile0[j + 1]) sums[t] = run + x;
-            run += total;
-        }
-        if (threadIdx.x == 0) {
-            const int n = (int)(run >> 32), c = (int)(run & 0xffffffffULL);
-            J.off[j][J.nkeys[j]] = c;
-            if (J.loff[j]) J.loff[j][n] = c;
-            rep.put(MAP_NLIST + j, (unsigned)n);
-        }
-    }
-}
-
 // First code of every key, the list of keys with contributions; cnt is left zero for the next maps.
+// Every tile adds up the map's tiles before it; its last one ends the offsets and reports the length
+// of the list.
 __global__ __launch_bounds__(256) void k_map_offsets(MapJobs J, int *__restrict__ cnt,
-                                                     const unsigned long long *__restrict__ sums)
+                                                     const unsigned long long *__restrict__ sums, Report rep)
 {
     __shared__ unsigned long long part[4];
     int k0;
     const int j = tile_job(J, k0);
-    unsigned long long run = sums[blockIdx.x], total;
+    k0 += (int)threadIdx.x * SCAN_ITEMS;
+    int c[SCAN_ITEMS];
+    unsigned long long v = 0, before = 0, run, total;
+#pragma unroll
     for (int r = 0; r < SCAN_ITEMS; r++) {
-        const int k = k0 + r * 256 + (int)threadIdx.x;
-        const bool in = k < J.nkeys[j];
-        int c = 0;
-        if (in) {
-            c = cnt[J.cnt0[j] + k];
-            if (c) cnt[J.cnt0[j] + k] = 0;
-        }
-        const unsigned long long x = run + scan256(scan_item(c), part, total);
-        run += total;
-        if (!in) continue;
+        c[r] = k0 + r < J.nkeys[j] ? cnt[J.cnt0[j] + k0 + r] : 0;
+        v += scan_item(c[r]);
+    }
+    for (unsigned t = J.tile0[j] + threadIdx.x; t < blockIdx.x; t += 256) before += sums[t];
+    (void)scan256(before, part, run);
+    unsigned long long x = run + scan256(v, part, total);
+#pragma unroll
+    for (int r = 0; r < SCAN_ITEMS; r++) {
+        const int k = k0 + r;
+        if (k >= J.nkeys[j]) break;
         const int first = (int)(x & 0xffffffffULL);
         J.off[j][k] = first;
-        if (c && J.keys[j]) {
-            const int p = (int)(x >> 32);
-            J.keys[j][p] = k;
-            J.loff[j][p] = first;
+        if (c[r]) {
+            cnt[J.cnt0[j] + k] = 0;
+            if (J.keys[j]) {
+                const int p = (int)(x >> 32);
+                J.keys[j][p] = k;
+                J.loff[j][p] = first;
+            }
         }
+        x += scan_item(c[r]);
+    }
+    if (blockIdx.x + 1 == J.tile0[j + 1] && threadIdx.x == 0) {
+        const unsigned long long all = run + total;
+        const int n = (int)(all >> 32), e = (int)(all & 0xffffffffULL);
+        J.off[j][J.nkeys[j]] = e;
+        if (J.loff[j]) J.loff[j][n] = e;
+        rep.put(MAP_NLIST + j, (unsigned)n);
     }
 }
 
@@ -314,8 +309,10 @@ constexpr int CAND_FP32 = 2 * NSC + 0, CAND_FP64 = 2 * NSC + 1;   // a context's
 // batched specimens mixed 621 (627-703), 779,000 tets FP64 190 (187-201), 309,000 tets FP64 65
 // (65-75), 146,000 tets mixed 30.0 (28.6-32.8).
 constexpr int CAND_UNTUNED = 1 * NSC + 1;
-// ... and where that leaves most of the chip idle, one wave of 64 keys with room for all of their
-// contributions.
+// ... and where that leaves most of the chip idle, up to 131,072 blocks to overwrite, one wave of 64
+// keys with room for all of their contributions: 17.2 against 17.7 us (3,072 tets), 18.4 against 21.7
+// (15,360), 19.4 against 21.4 (93,000 blocks); at 202,000 blocks 25.6 against 25.2.  (Impacts add few to
+// a block, which any shape takes in one round.)
 constexpr int CAND_SMALL = NCAND, SMALL_KEYS = 64, SMALL_STAGE = 16, VALS_SMALL = 1 << 17;
 template <typename L, int KEYS, int STAGE>
 __host__ __device__ constexpr int flat_cap() { return sizeof(L) == 4 ? STAGE * KEYS : STAGE * KEYS / 2; }
