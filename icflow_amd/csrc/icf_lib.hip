@@ -194,9 +194,8 @@ constexpr int shape_value(int role, int c)
 constexpr int shape_ncand(int role) { return role == ICF_SHAPE_ORDER ? 2 : 3; }
 constexpr int SHAPE_DEFAULT[NSHAPE] = {2, 2, 1, 2, 1};   // 256, 256, 8 lanes, 256, interleaved
 // What untuned launches use: the same, but node forces first.  Interleaved with the values they
-// gained 40 us on 256 specimens while both waited on memory; since they do not, the order costs up
-// to 9 us of 30 on 146,000 tets and nothing is left to hide (256 specimens: 621 first, 626
-// interleaved).
+// gained 40 us on 256 specimens while both waited on memory; since they do not, the order costs 6 us
+// of 34 on 146,000 tets and gives 4 of 584 on 256 specimens.
 constexpr int SHAPE_UNTUNED[NSHAPE] = {2, 2, 1, 2, 0};
 
 struct icf_ctx {

@@ -306,8 +306,8 @@ __host__ __device__ constexpr int cand_stage(int c) { return STAGE_CANDS[c % NSC
 constexpr int CAND_FP32 = 2 * NSC + 0, CAND_FP64 = 2 * NSC + 1;   // a context's shape until tuned or set
 // Launches of roles that are neither tuned nor set take 128 keys, 3 FP32 or 1.5 FP64 contributions
 // per key.  Time of the fused value launch, and of the other shapes of 64 to 256 keys (us): 256
-// batched specimens mixed 621 (627-703), 779,000 tets FP64 190 (187-201), 309,000 tets FP64 65
-// (65-75), 146,000 tets mixed 30.0 (28.6-32.8).
+// batched specimens mixed 584 (604-653), 787,000 tets FP64 176 (173-196), 24 specimens FP64 60.6
+// (60.1-72.4), 146,000 tets mixed 28.3 (25.9-30.4).
 constexpr int CAND_UNTUNED = 1 * NSC + 1;
 // ... and where that leaves most of the chip idle, up to 131,072 blocks to overwrite, one wave of 64
 // keys with room for all of their contributions: 17.2 against 17.7 us (3,072 tets), 18.4 against 21.7
