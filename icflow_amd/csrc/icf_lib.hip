@@ -197,6 +197,13 @@ constexpr int SHAPE_DEFAULT[NSHAPE] = {2, 2, 1, 2, 1};   // 256, 256, 8 lanes, 2
 // gained 40 us on 256 specimens while both waited on memory; since they do not, the order costs 6 us
 // of 34 on 146,000 tets and gives 4 of 584 on 256 specimens.
 constexpr int SHAPE_UNTUNED[NSHAPE] = {2, 2, 1, 2, 0};
+// ... and for launches of at most so many units, whose workgroups would leave compute units empty
+// while each runs through a long chain: phase 1 with 64 lanes (14.3 -> 11.9 us on 3,072 tets, 20.7 ->
+// 18.9 on 48,000, 42.9 -> 41.9 on 309,000; 113.7 -> 117.7 on 779,000), 64 impacts (21.9 -> 17.8 us for
+// 547, 27.0 -> 18.2 for 7,000, 25.2 -> 22.1 for 20,900; 25.3 -> 28.3 for 61,600), 16 lanes per
+// tuple (9.5 -> 8.3 us for 547, 11.2 -> 9.9 for 7,000; 14.8 -> 14.4 for 20,900, 27.6 -> 28.4 for 61,600).
+constexpr int SHAPE_SMALL[NSHAPE] = {0, 2, 2, 0, 0};
+constexpr long long SHAPE_SMALL_MAX[NSHAPE] = {1 << 19, 0, 1 << 14, 1 << 15, 0};
 
 struct icf_ctx {
     int id = 0;
@@ -274,6 +281,8 @@ struct icf_ctx {
         int sel = CAND_FP32;       // candidate in use
         bool tuned = false;        // a tuning has chosen it
         int untuned = -1;              // what launches use when it is neither tuned nor set; -1: by their size
+        int small = 0;                 // ... where they have at most small_max units
+        long long small_max = 0;
         bool active = false;       // timing the candidates in turn
         bool fixed = false;        // chosen by the caller (icf_set_chunk_keys / icf_set_shape)
         int turn = 0;              // launches started while tuning
@@ -1105,7 +1114,7 @@ int tune_begin(icf_ctx *ctx, icf_ctx::Tune &t, int role_id, long long units, boo
             std::lock_guard<std::mutex> lk(g_shape_cache.mu);
             auto it = g_shape_cache.choice.find({ctx->device, role_id, ctx->precision, bucket});
             if (it != g_shape_cache.choice.end()) return it->second;
-            if (!t.tuned) return t.untuned;
+            if (!t.tuned) return units <= t.small_max ? t.small : t.untuned;
         }
         return t.sel;
     }
@@ -1383,6 +1392,8 @@ int icf_create(int device, icf_ctx **out)
         ctx->shape[r].ncand = shape_ncand(r);
         ctx->shape[r].sel = SHAPE_DEFAULT[r];
         ctx->shape[r].untuned = SHAPE_UNTUNED[r];
+        ctx->shape[r].small = SHAPE_SMALL[r];
+        ctx->shape[r].small_max = SHAPE_SMALL_MAX[r];
     }
     ctx->id = g_next_ctx_id++;
     ctx->device = device;
