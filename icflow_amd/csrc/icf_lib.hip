@@ -386,7 +386,7 @@ bool map_keys_overlap(const SlotMap &m, uintptr_t lo, uintptr_t hi)
     return false;
 }
 
-void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = false, bool changed = false)
+void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = false)
 {
     if (ctx->adj.valid && ctx->adj.lo < hi && lo < ctx->adj.hi) {
         ctx->adj.valid = false;
@@ -401,19 +401,47 @@ void invalidate_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, bool erase = fal
             it = ctx->maps.erase(it);
         } else {
             if (hit) it->suspect = true;
-            if (hit && changed) it->changed = true;
             ++it;
         }
     }
 }
 
-// Fields in [lo, hi) were written again with the values they had: what was built from them holds,
-// and only graphs captured before are refused, as after any write to such fields.
-void touch_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi)
+// The built map that has one of its sources over these fields of a unit array; a map not in doubt
+// rather than one that is.
+SlotMap *map_over(icf_ctx *ctx, const int *base, int n, int stride, int field0, int nq, const int **snap)
 {
-    bool hit = ctx->adj.valid && ctx->adj.lo < hi && lo < ctx->adj.hi;
-    for (const SlotMap &m : ctx->maps) hit = hit || map_keys_overlap(m, lo, hi);
-    if (hit) ctx->epoch++;
+    SlotMap *found = nullptr;
+    for (SlotMap &m : ctx->maps) {
+        if (!m.built || (found && (!found->suspect || m.suspect))) continue;
+        for (size_t i = 0; i < m.srcs.size(); i++) {
+            const SrcKey &s = m.srcs[i];
+            if (s.base != base || s.n != n || s.stride != stride || s.field0 != field0 || s.nq != nq) continue;
+            found = &m;
+            *snap = m.snap[i];
+        }
+    }
+    return found;
+}
+
+// Fields in [lo, hi) were packed.  `held`, the map whose copy they were compared with, stays as it
+// is if they are still its own (same); every other map over them is compared with its copy before its
+// next use.  Graphs captured before are refused either way, as after any write to such fields.
+void packed_range(icf_ctx *ctx, uintptr_t lo, uintptr_t hi, const SlotMap *held, bool same, bool changed)
+{
+    if (ctx->adj.valid && ctx->adj.lo < hi && lo < ctx->adj.hi) {
+        ctx->adj.valid = false;
+        bump(ctx);
+    }
+    for (SlotMap &m : ctx->maps) {
+        if (!map_keys_overlap(m, lo, hi)) continue;
+        if (&m == held && same && !m.suspect) {
+            ctx->epoch++;
+            continue;
+        }
+        bump(ctx);
+        m.suspect = true;
+        if (&m == held && changed) m.changed = true;
+    }
 }
 
 // A write by the library into caller memory [p, p + bytes) (copies, kernels that write int
@@ -2614,6 +2642,14 @@ int icf_pack_pcsr(icf_ctx *ctx, const int *altId, int nNodes, const int *csr_row
         return fail(ctx, ICF_E_INVALID, "icf_pack_pcsr: invalid argument");
     if (ctx->capturing) return fail(ctx, ICF_E_CAPTURE, "icf_pack_pcsr reports index errors to the host");
     PackAll ps{{{ie, nElems, el_stride}, {icz, nCZs, cz_stride}, {icr, nImpacts, cr_stride}}, {}};
+    const SlotMap *held[3][2] = {};
+    for (int k = 0; k < 3; k++) {
+        PackPart &p = ps.part[k];
+        const int slot0 = k == 1 ? CZI_SLOTS : EL_SLOTS, row0 = k == 1 ? CZI_ROWS : EL_ROWS, K = k == 1 ? 6 : 4;
+        if (!p.n) continue;
+        held[k][0] = map_over(ctx, p.base, p.n, p.stride, slot0, K * K, &p.slots);
+        held[k][1] = map_over(ctx, p.base, p.n, p.stride, row0, K, &p.rows);
+    }
     ps.wave1[0] = pack_waves(nElems, 4);
     ps.wave1[1] = ps.wave1[0] + pack_waves(nCZs, 6);
     ps.wave1[2] = ps.wave1[1] + pack_waves(nImpacts, 4);
@@ -2624,7 +2660,6 @@ int icf_pack_pcsr(icf_ctx *ctx, const int *altId, int nNodes, const int *csr_row
     const hipError_t launched = hipGetLastError();
     const hipError_t waited = hipStreamSynchronize(ctx->stream);
     const bool err = launched != hipSuccess || waited != hipSuccess || reported(rep, PACK_ERR);
-    // maps built from slot or row fields that changed are checked before their next use
     for (int k = 0; k < 3; k++) {
         const PackPart &p = ps.part[k];
         if (!p.n) continue;
@@ -2634,8 +2669,8 @@ int icf_pack_pcsr(icf_ctx *ctx, const int *altId, int nNodes, const int *csr_row
                         hi = (uintptr_t)(p.base + (size_t)p.stride * (row0 + K));
         for (int f = 0; f < 2; f++) {
             const uintptr_t a = f ? mid : lo, b = f ? hi : mid;
-            if (err || reported(rep, PACK_CHANGED + 2 * k + f)) invalidate_range(ctx, a, b, false, !err);
-            else touch_range(ctx, a, b);
+            const bool differ = err || reported(rep, PACK_CHANGED + 2 * k + f);
+            packed_range(ctx, a, b, held[k][f], !differ, differ && !err);
         }
     }
     HIPCHK(ctx, launched);

@@ -386,6 +386,9 @@ __global__ __launch_bounds__(256) void k_pat_write(const int *__restrict__ srow,
 struct PackPart {
     int *base;
     int n, stride;
+    // copies of the slot and row fields that a slot map was built from (field after field, n units
+    // each), or null
+    const int *slots, *rows;
 };
 struct PackAll {
     PackPart part[3];      // elements, CZs, impacts
@@ -393,18 +396,20 @@ struct PackAll {
 };
 __host__ __device__ inline long long pack_waves(int n, int K) { return ((long long)n + 63) / 64 * K; }
 
-// Words of a call's report (Report).
+// Words of a call's report (Report): an error; fields that are not what their slot map was built from.
 constexpr int PACK_ERR = 0, PACK_CHANGED = 1;   // PACK_CHANGED + 2 part + (0: slots, 1: rows)
 
 // Slot and row fields of local row i of unit u.  A slot that already names its pair -- a position
 // inside row altId_i of the pattern whose column is altId_j, or -1 where there is no block -- is
 // the slot the search would find (a row's columns are distinct), and is left alone: between two
-// iterations with the same pattern nothing is searched or written, and the report tells the host
-// that the maps built from the fields still hold.  For the 830,320 CZs of 256 batched specimens
-// the call takes 118 us instead of 319 with a search per pair (and the assembly that follows no
-// longer compares 0.5 GB of fields with their copies, 1,360 instead of 1,810 us); what is left is
-// the reading of 36 slots and 21 columns per CZ.  Where a slot differs, the K searches of the row
-// go down together, one column load each per step.
+// iterations with the same pattern nothing is searched or written.  Whether the maps still hold is
+// another matter: a slot may be right because another context or a kernel of the caller's wrote it
+// since, so what is in the fields at the end is held against the copy that the map was built from,
+// written here or not.  For the 830,320 CZs of 256 batched specimens the call took 319 us with a
+// search per pair, 118 without, 135 with the comparison (and the assembly that follows
+// no longer compares 0.5 GB of fields with their copies, 1,360 instead of 1,810 us); what is left is
+// the reading of 36 slots, their copies and 21 columns per CZ.  Where a slot differs, the K searches
+// of the row go down together, one column load each per step.
 template <int K>
 __device__ __forceinline__ void pack_row(const PackPart &s, int u, int i, int node0, int slot0, int row0,
                                          const int *__restrict__ alt, int nNodes, const int *__restrict__ rows,
@@ -418,6 +423,10 @@ __device__ __forceinline__ void pack_row(const PackPart &s, int u, int i, int no
     for (int j = 0; j < K; j++) cur[j] = slot[(size_t)s.stride * j];
     int *row = s.base + u + (size_t)s.stride * (row0 + i);
     const int cur_row = *row;
+    int was[K];                            // no copy: nothing to differ from
+#pragma unroll
+    for (int j = 0; j < K; j++) was[j] = s.slots ? s.slots[u + (size_t)s.n * (i * K + j)] : cur[j];
+    const int was_row = s.rows ? s.rows[u + (size_t)s.n * i] : cur_row;
     int ai = -1;
     bool bad = false;
 #pragma unroll
@@ -430,10 +439,8 @@ __device__ __forceinline__ void pack_row(const PackPart &s, int u, int i, int no
     }
     err |= bad;
     const int want_row = ai >= 0 ? ai : -1;
-    if (cur_row != want_row) {
-        *row = want_row;
-        rowf = true;
-    }
+    if (cur_row != want_row) *row = want_row;
+    rowf |= was_row != want_row;
     const int r0 = ai >= 0 ? rows[ai] : 0, r1 = ai >= 0 ? rows[ai + 1] : 0;
     bool need[K], keep = true;
 #pragma unroll
@@ -443,7 +450,11 @@ __device__ __forceinline__ void pack_row(const PackPart &s, int u, int i, int no
         const int c = in ? cols[cur[j]] : -1;
         keep &= need[j] ? in && c == a[j] : cur[j] == -1;
     }
-    if (keep) return;
+    if (keep) {
+#pragma unroll
+        for (int j = 0; j < K; j++) slots |= was[j] != cur[j];
+        return;
+    }
     int at[K];
 #pragma unroll
     for (int j = 0; j < K; j++) at[j] = r0;
@@ -460,10 +471,8 @@ __device__ __forceinline__ void pack_row(const PackPart &s, int u, int i, int no
             if (r1 > r0 && cols[at[j]] == a[j]) v = at[j];
             else err = true;
         }
-        if (v != cur[j]) {
-            slot[(size_t)s.stride * j] = v;
-            slots = true;
-        }
+        if (v != cur[j]) slot[(size_t)s.stride * j] = v;
+        slots |= was[j] != v;
     }
 }
 

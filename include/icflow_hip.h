@@ -326,7 +326,10 @@ int icf_build_pattern(icf_ctx *ctx, const int *altId, int nNodes,
 /* Slot fields (position of (altId_i, altId_j) if both >= 0 and altId_j >= altId_i, else -1)
  * and row fields (altId_i or -1) of every element, CZ and impact, written in place; for CZs
  * also the current-failed, tentative-failed and tentative-damaged flags are reset to 0, as
- * TransferPCSR does.  ICF_E_INDEX if a needed pair is not in the pattern. */
+ * TransferPCSR does.  ICF_E_INDEX if a needed pair is not in the pattern.  The packed fields are held
+ * against what the context's lists (icf_pattern_changed) were built from, so the lists follow also
+ * where the fields were right before the call because another context or a kernel of the caller's
+ * had written them; fields that the call does not pack are not looked at. */
 int icf_pack_pcsr(icf_ctx *ctx, const int *altId, int nNodes, const int *csr_rows,
                   const int *csr_cols, int N, int *ie, int nElems, int el_stride,
                   int *icz, int nCZs, int cz_stride, int *icr, int nImpacts, int cr_stride);
