@@ -164,6 +164,13 @@ struct BpGrid {
 // negative, and in 16 bits that is its sign: tets of neighbouring cells are at most 3 cs apart along
 // an axis, 9 cs along a sum of three, 18,432 steps.  (Where rounding of the planes could add
 // to that, positions beyond 2^40 cs, all steps are 0, and every pair is left to the exact test.)
+//   Tets far smaller than the largest one, whose extent makes the cells, look alike in these steps: a
+// single tet drawn out to a hundred times the others' size, as before a Newton loop diverges, leaves
+// all pairs of a cell as candidates.  A search that finds more than BP_DENSE candidates per tet is
+// therefore repeated with the FP32 comparison behind that of the steps (168,000 tets
+// in eight cells, 1.8e9 pairs: 0.6 s a call, 7 s with FP32 alone; refused without).  Surfaces in contact have
+// some 5 candidates per tet (1.66M for 353,000).
+constexpr long long BP_DENSE = 64;
 constexpr double BP_STEPS = 2048;
 __device__ inline unsigned bp_step(double plane, double org, double invq)
 {
@@ -436,8 +443,24 @@ __device__ inline long long bp_slot(long long cap, const unsigned long long *__r
     return o < (n < capP ? n : capP) ? (long long)blockIdx.y * capP + o : -1;
 }
 
+// Whether two tets overlap in FP32, lo and hi rounded outward.
+__device__ inline bool bp_near32(const float4 *__restrict__ a, const float4 *__restrict__ b)
+{
+    bool hit = true;
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+        const float4 al = a[q], ah = a[3 + q], bl = b[q], bh = b[3 + q];
+        hit &= !(al.x > bh.x) & !(al.y > bh.y) & !(al.z > bh.z) & !(al.w > bh.w);
+        hit &= !(bl.x > ah.x) & !(bl.y > ah.y) & !(bl.z > ah.z) & !(bl.w > ah.w);
+    }
+    return hit;
+}
+
 // One wave's cell and slice of the pair search (k_bp_cellwave): on return, cnt pairs are left in buf.
-__device__ inline void bp_cell_pairs(const BpTet *__restrict__ srec, int exclude_shared, const BpGrid &g,
+// FINE: pairs that pass the steps have to overlap in FP32 as well.
+template <bool FINE>
+__device__ inline void bp_cell_pairs(const BpTet *__restrict__ srec, const float4 *__restrict__ sk32,
+                                     int exclude_shared, const BpGrid &g,
                                      const int *__restrict__ first, unsigned long long *__restrict__ total, unsigned long long *__restrict__ out,
                                      long long cap, int i, int slice, int slices, int chunk, BpWave &W, int lane,
                                      unsigned long long below, int &cnt)
@@ -501,6 +524,7 @@ __device__ inline void bp_cell_pairs(const BpTet *__restrict__ srec, int exclude
 #pragma unroll
                         for (int j1 = 0; j1 < 4; j1++) hit &= bn[j2] != an[j1];
                 }
+                if (FINE && hit) hit = bp_near32(sk32 + (size_t)(a0 + ia) * 6, sk32 + (size_t)pb * 6);
                 const unsigned long long mk = __ballot(hit);
                 if (hit) W.buf[cnt + __popcll(mk & below)] = ((unsigned long long)(a0 + ia) << 32) | (unsigned)pb;
                 cnt += __popcll(mk);
@@ -525,8 +549,9 @@ __device__ inline void bp_cell_pairs(const BpTet *__restrict__ srec, int exclude
     }
 }
 
+template <bool FINE>
 __global__ __launch_bounds__(64 * BPW_WAVES) void k_bp_cellwave(const BpTet *__restrict__ srec,
-                                                                int exclude_shared,
+                                                                const float4 *__restrict__ sk32, int exclude_shared,
                                                                 const BpGrid *__restrict__ grid, int slices, int chunk,
                                                                 const int *__restrict__ first,
                                                                 unsigned long long *__restrict__ total,
@@ -552,8 +577,8 @@ __global__ __launch_bounds__(64 * BPW_WAVES) void k_bp_cellwave(const BpTet *__r
     const int part = group % BP_PARTS;
     total += (size_t)part * BP_PART_STRIDE;
     out += (size_t)part * capP;
-    if (i < g.ncell) bp_cell_pairs(srec, exclude_shared, g, first, total, out, capP, i, w % slices, slices, chunk, waves[wave],
-                                   lane, below, cnt);
+    if (i < g.ncell) bp_cell_pairs<FINE>(srec, sk32, exclude_shared, g, first, total, out, capP, i, w % slices, slices, chunk,
+                                         waves[wave], lane, below, cnt);
     // the workgroup's last wave out writes every wave's remaining pairs
     if (lane == 0) wcnt[wave] = cnt;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");

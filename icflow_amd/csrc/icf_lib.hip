@@ -2716,7 +2716,7 @@ int icf_broad_phase(icf_ctx *ctx, const double *dn, int nd_stride, const int *ie
     long long cap = std::max<long long>({ctx->bp_cap, 4LL * nT, 64LL * BP_PARTS});
     const unsigned atiles = blocks_for(nT, BP_TILE);
     long long ncand = 0;
-    bool grown = false;
+    bool grown = false, fine = false;
     for (;;) {
         if (cap >= (1LL << 31)) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: more than 2^31 candidate pairs");
         const unsigned ctiles = blocks_for(capG, BP_TILE);
@@ -2751,9 +2751,9 @@ int icf_broad_phase(icf_ctx *ctx, const double *dn, int nd_stride, const int *ie
         // candidate count from device memory (their grids cover the buffer).  Below 16,384 cells several
         // waves share one.
         const int slices = (int)std::min<long long>(16, std::max(1LL, 20480 / capC));
-        hipLaunchKernelGGL(k_bp_cellwave, dim3(blocks_for(capC * slices, 512 * BPW_WAVES) * 512), dim3(64 * BPW_WAVES), 0,
-                           ctx->stream, srec, exclude_shared, grid, slices, slices > 1 ? 4 : BPW_OWN, first, tot,
-                           pa, cap);
+        hipLaunchKernelGGL(fine ? k_bp_cellwave<true> : k_bp_cellwave<false>,
+                           dim3(blocks_for(capC * slices, 512 * BPW_WAVES) * 512), dim3(64 * BPW_WAVES), 0, ctx->stream,
+                           srec, sk32, exclude_shared, grid, slices, slices > 1 ? 4 : BPW_OWN, first, tot, pa, cap);
         const dim3 gparts(blocks_for(cap / BP_PARTS, 256), BP_PARTS);   // a grid row per region
         hipLaunchKernelGGL(k_bp_exact, gparts, b, 0, ctx->stream, skd, sk32, sidx, tot, cap, pa, rnk, acount);
         hipLaunchKernelGGL(k_bp_tiles, dim3(atiles), b, 0, ctx->stream, acount, nT, grid, at);
@@ -2779,6 +2779,10 @@ int icf_broad_phase(icf_ctx *ctx, const double *dn, int nd_stride, const int *ie
         if (ncand <= cap / BP_PARTS) {
             *nOut = got[BP_NV];
             break;
+        }
+        if (!fine && BP_PARTS * ncand > BP_DENSE * nT) {
+            fine = true;
+            continue;
         }
         if (grown) return fail(ctx, ICF_E_CAPACITY, "icf_broad_phase: pair count changed between two searches");
         grown = true;

@@ -50,8 +50,9 @@ def _search(gf, x, room):
         yield d_pairs.download(2 * room).reshape(-1, 2)[:num.value]
 
 
-# 2.2e8 candidates, which the first pass's buffer holds if they are spread over its regions
-@pytest.mark.parametrize("n", [7400])
+# 2.2e8 pairs that the steps do not tell apart, which the buffer holds if they are spread over its regions,
+# and 1.8e9, which it does not
+@pytest.mark.parametrize("n", [7400, 21000])
 def test_crowded_cells(n):
     gf = GPUFunctionality(0)
     for count in (10, n):                   # the small scene sizes the second one's launches
