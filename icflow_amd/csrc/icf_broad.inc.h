@@ -602,7 +602,7 @@ __global__ __launch_bounds__(64 * BPW_WAVES) void k_bp_cellwave(const BpTet *__r
 
 // The pair search, second pass: per candidate (own, candidate) position pair of the first
 // pass, the exact test -- the FP64 12-direction overlap, the predicate of the reference's
-// k-DOP test.  The FP32 copies decide first where they can: the first pass's outward-rounded
+// k-DOP test.  The FP32 copies decide first where they can: the outward-rounded
 // values, each moved one step inward (nextafter), still overlap only if the FP64 values do
 // (lo <= nextafter(lo rounded down, +inf) and hi >= nextafter(hi rounded up, -inf)), so the
 // FP64 k-DOPs are read only for the pairs that are within an FP32 step of touching.  A pair

@@ -2745,11 +2745,14 @@ int icf_broad_phase(icf_ctx *ctx, const double *dn, int nd_stride, const int *ie
         hipLaunchKernelGGL(k_bp_scan, dim3(ctiles), b, 0, ctx->stream, count, -1, grid, ct, first, -1, rep);
         hipLaunchKernelGGL(k_bp_sorted, tets, b, 0, ctx->stream, dn, nd_stride, nT, key, rank, first, ie, el_all_stride,
                            grid, sidx, srec, skd, sk32);
-        // candidate pairs per cell (FP32 prefilter), collected in LDS and appended in batches; the
+        // candidate pairs per cell (16-bit steps), collected in LDS and appended in batches; the
         // exact test; the passing pairs grouped by a (a counting sort) and placed by their rank of b
         // within the group: the pairs in (a, b) order.  The launches after the search take the
-        // candidate count from device memory (their grids cover the buffer).  Below 16,384 cells several
-        // waves share one.
+        // candidate count from device memory (their grids cover the buffer).  Where the
+        // launch has room for 10,240 cells at most (the last search's, about 8,100, and a quarter) several
+        // waves share one: 166 us a call against 180 with 25 tets in each of 4,096 cells, 117 against 128
+        // in 1,728; from 8,000 cells on the shared ones are slower (244 against 235, 292 against 277 in
+        // 10,648).  With 6 tets a cell sharing costs 1 us of 71 to 5 of 95 over these sizes.
         const int slices = (int)std::min<long long>(16, std::max(1LL, 20480 / capC));
         hipLaunchKernelGGL(fine ? k_bp_cellwave<true> : k_bp_cellwave<false>,
                            dim3(blocks_for(capC * slices, 512 * BPW_WAVES) * 512), dim3(64 * BPW_WAVES), 0, ctx->stream,
