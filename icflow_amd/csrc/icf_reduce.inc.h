@@ -309,11 +309,12 @@ constexpr int CAND_FP32 = 2 * NSC + 0, CAND_FP64 = 2 * NSC + 1;   // a context's
 // batched specimens mixed 584 (604-653), 787,000 tets FP64 176 (173-196), 24 specimens FP64 60.6
 // (60.1-72.4), 146,000 tets mixed 28.3 (25.9-30.4).
 constexpr int CAND_UNTUNED = 1 * NSC + 1;
-// ... and where that leaves most of the chip idle, up to 131,072 blocks to overwrite, one wave of 64
-// keys with room for all of their contributions: 17.2 against 17.7 us (3,072 tets), 18.4 against 21.7
-// (15,360), 19.4 against 21.4 (93,000 blocks); at 202,000 blocks 25.6 against 25.2.  (Impacts add few to
-// a block, which any shape takes in one round.)
-constexpr int CAND_SMALL = NCAND, SMALL_KEYS = 64, SMALL_STAGE = 16, VALS_SMALL = 1 << 17;
+// ... and where that leaves most of the chip idle, up to 98,304 blocks to overwrite, one wave of 64
+// keys with room for all of their contributions: 14.5 against 16.5 us with 128 keys (7,900 blocks), 17.8
+// against 20.8 (33,800), 18.0 against 19.8 (93,800).  Beyond, its LDS (37 KB a wave) leaves the rest
+// waiting: 20.9 against 21.2 us in FP64 and 24.8 against 20.6 mixed at 109,800, 32.3 against 22.5 and 30.2
+// against 21.0 at 130,800.  (Impacts add few to a block, which any shape takes in one round.)
+constexpr int CAND_SMALL = NCAND, SMALL_KEYS = 64, SMALL_STAGE = 16, VALS_SMALL = 3 << 15;
 template <typename L, int KEYS, int STAGE>
 __host__ __device__ constexpr int flat_cap() { return sizeof(L) == 4 ? STAGE * KEYS : STAGE * KEYS / 2; }
 // bytes of LDS of a value reduction: the staged contributions, then the list of long keys
