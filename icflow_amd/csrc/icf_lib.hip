@@ -200,10 +200,11 @@ constexpr int SHAPE_UNTUNED[NSHAPE] = {2, 2, 1, 2, 0};
 // ... and for launches of at most so many units, whose workgroups would leave compute units empty
 // while each runs through a long chain: phase 1 with 64 lanes (14.3 -> 11.9 us on 3,072 tets, 20.7 ->
 // 18.9 on 48,000, 42.9 -> 41.9 on 309,000; 113.7 -> 117.7 on 779,000), 64 impacts (21.9 -> 17.8 us for
-// 547, 27.0 -> 18.2 for 7,000, 25.2 -> 22.1 for 20,900; 25.3 -> 28.3 for 61,600), 16 lanes per
-// tuple (9.5 -> 8.3 us for 547, 11.2 -> 9.9 for 7,000; 14.8 -> 14.4 for 20,900, 27.6 -> 28.4 for 61,600).
-constexpr int SHAPE_SMALL[NSHAPE] = {0, 2, 2, 0, 0};
-constexpr long long SHAPE_SMALL_MAX[NSHAPE] = {1 << 19, 0, 1 << 14, 1 << 15, 0};
+// 547, 27.0 -> 18.2 for 7,000, 25.2 -> 22.1 for 20,900; 25.3 -> 28.3 for 61,600).  (16 lanes per tuple would
+// take 1 us of 10 off the closest face below 16,384 tuples, but 8 is what an untuned context has always
+// reported and kept for a later run.)
+constexpr int SHAPE_SMALL[NSHAPE] = {0, 2, 1, 0, 0};
+constexpr long long SHAPE_SMALL_MAX[NSHAPE] = {1 << 19, 0, 0, 1 << 15, 0};
 
 struct icf_ctx {
     int id = 0;
@@ -280,14 +281,18 @@ struct icf_ctx {
         int ncand = NCAND;
         int sel = CAND_FP32;       // candidate in use
         bool tuned = false;        // a tuning has chosen it
-        int untuned = -1;              // what launches use when it is neither tuned nor set; -1: by their size
-        int small = 0;                 // ... where they have at most small_max units
+        int untuned = CAND_UNTUNED;    // what launches use when it is neither tuned nor set
+        int small = CAND_SMALL;        // ... where they have at most small_max units
         long long small_max = 0;
         bool active = false;       // timing the candidates in turn
         bool fixed = false;        // chosen by the caller (icf_set_chunk_keys / icf_set_shape)
         int turn = 0;              // launches started while tuning
         int samples = 0;           // launches timed
         int cand = -1;             // candidate of the launch being timed, -1: none
+        int last = -1;             // candidate of the role's last launch
+        // the shape that the role's launches use, as far as the caller can be told: a launch that is
+        // neither tuned nor set goes by its size
+        int in_use() const { return active || fixed || tuned || last < 0 ? sel : last; }
         int bucket = -1;           // size class of the launches timed (the shape cache's key)
         float best[NCAND] = {};    // fastest launch per candidate (ms), 0: not timed
         hipEvent_t ev[2] = {nullptr, nullptr};
@@ -1136,20 +1141,21 @@ void tune_fold(icf_ctx *ctx, icf_ctx::Tune &t, int role_id)
 // (not when `peek`).
 int tune_begin(icf_ctx *ctx, icf_ctx::Tune &t, int role_id, long long units, bool peek = false)
 {
-    const int bucket = size_class(units);
+    const int bucket = size_class(units) + (units <= t.small_max ? 64 : 0);   // small launches are apart
     if (!t.active || ctx->capturing || peek) {
+        t.last = t.sel;
         if (!t.active && !t.fixed) {
             std::lock_guard<std::mutex> lk(g_shape_cache.mu);
             auto it = g_shape_cache.choice.find({ctx->device, role_id, ctx->precision, bucket});
-            if (it != g_shape_cache.choice.end()) return it->second;
-            if (!t.tuned) return units <= t.small_max ? t.small : t.untuned;
+            if (it != g_shape_cache.choice.end()) t.last = it->second;
+            else if (!t.tuned) t.last = units <= t.small_max ? t.small : t.untuned;
         }
-        return t.sel;
+        return t.last;
     }
     tune_fold(ctx, t, role_id);
-    if (!t.active) return t.sel;
+    if (!t.active) return t.last = t.sel;
     t.bucket = bucket;
-    t.cand = t.turn++ % t.ncand;
+    t.last = t.cand = t.turn++ % t.ncand;
     (void)hipEventRecord(t.ev[0], ctx->cur);
     return t.cand;
 }
@@ -1162,8 +1168,7 @@ void tune_end(icf_ctx *ctx, icf_ctx::Tune &t)
 // value-reduction roles: ids 0-3
 int tune_begin(icf_ctx *ctx, bool acc, bool fp64, long long keys)
 {
-    const int c = tune_begin(ctx, ctx->tune[acc][fp64], 2 * acc + fp64, keys);
-    return c >= 0 ? c : !acc && keys <= VALS_SMALL ? CAND_SMALL : CAND_UNTUNED;
+    return tune_begin(ctx, ctx->tune[acc][fp64], 2 * acc + fp64, keys);
 }
 void tune_end(icf_ctx *ctx, bool acc, bool fp64) { tune_end(ctx, ctx->tune[acc][fp64]); }
 
@@ -1208,12 +1213,17 @@ void phase1_fused(icf_ctx *ctx, const int *ie, const double *dn, int nt, int es,
     shape_end(ctx, ICF_SHAPE_PHASE1);
 }
 
-// Calls f(integral_constant<cand_keys(c)>, integral_constant<cand_stage(c)>), or the small shape.
-template <typename F>
-void with_cand(int c, F &&f)
+// Calls f(integral_constant<cand_keys(c)>, integral_constant<cand_stage(c)>); OVER: for a launch that
+// overwrites `keys` blocks, where few of them give the candidates of 64 keys more room.
+template <bool OVER, typename F>
+void with_cand(int c, long long keys, F &&f)
 {
     static_assert(NCAND == 8, "one case per candidate");
     using std::integral_constant;
+    if constexpr (OVER) {
+        if (cand_keys(c) == SMALL_KEYS && keys <= VALS_SMALL)
+            return f(integral_constant<int, SMALL_KEYS>(), integral_constant<int, SMALL_STAGE>());
+    }
     switch (c) {
     case 0: f(integral_constant<int, cand_keys(0)>(), integral_constant<int, cand_stage(0)>()); break;
     case 1: f(integral_constant<int, cand_keys(1)>(), integral_constant<int, cand_stage(1)>()); break;
@@ -1222,8 +1232,7 @@ void with_cand(int c, F &&f)
     case 4: f(integral_constant<int, cand_keys(4)>(), integral_constant<int, cand_stage(4)>()); break;
     case 5: f(integral_constant<int, cand_keys(5)>(), integral_constant<int, cand_stage(5)>()); break;
     case 6: f(integral_constant<int, cand_keys(6)>(), integral_constant<int, cand_stage(6)>()); break;
-    case 7: f(integral_constant<int, cand_keys(7)>(), integral_constant<int, cand_stage(7)>()); break;
-    default: f(integral_constant<int, SMALL_KEYS>(), integral_constant<int, SMALL_STAGE>()); break;
+    default: f(integral_constant<int, cand_keys(7)>(), integral_constant<int, cand_stage(7)>()); break;
     }
 }
 
@@ -1238,7 +1247,7 @@ bool vals_force_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const SlotMap 
     double *ts = (double *)ctx->tsum.p;
     const int c = tune_begin(ctx, false, !mixed, mv->nlaunch);
     const int ilv = shape_begin(ctx, ICF_SHAPE_ORDER, mv->nlaunch);
-    with_cand(c, [&](auto kc, auto sc) {
+    with_cand<true>(c, mv->nlaunch, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
         const int nch = (int)blocks_for(mv->nlaunch, K);
         const int nbf = mf->nlaunch ? round8(blocks_for(mf->nlaunch, K)) : 0;
@@ -1270,7 +1279,7 @@ bool vals_force_rhs_fused(icf_ctx *ctx, const SlotMap *mv, double *A, const Slot
     const bool mixed = ctx->precision == ICF_MIXED, iso = ctx->hc.iso != 0;
     const int c = tune_begin(ctx, false, !mixed, mv->nlaunch);
     const int ilv = shape_begin(ctx, ICF_SHAPE_ORDER, mv->nlaunch);
-    with_cand(c, [&](auto kc, auto sc) {
+    with_cand<true>(c, mv->nlaunch, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
         const int nch = (int)blocks_for(mv->nlaunch, K);
         const int nbf = mf->nlaunch ? round8(blocks_for(mf->nlaunch, K)) : 0;
@@ -1306,7 +1315,7 @@ bool contact_sums_fused(icf_ctx *ctx, const SlotMap *mf, double *F, int ns, cons
     if (mf->nlaunch == 0 && mv->nlaunch == 0 && mr->nlaunch == 0) return true;
     const bool mixed = ctx->precision == ICF_MIXED;
     const int c = tune_begin(ctx, true, !mixed, mv->nlaunch);
-    with_cand(c, [&](auto kc, auto sc) {
+    with_cand<false>(c, mv->nlaunch, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
         const int nch = (int)blocks_for(mv->nlaunch, K);
         const int nb0 = mf->nlaunch ? round8(blocks_for(mf->nlaunch, K)) : 0, nb1 = round8(nch);
@@ -1345,7 +1354,7 @@ void vals_kernel(icf_ctx *ctx, const char *name, const SlotMap *m, double *A, co
     const int k = sizeof(L) == 4 ? 0 : 1;
     if (m->nlaunch == 0) return;
     const int c = tune_begin(ctx, ACC, k == 1, m->nlaunch);
-    with_cand(c, [&](auto kc, auto sc) {
+    with_cand<!ACC>(c, m->nlaunch, [&](auto kc, auto sc) {
         constexpr int K = decltype(kc)::value, S = decltype(sc)::value;
         LAUNCH(ctx, name, (k_reduce_vals<MX, IS, ACC, L, K, S>), dim3(blocks_for(m->nlaunch, K)), dim3(K), m->loff,
                m->codes, m->keys, m->nlaunch, A, sv);
@@ -1416,6 +1425,7 @@ int icf_create(int device, icf_ctx **out)
     if (device >= ndev) return ICF_E_INVALID;
     icf_ctx *ctx = new icf_ctx();
     for (auto &row : ctx->tune) row[1].sel = CAND_FP64;   // FP64 staging roles
+    for (auto &t : ctx->tune[0]) t.small_max = VALS_SMALL;
     for (int r = 0; r < NSHAPE; r++) {
         ctx->shape[r].ncand = shape_ncand(r);
         ctx->shape[r].sel = SHAPE_DEFAULT[r];
@@ -1871,8 +1881,8 @@ int icf_get_autotune(icf_ctx *ctx, int *keys, int *stage, int *tuning, float *be
     for (int r = 0; r < 4; r++) {
         icf_ctx::Tune &t = ctx->tune[r >> 1][r & 1];
         if (t.active && !ctx->capturing) tune_fold(ctx, t, r);   // a finished last timing counts
-        if (keys) keys[r] = cand_keys(t.sel);
-        if (stage) stage[r] = cand_stage(t.sel);
+        if (keys) keys[r] = cand_keys(t.in_use());
+        if (stage) stage[r] = cand_stage(t.in_use());
         if (tuning) tuning[r] = t.active ? 1 : 0;
         if (best_ms)
             for (int c = 0; c < NCAND; c++) best_ms[r * NCAND + c] = t.best[c];
@@ -1922,7 +1932,7 @@ int icf_get_shape(icf_ctx *ctx, int role, int *value, int *tuning, float *best_m
     if (role < 0 || role >= NSHAPE) return fail(ctx, ICF_E_INVALID, "icf_get_shape: unknown role");
     icf_ctx::Tune &t = ctx->shape[role];
     if (t.active && !ctx->capturing) tune_fold(ctx, t, 4 + role);
-    if (value) *value = shape_value(role, t.sel);
+    if (value) *value = shape_value(role, t.in_use());
     if (tuning) *tuning = t.active ? 1 : 0;
     if (best_ms)
         for (int c = 0; c < NSHAPE_CAND; c++) best_ms[c] = c < t.ncand ? t.best[c] : 0.f;

@@ -313,8 +313,11 @@ constexpr int CAND_UNTUNED = 1 * NSC + 1;
 // keys with room for all of their contributions: 14.5 against 16.5 us with 128 keys (7,900 blocks), 17.8
 // against 20.8 (33,800), 18.0 against 19.8 (93,800).  Beyond, its LDS (37 KB a wave) leaves the rest
 // waiting: 20.9 against 21.2 us in FP64 and 24.8 against 20.6 mixed at 109,800, 32.3 against 22.5 and 30.2
-// against 21.0 at 130,800.  (Impacts add few to a block, which any shape takes in one round.)
-constexpr int CAND_SMALL = NCAND, SMALL_KEYS = 64, SMALL_STAGE = 16, VALS_SMALL = 3 << 15;
+// against 21.0 at 130,800.  In such launches both candidates of 64 keys take that room, whatever their
+// staging, so that the tuner and the callers that set a shape have it too (with 2 or 3 a key they
+// took 16.1 to 17.4 us, 20.5 and 21.5, 22.2 and 23.7).  (Impacts add few to a block, which any shape takes in
+// one round.)
+constexpr int CAND_SMALL = 0 * NSC + 1, SMALL_KEYS = cand_keys(CAND_SMALL), SMALL_STAGE = 16, VALS_SMALL = 3 << 15;
 template <typename L, int KEYS, int STAGE>
 __host__ __device__ constexpr int flat_cap() { return sizeof(L) == 4 ? STAGE * KEYS : STAGE * KEYS / 2; }
 // bytes of LDS of a value reduction: the staged contributions, then the list of long keys

@@ -180,7 +180,7 @@ class GPUFunctionality:
 
     def tuned_shapes(self):
         """{role: [keys, stage]} for the value reductions and {role: value} for the other launch
-        shapes in use, to keep for a later run on the same specimen."""
+        shapes in use, tuned or not, to keep for a later run on the same specimen."""
         out = {r: list(v[0]) for r, v in self.autotune_state().items()}
         out.update({r: v[0] for r, v in self.shape_state().items()})
         return out

@@ -235,9 +235,11 @@ int icf_set_overlap(icf_ctx *ctx, int on);
  * (BCSR blocks), one key per lane, with the chunk's contributions staged in LDS.  A chunk
  * shape is a key limit (the workgroup size: 64, 128, 256 or 512) and a staging size (stage =
  * 2 or 3 FP32 contributions per key, half as many FP64 ones); the ICF_CHUNK_CANDIDATES = 8
- * shapes are numbered c = 2 * (index of the key limit) + (stage - 2).  Until tuned: 256 keys,
- * stage 2 for FP32 staging, 3 for FP64 (what icf_get_autotune reports; launches of a role that was
- * never tuned or set may use another shape that the library finds better for their size).  There are four roles, r = 2 * accumulate + fp64:
+ * shapes are numbered c = 2 * (index of the key limit) + (stage - 2).  With 64 keys a launch that
+ * overwrites at most 98,304 blocks stages 16 FP32 or 8 FP64 contributions per key in place of either
+ * stage.  A role that was never tuned or set takes (64, 3) for those launches and (128, 3) for others;
+ * before its first launch 256 keys are reported, stage 2 for FP32 staging and 3 for FP64.  There are
+ * four roles, r = 2 * accumulate + fp64:
  * overwrite maps (icf_assemble_elems_and_czs) and accumulate maps (icf_collision_response and
  * the single-kernel calls), each with FP32 (mixed) or FP64 staging.
  * icf_set_autotune(ctx, rounds > 0) starts tuning every role: its next launches take the
@@ -245,9 +247,9 @@ int icf_set_overlap(icf_ctx *ctx, int on);
  * role), until every candidate has `rounds` timings; then the fastest (least time over its
  * timings) is kept.  rounds = 0 stops tuning and keeps the fastest timed so far.  Captured
  * calls are never timed.  Time it in blocking mode or with overlap off for clean timings.
- * icf_get_autotune: per role, keys[r] and stage[r] = the shape in use, tuning[r] = 1 while
- * tuning, best_ms[r * ICF_CHUNK_CANDIDATES + c] = fastest timing of candidate c (0 = none);
- * any of the four may be null.  icf_set_chunk_keys fixes one role's shape (stage 0: keep the
+ * icf_get_autotune: per role, keys[r] and stage[r] = the shape in use (of a role that was neither
+ * tuned nor set its last launch's), tuning[r] = 1 while tuning, best_ms[r * ICF_CHUNK_CANDIDATES + c] =
+ * fastest timing of candidate c (0 = none); any of the four may be null.  icf_set_chunk_keys fixes one role's shape (stage 0: keep the
  * role's staging) and ends its tuning.  Results do not depend on the shape: each key's
  * contributions are added in list order whatever the chunking.  No reference counterpart (the
  * reference launches every kernel with a fixed block_size = 128, GPU_Functionality.cs:38,123-136). */
@@ -266,8 +268,9 @@ int icf_set_chunk_keys(icf_ctx *ctx, int accumulate, int fp64, int keys, int sta
  *   ICF_SHAPE_ORDER    the fused value launch's phases: 0 node forces first, then the BCSR
  *                      values; 1 interleaved in rounds of eight workgroups (0, 1)
  * Every candidate gives the same results bit for bit.  icf_set_shape fixes a role's value on
- * this context (ICF_E_INVALID for other values); icf_get_shape reports the context's value
- * (the default until tuned or set; a launch of such a role may use another), whether the role is still being tuned and the fastest
+ * this context (ICF_E_INVALID for other values); icf_get_shape reports the value in use
+ * (until tuned or set that of the role's last launch, whose size may decide it; before any 256, 8
+ * lanes, order 1), whether the role is still being tuned and the fastest
  * timing per candidate (best_ms[3], 0: not timed or no such candidate).  Finished tunings, of these roles and of the
  * value reductions, are kept by the library per device, role, precision and size class (units
  * of the launch to the next power of two); a context's launches of a role that it is neither
