@@ -200,11 +200,13 @@ constexpr int SHAPE_UNTUNED[NSHAPE] = {2, 2, 1, 2, 0};
 // ... and for launches of at most so many units, whose workgroups would leave compute units empty
 // while each runs through a long chain: phase 1 with 64 lanes (14.3 -> 11.9 us on 3,072 tets, 20.7 ->
 // 18.9 on 48,000, 42.9 -> 41.9 on 309,000; 113.7 -> 117.7 on 779,000), 64 impacts (21.9 -> 17.8 us for
-// 547, 27.0 -> 18.2 for 7,000, 25.2 -> 22.1 for 20,900; 25.3 -> 28.3 for 61,600).  (16 lanes per tuple would
-// take 1 us of 10 off the closest face below 16,384 tuples, but 8 is what an untuned context has always
-// reported and kept for a later run.)
+// 547, 27.0 -> 18.2 for 7,000, 25.2 -> 22.1 for 20,900; 25.3 -> 28.3 for 61,600).
 constexpr int SHAPE_SMALL[NSHAPE] = {0, 2, 1, 0, 0};
 constexpr long long SHAPE_SMALL_MAX[NSHAPE] = {1 << 19, 0, 0, 1 << 15, 0};
+// For the same reason the closest face's candidate of 8 lanes takes 16 for at most so many tuples (9.5 ->
+// 8.3 us for 547, 11.2 -> 9.9 for 7,000; 14.8 -> 14.4 for 20,900, 27.6 -> 28.4 for 61,600), tuned, set or
+// neither: a candidate's launch, so that 8, which untuned contexts report, stays what they use.
+constexpr int CLOSEST_SMALL = 1 << 14;
 
 struct icf_ctx {
     int id = 0;
@@ -2083,7 +2085,8 @@ void launch_closest_face(icf_ctx *ctx, int nPairs, int ts, int *nl2, const doubl
                          const int *adj_ids, const int *faces, int ns, int fs, hipStream_t stream)
 {
     const bool timed = stream == ctx->cur;   // tuning times launches on the current stream only
-    const int G = shape_begin(ctx, ICF_SHAPE_CLOSEST, nPairs, !timed);
+    int G = shape_begin(ctx, ICF_SHAPE_CLOSEST, nPairs, !timed);
+    if (G == 8 && nPairs <= CLOSEST_SMALL) G = 16;
     const dim3 g(blocks_for((long long)nPairs * G, 256)), b(256);
     auto go = [&](auto kern) {
         if (stream == ctx->cur) LAUNCH(ctx, "k_closest_face", kern, g, b, nPairs, ts, nl2, dn, adj_off, adj_ids, faces, ns, fs);

@@ -263,7 +263,8 @@ int icf_set_chunk_keys(icf_ctx *ctx, int accumulate, int fp64, int keys, int sta
  * by icf_set_autotune (the candidates of each role timed in turn on the role's launches):
  *   ICF_SHAPE_PHASE1   workgroup size of phase 1 of the fused call (64, 128, 256)
  *   ICF_SHAPE_NARROW   workgroup size of the narrow phase (64, 128, 256)
- *   ICF_SHAPE_CLOSEST  lanes per (node, tet) tuple of the closest face (4, 8, 16)
+ *   ICF_SHAPE_CLOSEST  lanes per (node, tet) tuple of the closest face (4, 8, 16; a launch of at
+ *                      most 16,384 tuples takes 16 for 8)
  *   ICF_SHAPE_IMPACT   workgroup size of the impacts' phase 1 (64, 128, 256)
  *   ICF_SHAPE_ORDER    the fused value launch's phases: 0 node forces first, then the BCSR
  *                      values; 1 interleaved in rounds of eight workgroups (0, 1)
