@@ -428,9 +428,9 @@ struct BpWave {
     unsigned short list[BPW_LIST];      // own << 6 | candidate
 };
 // The candidate buffer is split into BP_PARTS regions of cap / BP_PARTS entries, each with its
-// own counter (BP_PART_STRIDE counters apart, so that no two share a cache line): the w-th pair of
-// waves, in the cells' order, appends to region w mod BP_PARTS, which spreads the reservations over as many
-// addresses and neighbouring cells' candidates over all regions.
+// own counter (BP_PART_STRIDE counters apart, so that no two share a cache line): consecutive cells, or
+// pairs of cells where a workgroup has two, append to one after the other, which spreads the
+// reservations over as many addresses and neighbouring cells' candidates over all regions.
 constexpr int BP_PARTS = 8, BP_PART_STRIDE = 64;
 
 // The later passes run a grid row per region (blockIdx.y): this thread's position in the
@@ -572,9 +572,11 @@ __global__ __launch_bounds__(64 * BPW_WAVES) void k_bp_cellwave(const BpTet *__r
     const int group = run + in % 8 * 64 + in / 8;
     const int w = group * BPW_WAVES + wave, i = w / slices;
     const long long capP = cap / BP_PARTS;
-    // by the group of cells, not by blockIdx, whose eighths are runs of cells: candidates crowd into
-    // neighbouring cells, and the fullest region decides how large the buffer has to be
-    const int part = group % BP_PARTS;
+    // by the group's cells (slices: 1 or an even number), not by blockIdx, whose eighths are runs of cells:
+    // candidates crowd into neighbouring cells, and the fullest region decides how large the buffer has
+    // to be.  All slices of a cell go to one region, which then counts the same in a repeated search,
+    // whatever the order of the tets in their cells.
+    const int part = (slices > 1 ? i : group) % BP_PARTS;
     total += (size_t)part * BP_PART_STRIDE;
     out += (size_t)part * capP;
     if (i < g.ncell) bp_cell_pairs<FINE>(srec, sk32, exclude_shared, g, first, total, out, capP, i, w % slices, slices, chunk,

@@ -2766,7 +2766,8 @@ int icf_broad_phase(icf_ctx *ctx, const double *dn, int nd_stride, const int *ie
         // waves share one: 166 us a call against 180 with 25 tets in each of 4,096 cells, 117 against 128
         // in 1,728; from 8,000 cells on the shared ones are slower (244 against 235, 292 against 277 in
         // 10,648).  With 6 tets a cell sharing costs 1 us of 71 to 5 of 95 over these sizes.
-        const int slices = (int)std::min<long long>(16, std::max(1LL, 20480 / capC));
+        int slices = (int)std::min<long long>(16, std::max(1LL, 20480 / capC));
+        if (slices > 1) slices -= slices % BPW_WAVES;      // a workgroup's waves share a cell
         hipLaunchKernelGGL(fine ? k_bp_cellwave<true> : k_bp_cellwave<false>,
                            dim3(blocks_for(capC * slices, 512 * BPW_WAVES) * 512), dim3(64 * BPW_WAVES), 0, ctx->stream,
                            srec, sk32, exclude_shared, grid, slices, slices > 1 ? 4 : BPW_OWN, first, tot, pa, cap);

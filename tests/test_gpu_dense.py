@@ -6,7 +6,7 @@ import ctypes
 import numpy as np
 import pytest
 
-from icflow_amd import _lib
+from icflow_amd import _lib, specimens
 from icflow_amd.gpu_functionality import GPUFunctionality
 
 pytestmark = pytest.mark.gpu
@@ -34,12 +34,11 @@ def _scene(n):
     return x, np.array(pairs)
 
 
-def _search(gf, x, room):
-    n = len(x)
-    ns, es = 4 * n, n
+def _search(gf, x, ids, room):
+    n, ns, es = len(ids), len(x), len(ids)
     dn, ie = np.zeros((18, ns)), np.zeros((5, es), np.int32)
-    dn[15:18] = x.reshape(-1, 3).T
-    ie[:4] = np.arange(4 * n).reshape(n, 4).T
+    dn[15:18] = x.T
+    ie[:4] = ids.T
     d_dn, d_ie = gf.buf("dn%d" % n, dn.size, np.float64), gf.buf("ie%d" % n, ie.size, np.int32)
     d_dn.upload(dn.ravel())
     d_ie.upload(ie.ravel())
@@ -57,6 +56,19 @@ def test_crowded_cells(n):
     gf = GPUFunctionality(0)
     for count in (10, n):                   # the small scene sizes the second one's launches
         x, want = _scene(count)
-        for got in _search(gf, x, 4096):
+        for got in _search(gf, x.reshape(-1, 3), np.arange(4 * len(x)).reshape(-1, 4), 4096):
             assert np.array_equal(got, want), count
     gf.close()
+
+
+def test_first_search_of_a_context(specimen_consts):
+    """More candidates than a new context's buffer takes: the tets of a cell may lie in another order in
+    the second search, whose regions have to hold what the first one counted."""
+    col = specimens.make_specimen((3, 3, 3), (0.0075,) * 3, 2, 1, platens=(2, 2)).finalize()
+    for seed in range(150):
+        st = specimens.synthetic_state(col, specimen_consts, seed, platen_dz=0.3 * 0.0025)
+        gf, want = GPUFunctionality(0), None
+        for got in _search(gf, col.x0 + st.un, col.surf, 10000):
+            want = got if want is None else want
+            assert len(want) > 0 and np.array_equal(got, want)
+        gf.close()
