@@ -206,9 +206,11 @@ __device__ inline void sort_codes(uint32_t *c, int b, int e)
 
 // Each key's codes ascending: 256 consecutive keys per workgroup, whose codes are one run, sorted
 // in LDS by one thread per key (insertion: a block receives a few tens of contributions at most);
-// in place where the run does not fit.  In memory the same sort took 219 us for the four maps of
-// the 384,000-tet compression, a chain of dependent loads and stores per key.
-constexpr int SORT_CAP = 4096;
+// in place where the run does not fit, a chain of dependent loads and stores per key.  256 rhs rows have
+// some 4,400 contributions, 4,954 at most in the meshes measured; with room for 4,096 four
+// fifths of their workgroups sorted in place: the three maps of the 15,360-tet beam took 62 us, now 34,
+// those of the 384,000-tet compression 140, now 92.  6,144 and 8,192 take 100 and 131 there: less of the chip's LDS is left for other workgroups.
+constexpr int SORT_CAP = 5120;
 __global__ __launch_bounds__(256) void k_map_sort(MapJobs J)
 {
     __shared__ uint32_t lds[SORT_CAP];
