@@ -1896,7 +1896,7 @@ int icf_set_chunk_keys(icf_ctx *ctx, int accumulate, int fp64, int keys, int sta
 {
     if (!ctx) return ICF_E_INVALID;
     icf_ctx::Tune &t = ctx->tune[accumulate != 0][fp64 != 0];
-    if (stage == 0) stage = cand_stage(t.sel);
+    if (stage == 0) stage = cand_stage(t.in_use());
     int c = 0;
     while (c < NCAND && (cand_keys(c) != keys || cand_stage(c) != stage)) c++;
     if (c == NCAND)

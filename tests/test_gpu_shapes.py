@@ -41,6 +41,9 @@ def test_untuned_shapes_are_reported(specimen_consts, precision):
         for k in ("vals", "rhs", "F", "dcz"):
             assert np.array_equal(got[k], ref[k]), k
         q.gf.close()
+    # stage 0 keeps the staging that is reported
+    p.gf.set_chunk_keys(1, precision == _lib.ICF_FP64, 256, 0)
+    assert p.gf.tuned_shapes()["accumulate," + stage] == [256, 3]
     # what is set is what is reported
     p.gf.set_shape("phase1", 128)
     p.gf.set_chunk_keys(0, precision == _lib.ICF_FP64, 512, 2)
